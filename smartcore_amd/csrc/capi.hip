@@ -469,12 +469,10 @@ size_t scratch_round(size_t want) {
   return r;
 }
 
-namespace {
-bool capturing(hipStream_t s) {
+bool stream_capturing(hipStream_t s) {
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   return hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone;
 }
-}  // namespace
 
 void* scratch_take(hipStream_t s, size_t want, size_t* cap) {
   ScratchCache& c = scratch_cache();
@@ -486,7 +484,7 @@ void* scratch_take(hipStream_t s, size_t want, size_t* cap) {
     // the smallest block that fits and is not far larger than needed
     auto b = ps.blocks.lower_bound(want);
     if (b == ps.blocks.end() || b->first > 2 * scratch_round(want)) return nullptr;
-    if (capturing(s)) return nullptr;
+    if (stream_capturing(s)) return nullptr;
     void* p = b->second;
     *cap = b->first;
     ps.bytes -= b->first;
@@ -499,7 +497,7 @@ bool scratch_give(hipStream_t s, void* p, size_t cap) {
   ScratchCache& c = scratch_cache();
   std::lock_guard<std::mutex> lk(c.mu);
   auto it = c.streams.find(s);
-  if (it == c.streams.end() || capturing(s)) return false;
+  if (it == c.streams.end() || stream_capturing(s)) return false;
   auto& ps = it->second;
   if (ps.bytes + cap > kScratchKeepPerStream) return false;
   ps.blocks.emplace(cap, p);
@@ -646,6 +644,7 @@ int sc_index_destroy(sc_index* index) {
   if (index->rows) (void)hipFree(index->rows);
   if (index->rows_bf16) (void)hipFree(index->rows_bf16);
   if (index->norms2) (void)hipFree(index->norms2);
+  if (index->norms64) (void)hipFree(index->norms64);
   if (index->rows_q16) (void)hipFree(index->rows_q16);
   if (index->err_q16) (void)hipFree(index->err_q16);
   (void)hipSetDevice(cur);

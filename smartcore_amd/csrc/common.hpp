@@ -116,6 +116,9 @@ struct sc_index {
   uint32_t* err_q16;
   double q16_lo, q16_step;
   int q16_state;
+  // Lazily built for the FP64 matrix form (guarded by mu): per row, padded to
+  // whole 128-row tiles, a lower bound of the squared norm.
+  double* norms64;
   void* mu;         // std::mutex*
 };
 
@@ -219,6 +222,9 @@ class ProfScope {
   hipEvent_t start_ = nullptr;
 };
 
+// Whether work on s is being recorded into a graph (or that cannot be told).
+bool stream_capturing(hipStream_t s);
+
 // Whether the tracing hooks are on (sc_profile_enable).
 bool profiling_enabled();
 
@@ -236,6 +242,11 @@ hipStream_t copy_stream_for_device(int device);
 int knn_exact_device(const sc_index* index, const void* d_queries, size_t q, size_t k,
                      sc_metric metric, int p, int64_t* d_idx, double* d_dist, uint32_t* d_count,
                      hipStream_t stream, sc_stats* stats);
+
+// The same for the Euclidian metric and k <= 64, on FP64 matrix instructions
+// (queries: at least one).
+int knn_f64_device(const sc_index* index, const void* d_queries, int64_t q, int k, int64_t* d_idx,
+                   double* d_dist, uint32_t* d_count, hipStream_t stream, sc_stats* stats);
 
 // SC_MIXED Manhattan: bounded f32 scan, candidates rescored in the
 // reference arithmetic (f32 rows; f64 rows take the exact form).

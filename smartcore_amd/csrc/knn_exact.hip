@@ -1,5 +1,7 @@
 // Exact brute-force kNN (LinearKNNSearch::find, linear_search.rs:52-84) for
-// the Euclidian, Manhattan and Minkowski metrics on f64 / f32 rows.
+// the Manhattan and Minkowski metrics on f64 / f32 rows, and the sequential
+// kernel every form falls back to.  (Euclidian searches with k <= 64 run on
+// FP64 matrix instructions, knn_f64.hip: their sums have a dot-product form.)
 //
 // Three kernels:
 //   scan    Tiled distance kernel.  A workgroup owns 32 queries x one
@@ -30,6 +32,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "heap.hpp"
 #include "metric.hpp"
 #include "tile.hpp"
 
@@ -579,49 +582,6 @@ struct CandSet {
 // <) enter one after another, in row order, by a sift-down of the heap
 // held across the lanes, and the rest are tested again against the new top.
 constexpr int kReplayWaves = 4;
-__device__ __forceinline__ double lane_value(double v, int l) {
-  const int lo = __builtin_amdgcn_readlane(static_cast<int>(__double_as_longlong(v)), l);
-  const int hi = __builtin_amdgcn_readlane(static_cast<int>(__double_as_longlong(v) >> 32), l);
-  return __longlong_as_double((static_cast<long long>(hi) << 32) |
-                              static_cast<unsigned long long>(static_cast<uint32_t>(lo)));
-}
-
-// The reference heap held across a wave's lanes: lane j < k holds entry j
-// (distance hd, row hi); root replacement and HeapSelection::sift_down
-// (heap_select.rs:71-86) with readlane reads and select swaps.
-__device__ __forceinline__ void lane_heap_push_root(double& hd, uint32_t& hi, int lane, int k,
-                                                    double d, uint32_t row) {
-  if (lane == 0) {
-    hd = d;
-    hi = row;
-  }
-  const int n = k - 1;
-  int kk = 0;
-  const double vk = d;
-  while (2 * kk <= n) {
-    int j = 2 * kk;
-    double vj = lane_value(hd, j);
-    if (j < n) {
-      const double vj1 = lane_value(hd, j + 1);
-      if (vj < vj1) {
-        j += 1;
-        vj = vj1;
-      }
-    }
-    if (vk == vj || vk > vj) break;
-    const uint32_t ij = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(hi), j));
-    const uint32_t ik = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(hi), kk));
-    if (lane == kk) {
-      hd = vj;
-      hi = ij;
-    } else if (lane == j) {
-      hd = vk;
-      hi = ik;
-    }
-    kk = j;
-  }
-}
-
 template <int M>
 __global__ __launch_bounds__(64 * kReplayWaves) void knn_replay_kernel(
     int64_t q, int k, double p, CandSet pre, int nseg, int cap,
@@ -678,20 +638,7 @@ __global__ __launch_bounds__(64 * kReplayWaves) void knn_replay_kernel(
     walk(cand_idx, cand_s, base, cand_count[static_cast<size_t>(qi) * nseg + s2]);
   }
   if (lane == 0) atomicAdd(total_cand, seen);
-  // linear_search.rs:79-83: keep heap-array order, drop None entries.
-  const bool full = lane < k && hi != 0xffffffffu;
-  const uint64_t fm = __ballot(full);
-  const int c = __popcll(fm);
-  if (full) {
-    const int pos = __popcll(fm & ((uint64_t(1) << lane) - 1));
-    out_idx[qi * k + pos] = static_cast<int64_t>(hi);
-    out_dist[qi * k + pos] = hd;
-  }
-  if (lane >= c && lane < k) {
-    out_idx[qi * k + lane] = -1;
-    out_dist[qi * k + lane] = NAN;
-  }
-  if (lane == 0) out_count[qi] = static_cast<uint32_t>(c);
+  lane_heap_store(hd, hi, lane, k, out_idx + qi * k, out_dist + qi * k, out_count + qi);
 }
 
 // One workgroup per listed query; persistent over the list so the grid can
@@ -798,6 +745,67 @@ Plan make_plan(int64_t n, int64_t q, int k) {
   return Plan{static_cast<int>(nseg), seg_len, static_cast<int>(cap)};
 }
 
+// The scan, replay and serial kernels over batches of queries.
+template <typename T, int M>
+int run_tiled(const sc_index* index, const T* d_queries, int64_t q, int k, double p,
+              int64_t* d_idx, double* d_dist, uint32_t* d_count, uint32_t* olist,
+              uint32_t* overflow_n, unsigned long long* total_cand, hipStream_t stream,
+              sc_stats* stats) {
+  const int64_t n = static_cast<int64_t>(index->n);
+  const int ld = static_cast<int>(index->ld);
+  const T* refs = static_cast<const T*>(index->rows);
+  // Bound the candidate store to ~1 GiB by processing query batches.
+  Plan plan = make_plan(n, q, k);
+  const size_t per_query = static_cast<size_t>(plan.nseg) * plan.cap * 12 + plan.nseg * 4;
+  int64_t qb = std::max<int64_t>(QT, static_cast<int64_t>((size_t(1) << 30) / per_query) / QT * QT);
+  qb = std::min(qb, q);
+  DevBuf cidx, cs, ccnt;
+  SC_HIP(cidx.alloc(sizeof(uint32_t) * qb * plan.nseg * plan.cap, stream));
+  SC_HIP(cs.alloc(sizeof(double) * qb * plan.nseg * plan.cap, stream));
+  SC_HIP(ccnt.alloc(sizeof(uint32_t) * qb * plan.nseg, stream));
+  for (int64_t b0 = 0; b0 < q; b0 += qb) {
+    const int64_t qn = std::min(qb, q - b0);
+    dim3 grid(static_cast<unsigned>((qn + QT - 1) / QT), static_cast<unsigned>(plan.nseg));
+    {
+      ProfScope ps("knn_scan", stream);
+      hipLaunchKernelGGL((knn_scan_kernel<T, M>), grid, dim3(NT), 0, stream, refs, n, ld,
+                         static_cast<int>(index->d), d_queries + b0 * ld, qn, k, p,
+                         plan.seg_len, plan.nseg,
+                         cidx.as<uint32_t>(), cs.as<double>(), ccnt.as<uint32_t>(), plan.cap);
+      SC_HIP(hipGetLastError());
+    }
+    {
+      ProfScope ps("knn_replay", stream);
+      hipLaunchKernelGGL((knn_replay_kernel<M>),
+                         dim3(static_cast<unsigned>((qn + kReplayWaves - 1) / kReplayWaves)),
+                         dim3(64 * kReplayWaves), 0, stream, qn, k, p, CandSet{nullptr, nullptr, nullptr, 0, 1},
+                         plan.nseg, plan.cap,
+                         cidx.as<uint32_t>(), cs.as<double>(), ccnt.as<uint32_t>(),
+                         d_idx + b0 * k, d_dist + b0 * k, d_count + b0, olist, overflow_n,
+                         total_cand);
+      SC_HIP(hipGetLastError());
+    }
+    {
+      // batch-relative query ids in the overflow list
+      ProfScope ps("knn_serial", stream);
+      hipLaunchKernelGGL((knn_serial_kernel<T, M>), dim3(512), dim3(NT), 0, stream, refs, n,
+                         ld, d_queries + b0 * ld, k, p, olist, overflow_n, d_idx + b0 * k,
+                         d_dist + b0 * k, d_count + b0);
+      SC_HIP(hipGetLastError());
+    }
+    if (stats) {
+      uint32_t ov = 0;
+      SC_HIP(hipMemcpyAsync(&ov, overflow_n, 4, hipMemcpyDeviceToHost, stream));
+      SC_HIP(hipStreamSynchronize(stream));
+      stats->overflow_queries += ov;
+    }
+    SC_HIP(hipMemsetAsync(overflow_n, 0, 4, stream));
+  }
+  return SC_OK;
+}
+
+// Euclidian searches come here with k > KMAX_TILED only (knn_f64.hip takes
+// the others), so their scan is not built.
 template <typename T, int M>
 int run_exact(const sc_index* index, const T* d_queries, int64_t q, int k, double p, int64_t* d_idx,
               double* d_dist, uint32_t* d_count, hipStream_t stream, sc_stats* stats) {
@@ -813,55 +821,14 @@ int run_exact(const sc_index* index, const T* d_queries, int64_t q, int k, doubl
   DevBuf olist;
   SC_HIP(olist.alloc(sizeof(uint32_t) * std::max<int64_t>(q, 1), stream));
 
-  if (k <= KMAX_TILED) {
-    // Bound the candidate store to ~1 GiB by processing query batches.
-    Plan plan = make_plan(n, q, k);
-    const size_t per_query = static_cast<size_t>(plan.nseg) * plan.cap * 12 + plan.nseg * 4;
-    int64_t qb = std::max<int64_t>(QT, static_cast<int64_t>((size_t(1) << 30) / per_query) / QT * QT);
-    qb = std::min(qb, q);
-    DevBuf cidx, cs, ccnt;
-    SC_HIP(cidx.alloc(sizeof(uint32_t) * qb * plan.nseg * plan.cap, stream));
-    SC_HIP(cs.alloc(sizeof(double) * qb * plan.nseg * plan.cap, stream));
-    SC_HIP(ccnt.alloc(sizeof(uint32_t) * qb * plan.nseg, stream));
-    for (int64_t b0 = 0; b0 < q; b0 += qb) {
-      const int64_t qn = std::min(qb, q - b0);
-      dim3 grid(static_cast<unsigned>((qn + QT - 1) / QT), static_cast<unsigned>(plan.nseg));
-      {
-        ProfScope ps("knn_scan", stream);
-        hipLaunchKernelGGL((knn_scan_kernel<T, M>), grid, dim3(NT), 0, stream, refs, n, ld,
-                           static_cast<int>(index->d), d_queries + b0 * ld, qn, k, p,
-                           plan.seg_len, plan.nseg,
-                           cidx.as<uint32_t>(), cs.as<double>(), ccnt.as<uint32_t>(), plan.cap);
-        SC_HIP(hipGetLastError());
-      }
-      {
-        ProfScope ps("knn_replay", stream);
-        hipLaunchKernelGGL((knn_replay_kernel<M>),
-                           dim3(static_cast<unsigned>((qn + kReplayWaves - 1) / kReplayWaves)),
-                           dim3(64 * kReplayWaves), 0, stream, qn, k, p, CandSet{nullptr, nullptr, nullptr, 0, 1},
-                           plan.nseg, plan.cap,
-                           cidx.as<uint32_t>(), cs.as<double>(), ccnt.as<uint32_t>(),
-                           d_idx + b0 * k, d_dist + b0 * k, d_count + b0, olist.as<uint32_t>(),
-                           overflow_n, total_cand);
-        SC_HIP(hipGetLastError());
-      }
-      {
-        // batch-relative query ids in the overflow list
-        ProfScope ps("knn_serial", stream);
-        hipLaunchKernelGGL((knn_serial_kernel<T, M>), dim3(512), dim3(NT), 0, stream, refs, n,
-                           ld, d_queries + b0 * ld, k, p, olist.as<uint32_t>(), overflow_n,
-                           d_idx + b0 * k, d_dist + b0 * k, d_count + b0);
-        SC_HIP(hipGetLastError());
-      }
-      if (stats) {
-        uint32_t ov = 0;
-        SC_HIP(hipMemcpyAsync(&ov, overflow_n, 4, hipMemcpyDeviceToHost, stream));
-        SC_HIP(hipStreamSynchronize(stream));
-        stats->overflow_queries += ov;
-      }
-      SC_HIP(hipMemsetAsync(overflow_n, 0, 4, stream));
+  if constexpr (M != kEuclid) {
+    if (k <= KMAX_TILED) {
+      if (int rc = run_tiled<T, M>(index, d_queries, q, k, p, d_idx, d_dist, d_count,
+                                   olist.as<uint32_t>(), overflow_n, total_cand, stream, stats))
+        return rc;
     }
-  } else {
+  }
+  if (k > KMAX_TILED) {
     hipLaunchKernelGGL(iota_list_kernel, dim3(static_cast<unsigned>((q + 255) / 256)), dim3(256), 0,
                        stream, olist.as<uint32_t>(), overflow_n, q);
     SC_HIP(hipGetLastError());
@@ -1145,14 +1112,20 @@ int dispatch_metric(const sc_index* index, const void* d_queries, size_t q, size
 
 }  // namespace
 
-int launch_serial_exact_f32(const sc_index* index, const float* d_queries, int k,
-                            const uint32_t* list, const uint32_t* list_n, int64_t* d_idx,
-                            double* d_dist, uint32_t* d_count, hipStream_t stream) {
+int launch_serial_exact(const sc_index* index, const void* d_queries, int k, const uint32_t* list,
+                        const uint32_t* list_n, int64_t* d_idx, double* d_dist, uint32_t* d_count,
+                        hipStream_t stream) {
   ProfScope ps("knn_serial", stream);
-  hipLaunchKernelGGL((knn_serial_kernel<float, kEuclid>), dim3(512), dim3(NT), 0, stream,
-                     static_cast<const float*>(index->rows), static_cast<int64_t>(index->n),
-                     static_cast<int>(index->ld), d_queries, k, 2.0, list, list_n, d_idx, d_dist,
-                     d_count);
+  if (index->dtype == SC_F64)
+    hipLaunchKernelGGL((knn_serial_kernel<double, kEuclid>), dim3(512), dim3(NT), 0, stream,
+                       static_cast<const double*>(index->rows), static_cast<int64_t>(index->n),
+                       static_cast<int>(index->ld), static_cast<const double*>(d_queries), k, 2.0,
+                       list, list_n, d_idx, d_dist, d_count);
+  else
+    hipLaunchKernelGGL((knn_serial_kernel<float, kEuclid>), dim3(512), dim3(NT), 0, stream,
+                       static_cast<const float*>(index->rows), static_cast<int64_t>(index->n),
+                       static_cast<int>(index->ld), static_cast<const float*>(d_queries), k, 2.0,
+                       list, list_n, d_idx, d_dist, d_count);
   SC_HIP(hipGetLastError());
   return SC_OK;
 }
@@ -1172,6 +1145,9 @@ int knn_exact_device(const sc_index* index, const void* d_queries, size_t q, siz
                      sc_metric metric, int p, int64_t* d_idx, double* d_dist, uint32_t* d_count,
                      hipStream_t stream, sc_stats* stats) {
   if (q == 0) return SC_OK;
+  if (metric == SC_EUCLIDIAN && k <= KMAX_TILED)
+    return knn_f64_device(index, d_queries, static_cast<int64_t>(q), static_cast<int>(k), d_idx,
+                          d_dist, d_count, stream, stats);
   if (index->dtype == SC_F64)
     return dispatch_metric<double>(index, d_queries, q, k, metric, p, d_idx, d_dist, d_count,
                                    stream, stats);

@@ -1,0 +1,767 @@
+// Euclidian kNN in FP64 on the matrix cores (LinearKNNSearch::find,
+// linear_search.rs:52-84) for f64 and f32 rows.
+//
+//   dense    The first rows (kDenseRows) of the index: L, the lower bound on
+//            D of mfma64.hpp, of every (query, row), written out.
+//   select0  One wavefront per query walks its L values in row order with
+//            the k smallest upper bounds U seen so far across its lanes: a
+//            row whose L is below the running k-th is a candidate.
+//   scan     The rest in levels whose row ranges grow geometrically.  Each
+//            row is tested against T, the k-th smallest U of all earlier
+//            levels' candidates (at or above the k-th smallest S of the rows
+//            before the level, hence at or above the heap's threshold), and
+//            the rows below it go to a list per (query, piece), in row
+//            order.  A piece that collects many candidates (rows sorted by
+//            class, say) lowers T by its own k-th U as it goes, so lists stay
+//            short for any order of the rows that the heap itself would not
+//            thrash on.
+//   select   The k smallest U so far, with the new level's candidates.
+//   finish   One workgroup per query: S of every candidate in the
+//            reference's arithmetic and order, then HeapSelection replayed
+//            over them in row order.  A row that enters the reference heap
+//            has S below the running k-th S of the earlier rows, so the
+//            candidates are a superset of the entrants and every other row
+//            would be a no-op: the heap array, order included, and the
+//            distance bits are the reference's.
+// Queries whose lists overflow, or whose norm is out of the bound's range,
+// are recomputed by the sequential exact kernel.
+//
+// All arithmetic is FP64 (f32 rows are widened exactly); the bound's band is
+// 1e-13 of the norms for f64 rows and 2e-7 of the distance for f32 rows, so
+// hardly a row is tested in vain.
+//
+// Bound by the FP64 matrix rate (72 TFLOP/s in a large matrix product on
+// this card): 4,096 queries x 200,000 x 64 f64 rows take 2.83 ms (12.8 ms
+// with a tile of vector subtract, multiply, add), 3,001 x 750,000 x 100 f32
+// 8.5 ms (42.1), 54 TFLOP/s.  The prefix is 1,024 rows because its selection
+// is a walk per query; two levels then leave about 250 candidates per query
+// at k = 10, and one more level would cost two launches to save 100.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cmath>
+#include <mutex>
+#include <vector>
+
+#include "common.hpp"
+#include "heap.hpp"
+#include "metric.hpp"
+#include "mfma64.hpp"
+
+namespace sc {
+
+// from knn_exact.hip
+int launch_serial_exact(const sc_index* index, const void* d_queries, int k, const uint32_t* list,
+                        const uint32_t* list_n, int64_t* d_idx, double* d_dist, uint32_t* d_count,
+                        hipStream_t stream);
+
+namespace {
+
+constexpr int64_t kDenseRows = 1024;
+constexpr int kFinishThreads = 128;
+constexpr int kFinishBatch = 1024;   // candidates rescored and replayed at a time
+constexpr int kSelectWaves = 4;
+constexpr int kMaxLevels = 8;
+
+// Sixteen lanes per row: the squared norm (any order: the gap covers it).
+template <typename T>
+__device__ __forceinline__ double row_norm(const T* __restrict__ r, int ld, int sub, bool* finite) {
+  double s = 0.0;
+  bool ok = true;
+  for (int j = sub; j < ld; j += 16) {
+    const double v = static_cast<double>(r[j]);
+    ok = ok && isfinite(v);
+    s += v * v;
+  }
+#pragma unroll
+  for (int o = 8; o >= 1; o >>= 1) {
+    s += __shfl_xor(s, o, 16);
+    ok = (__shfl_xor(static_cast<int>(ok), o, 16) != 0) && ok;
+  }
+  *finite = ok;
+  return s;
+}
+
+template <typename T>
+__global__ void row_norms_kernel(const T* __restrict__ rows, int64_t n, int64_t npad, int ld,
+                                 double shrink, double* __restrict__ y2m) {
+  const int sub = threadIdx.x & 15;
+  const int64_t i = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) >> 4;
+  if (i >= npad) return;  // sixteen lanes together
+  double out = INFINITY;
+  if (i < n) {
+    bool finite;
+    const double s = row_norm(rows + i * ld, ld, sub, &finite);
+    if (finite) out = s < kNorm64Limit ? s * shrink : NAN;
+  }
+  if (sub == 0) y2m[i] = out;
+}
+
+template <typename T>
+__global__ void query_norms_kernel(const T* __restrict__ qs, int64_t q, int ld, double shrink,
+                                   double* __restrict__ x2m, uint32_t* __restrict__ list,
+                                   uint32_t* __restrict__ list_n) {
+  const int sub = threadIdx.x & 15;
+  const int64_t i = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) >> 4;
+  if (i >= q) return;
+  bool finite;
+  const double s = row_norm(qs + i * ld, ld, sub, &finite);
+  if (sub != 0) return;
+  const bool in = finite && s < kNorm64Limit;
+  x2m[i] = in ? s * shrink : INFINITY;
+  if (finite && !in) list[atomicAdd(list_n, 1u)] = static_cast<uint32_t>(i);
+}
+
+__global__ void zero_words_kernel(uint32_t* p, int64_t n) {
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
+       i += static_cast<int64_t>(gridDim.x) * blockDim.x)
+    p[i] = 0u;
+}
+
+// L of queries x the first `cols` rows (a multiple of kMR, rows past the
+// index +inf), row-major by query.  One workgroup per (query tile, row tile).
+template <typename T>
+__global__ __launch_bounds__(kMT, 2) void dense_kernel(const T* __restrict__ rows, int64_t n,
+                                                       int ld, int d,
+                                                       const double* __restrict__ y2m,
+                                                       const T* __restrict__ queries, int64_t q,
+                                                       const double* __restrict__ x2m,
+                                                       int64_t cols, double* __restrict__ out) {
+  __shared__ MSmem sm;
+  __shared__ double sx[kMQ];
+  const int64_t q0 = static_cast<int64_t>(blockIdx.x) * kMQ;
+  const int64_t tile = blockIdx.y;
+  const int tid = threadIdx.x;
+  if (tid < kMQ) sx[tid] = x2m[min(q0 + tid, q - 1)];
+  mfma64_sweep<T, true>(sm, rows, n, ld, d, y2m, queries, q, q0, 0, tile, tile + 1,
+                        [&](int64_t t, f64x4(&acc)[4][4], int par) {
+    const int lane = tid & 63, wave = tid >> 6;
+    const int wr = wave & 1, wq = wave >> 1, lr = lane & 15, lg = lane >> 4;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int rl = wr * 64 + 16 * i + lr;
+      const double y = sm.y2[par][rl];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int ql = wq * 64 + 16 * j + 4 * v + lg;
+          if (q0 + ql < q) out[(q0 + ql) * cols + t * kMR + rl] = acc[i][j][v] + (sx[ql] + y);
+        }
+    }
+  });
+}
+
+// The k smallest values a wavefront has seen, ascending in lanes 0 .. k-1.
+struct KSmallest {
+  double b;    // lane's entry
+  double kth;
+  // "none seen".  The compiler keeps a uniform f64 in a scalar register pair
+  // and writes the constant +inf there with one s_mov_b64, whose literal
+  // holds the low half only (it reads back as 0.0); the empty asm keeps the
+  // value in vector registers.
+  __device__ __forceinline__ void clear() {
+    double inf = INFINITY;
+    asm volatile("" : "+v"(inf));
+    b = inf;
+    kth = inf;
+  }
+  __device__ __forceinline__ void insert(double x, int lane, int k) {
+    double prev = __shfl_up(b, 1);
+    if (lane == 0) prev = -INFINITY;
+    if (lane < k && x < b) b = x < prev ? prev : x;
+    kth = lane_value(b, k - 1);
+  }
+};
+
+__global__ __launch_bounds__(64 * kSelectWaves) void select_dense_kernel(
+    const double* __restrict__ L, int64_t cols, const double* __restrict__ y2m,
+    const double* __restrict__ x2m, int64_t q, int k, Bound64 bd, int cap,
+    uint32_t* __restrict__ cand_idx, uint32_t* __restrict__ cand_count, double* __restrict__ seed) {
+  const int lane = threadIdx.x & 63;
+  const int64_t qi = static_cast<int64_t>(blockIdx.x) * kSelectWaves + (threadIdx.x >> 6);
+  if (qi >= q) return;  // the whole wave
+  const double x2 = x2m[qi];
+  KSmallest ks;
+  ks.clear();
+  uint32_t cnt = 0;
+  const double* l = L + qi * cols;
+  if (x2 < INFINITY) {
+    double lv = l[lane], yv = y2m[lane];
+    for (int64_t c0 = 0; c0 < cols; c0 += 64) {
+      const double cl = lv, cy = yv;
+      if (c0 + 64 < cols) {  // the next chunk's loads run under this one's work
+        lv = l[c0 + 64 + lane];
+        yv = y2m[c0 + 64 + lane];
+      }
+      const double u = sum_upper(bd, cl, x2 + cy);
+      const bool live = !(cy == INFINITY);
+      // below the running k-th (on D's scale); NaN stays a candidate
+      double th = ks.kth < INFINITY ? ks.kth * bd.up + bd.tiny : INFINITY;
+      uint64_t m = __ballot(live && !(cl >= th));
+      while (m) {
+        const int src = __builtin_ctzll(m);
+        if (cnt < static_cast<uint32_t>(cap) && lane == 0)
+          cand_idx[qi * cap + cnt] = static_cast<uint32_t>(c0 + src);
+        ++cnt;
+        const double x = lane_value(u, src);
+        m &= m - 1;
+        if (x < ks.kth) {
+          ks.insert(x, lane, k);
+          th = ks.kth < INFINITY ? ks.kth * bd.up + bd.tiny : INFINITY;
+          m &= __ballot(live && !(cl >= th));
+        }
+      }
+    }
+  }
+  if (lane < k) seed[qi * k + lane] = ks.b;
+  if (lane == 0) cand_count[qi] = cnt;
+}
+
+// One level of the scan.  Its (query tile, row tile) pairs, query tiles
+// outermost, are dealt to the workgroups in contiguous runs of `per`, so all
+// end together; the part of a run inside one query tile is a piece, with one
+// candidate list per query.  The pieces of query tile qt are the workgroups
+// from qt * tiles / per on.
+struct Level {
+  int64_t row0, tiles, per, groups;
+  int lists;  // per query
+  int cap;    // entries per list
+  int64_t entry0, list0;  // where the level's lists begin (per query)
+};
+struct ScanOut {
+  uint32_t* idx;    // q x entries
+  double* u;        // q x entries
+  uint32_t* count;  // q x lists
+  int64_t entries, lists;  // per query, all levels
+};
+
+template <typename T>
+__global__ __launch_bounds__(kMT, 2) void scan_kernel(
+    const T* __restrict__ rows, int64_t n, int ld, int d, const double* __restrict__ y2m,
+    const T* __restrict__ queries, int64_t q, const double* __restrict__ x2m,
+    const double* __restrict__ seed, int k, Bound64 bd, Level lv, ScanOut out) {
+  __shared__ MSmem sm;
+  __shared__ double sx[kMQ], sth[kMQ];
+  __shared__ uint32_t mask[kMQ][kMR / 32];
+  __shared__ uint32_t cnt[kMQ], mark[kMQ];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = tid >> 6;
+  const int wr = wave & 1, wq = wave >> 1, lr = lane & 15, lg = lane >> 4;
+  const int64_t nqt = (q + kMQ - 1) / kMQ;
+  const uint32_t grow = static_cast<uint32_t>(max(2 * k, 32));
+  int64_t pos = static_cast<int64_t>(blockIdx.x) * lv.per;
+  const int64_t end = min(pos + lv.per, nqt * lv.tiles);
+  while (pos < end) {
+    const int64_t qt = pos / lv.tiles;
+    const int64_t tb = pos - qt * lv.tiles;
+    const int64_t te = min(lv.tiles, tb + (end - pos));
+    const int list = static_cast<int>(blockIdx.x - qt * lv.tiles / lv.per);
+    const int64_t q0 = qt * kMQ;
+    __syncthreads();  // the previous piece's last reads
+    if (tid < kMQ) {
+      const int64_t qi = q0 + tid;
+      const double x2 = qi < q ? x2m[qi] : INFINITY;
+      sx[tid] = x2;
+      // queries that take no part: nothing is below -inf
+      sth[tid] = x2 < INFINITY ? acc_threshold(bd, seed[qi * k + k - 1], x2) : -INFINITY;
+      cnt[tid] = 0u;
+      mark[tid] = 0u;
+#pragma unroll
+      for (int w = 0; w < kMR / 32; ++w) mask[tid][w] = 0u;
+    }
+    auto slot_of = [&](int ql, uint32_t c) {
+      return (q0 + ql) * out.entries + lv.entry0 + static_cast<int64_t>(list) * lv.cap + c;
+    };
+    mfma64_sweep<T, false>(sm, rows, n, ld, d, y2m, queries, q, q0, lv.row0, tb, te,
+                           [&](int64_t t, f64x4(&acc)[4][4], int par) {
+      // acc[i][j][v]: row wr 64 + 16 i + 4 v + lg, query wq 64 + 16 j + lr
+      uint32_t hm[4];
+      bool any = false;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const double th = sth[wq * 64 + 16 * j + lr];
+        hm[j] = 0u;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int v = 0; v < 4; ++v)
+            hm[j] |= static_cast<uint32_t>(!(acc[i][j][v] >= th)) << (4 * i + v);
+        if (!(th > -INFINITY)) hm[j] = 0u;
+        any = any || hm[j] != 0u;
+      }
+      if (any) {
+        // rows left out (padding, non-finite) drop; the others mark their bit
+        any = false;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          uint32_t m = hm[j];
+          while (m) {
+            const int b = __builtin_ctz(m);
+            m &= m - 1;
+            const int rl = wr * 64 + 16 * (b >> 2) + 4 * (b & 3) + lg;
+            if (sm.y2[par][rl] == INFINITY)
+              hm[j] &= ~(1u << b);
+            else
+              atomicOr(&mask[wq * 64 + 16 * j + lr][rl >> 5], 1u << (rl & 31));
+          }
+          any = any || hm[j] != 0u;
+        }
+      }
+      if (!__syncthreads_or(any)) return;
+      const int64_t r0 = lv.row0 + t * kMR;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (hm[j] == 0u) continue;
+        const int ql = wq * 64 + 16 * j + lr;
+        const uint32_t base = cnt[ql];
+        const double x2 = sx[ql];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            if (!((hm[j] >> (4 * i + v)) & 1u)) continue;
+            const int rl = wr * 64 + 16 * i + 4 * v + lg;
+            // the place in row order: the marked rows before this one
+            uint32_t c = base + __popc(mask[ql][rl >> 5] & ((1u << (rl & 31)) - 1u));
+            for (int w = 0; w < (rl >> 5); ++w) c += __popc(mask[ql][w]);
+            if (c < static_cast<uint32_t>(lv.cap)) {
+              const int64_t s = slot_of(ql, c);
+              out.idx[s] = static_cast<uint32_t>(r0 + rl);
+              out.u[s] = sum_upper(bd, acc[i][j][v] + x2, x2 + sm.y2[par][rl]);
+            }
+          }
+      }
+      __syncthreads();
+      bool grown = false;
+      if (tid < kMQ) {
+        uint32_t c = 0;
+#pragma unroll
+        for (int w = 0; w < kMR / 32; ++w) {
+          c += __popc(mask[tid][w]);
+          mask[tid][w] = 0u;
+        }
+        if (c) {
+          c += cnt[tid];
+          cnt[tid] = c;
+          grown = c - mark[tid] >= grow;
+        }
+      }
+      if (!__syncthreads_or(grown)) return;
+      // lists that grew by `grow` since they were last looked at: their own
+      // k-th U is a threshold too
+      for (int ql = wave; ql < kMQ; ql += kMT / 64) {
+        const uint32_t c = cnt[ql];
+        if (c - mark[ql] < grow) continue;  // the same for the whole wave
+        const uint32_t m = min(c, static_cast<uint32_t>(lv.cap));
+        KSmallest ks;
+        ks.clear();
+        const double* u = out.u + slot_of(ql, 0);
+        for (uint32_t c0 = 0; c0 < m; c0 += 64) {
+          const double x = c0 + lane < m ? u[c0 + lane] : INFINITY;
+          uint64_t b = __ballot(x < ks.kth);
+          while (b) {
+            const int src = __builtin_ctzll(b);
+            ks.insert(lane_value(x, src), lane, k);
+            b &= b - 1;
+            b &= __ballot(x < ks.kth);
+          }
+        }
+        if (lane == 0) {
+          const double th = acc_threshold(bd, ks.kth, sx[ql]);
+          if (th < sth[ql]) sth[ql] = th;
+          mark[ql] = c;
+        }
+      }
+      __syncthreads();
+    });
+    __syncthreads();
+    if (tid < kMQ && q0 + tid < q) out.count[(q0 + tid) * out.lists + lv.list0 + list] = cnt[tid];
+    pos += te - tb;
+  }
+}
+
+// The k smallest U of the earlier levels (seed) and the entries of one
+// level's lists, in place.
+__global__ __launch_bounds__(64 * kSelectWaves) void select_level_kernel(Level lv, ScanOut in,
+                                                                         int64_t q, int k,
+                                                                         double* __restrict__ seed) {
+  const int lane = threadIdx.x & 63;
+  const int64_t qi = static_cast<int64_t>(blockIdx.x) * kSelectWaves + (threadIdx.x >> 6);
+  if (qi >= q) return;  // the whole wave
+  KSmallest ks;
+  ks.b = lane < k ? seed[qi * k + lane] : INFINITY;
+  ks.kth = lane_value(ks.b, k - 1);
+  const uint32_t* cc = in.count + qi * in.lists + lv.list0;
+  const double* u = in.u + qi * in.entries + lv.entry0;
+  for (int l0 = 0; l0 < lv.lists; l0 += 64) {
+    // 64 counts at once, then the non-empty lists one by one
+    const uint32_t cl = l0 + lane < lv.lists ? min(cc[l0 + lane], static_cast<uint32_t>(lv.cap)) : 0u;
+    uint64_t some = __ballot(cl != 0u);
+    while (some) {
+      const int li = __builtin_ctzll(some);
+      some &= some - 1;
+      const uint32_t c = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(cl), li));
+      const double* ul = u + static_cast<int64_t>(l0 + li) * lv.cap;
+      for (uint32_t c0 = 0; c0 < c; c0 += 64) {
+        const double x = c0 + lane < c ? ul[c0 + lane] : INFINITY;
+        uint64_t m = __ballot(x < ks.kth);
+        while (m) {
+          const int src = __builtin_ctzll(m);
+          ks.insert(lane_value(x, src), lane, k);
+          m &= m - 1;
+          m &= __ballot(x < ks.kth);
+        }
+      }
+    }
+  }
+  if (lane < k) seed[qi * k + lane] = ks.b;
+}
+
+// Where the lists of a query lie: list 0 is the dense prefix's (its own
+// array), then each level's.
+struct Lists {
+  const uint32_t* pre_idx;
+  const uint32_t* pre_count;
+  int pre_cap;
+  ScanOut out;
+  int nlevels;
+  Level lv[kMaxLevels];
+};
+
+// S of every candidate and the heap replay (see the file comment).  The
+// candidates are numbered across the lists by a prefix sum of the counts and
+// taken kFinishBatch at a time: all threads compute their S, then the first
+// wavefront replays the batch from LDS, 64 entries at a time.
+template <typename T>
+__global__ __launch_bounds__(kFinishThreads) void finish_kernel(
+    const T* __restrict__ rows, int ld, const T* __restrict__ queries, int64_t q, int k, Lists ls,
+    int64_t* __restrict__ out_idx, double* __restrict__ out_dist, uint32_t* __restrict__ out_count,
+    uint32_t* __restrict__ list, uint32_t* __restrict__ list_n,
+    unsigned long long* __restrict__ total_cand) {
+  constexpr int PV = 16 / sizeof(T);
+  typedef T Piece __attribute__((ext_vector_type(PV)));
+  extern __shared__ __align__(16) uint32_t start[];  // nl + 1
+  __shared__ double s_S[kFinishBatch];
+  __shared__ uint32_t s_row[kFinishBatch];
+  __shared__ uint32_t s_over;
+  const int64_t qi = blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int nl = 1 + static_cast<int>(ls.out.lists);
+  if (tid == 0) s_over = 0u;
+  __syncthreads();
+  if (tid < 64) {
+    uint32_t acc = 0;
+    bool over = false;
+    for (int l0 = 0; l0 < nl; l0 += 64) {
+      const int l = l0 + lane;
+      uint32_t c = 0;
+      if (l < nl) {
+        c = l == 0 ? ls.pre_count[qi] : ls.out.count[qi * ls.out.lists + l - 1];
+        int cap = ls.pre_cap;
+        if (l > 0) {
+          cap = ls.lv[0].cap;
+          for (int v = 1; v < ls.nlevels; ++v)
+            if (l - 1 >= ls.lv[v].list0) cap = ls.lv[v].cap;
+        }
+        over = over || c > static_cast<uint32_t>(cap);
+      }
+      uint32_t inc = c;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t up = __shfl_up(inc, o);
+        if (lane >= o) inc += up;
+      }
+      if (l < nl) start[l] = acc + inc - c;
+      acc += __shfl(inc, 63);
+    }
+    if (lane == 0) start[nl] = acc;
+    if (__ballot(over) != 0 && lane == 0) {
+      s_over = 1u;
+      list[atomicAdd(list_n, 1u)] = static_cast<uint32_t>(qi);
+      out_count[qi] = 0u;
+    }
+  }
+  __syncthreads();
+  if (s_over) return;
+  const uint32_t total = start[nl];
+  const T* qrow = queries + qi * ld;
+  double hd = INFINITY, top = INFINITY;
+  uint32_t hi = 0xffffffffu;
+  for (uint32_t e0 = 0; e0 < total; e0 += kFinishBatch) {
+    const uint32_t m = min(total - e0, static_cast<uint32_t>(kFinishBatch));
+    for (uint32_t e = tid; e < m; e += kFinishThreads) {
+      // the list of candidate e0 + e: the last whose start is at or below it
+      int lo = 0, hi_l = nl;
+      while (hi_l - lo > 1) {
+        const int mid = (lo + hi_l) >> 1;
+        if (start[mid] <= e0 + e)
+          lo = mid;
+        else
+          hi_l = mid;
+      }
+      const uint32_t at = e0 + e - start[lo];
+      uint32_t row;
+      if (lo == 0) {
+        row = ls.pre_idx[qi * ls.pre_cap + at];
+      } else {
+        int v = 0;
+        while (v + 1 < ls.nlevels && lo - 1 >= ls.lv[v + 1].list0) ++v;
+        row = ls.out.idx[qi * ls.out.entries + ls.lv[v].entry0 +
+                         (lo - 1 - ls.lv[v].list0) * ls.lv[v].cap + at];
+      }
+      const Piece* r = reinterpret_cast<const Piece*>(rows + static_cast<int64_t>(row) * ld);
+      const Piece* x = reinterpret_cast<const Piece*>(qrow);
+      double s = 0.0;
+      for (int j = 0; j < ld / PV; j += 16 / PV) {
+        Piece rv[16 / PV], xv[16 / PV];
+#pragma unroll
+        for (int c = 0; c < 16 / PV; ++c) {
+          rv[c] = r[j + c];
+          xv[c] = x[j + c];
+        }
+#pragma unroll
+        for (int c = 0; c < 16 / PV; ++c)
+#pragma unroll
+          for (int w = 0; w < PV; ++w) s = s + Term<T, kEuclid>::f(xv[c][w], rv[c][w], 2.0);
+      }
+      s_S[e] = s;
+      s_row[e] = row;
+    }
+    __syncthreads();
+    if (tid < 64) {
+      for (uint32_t c0 = 0; c0 < m; c0 += 64) {
+        const bool valid = c0 + lane < m;
+        const double dv = valid ? __builtin_sqrt(s_S[c0 + lane]) : 0.0;
+        const uint32_t row = valid ? s_row[c0 + lane] : 0u;
+        uint64_t b = __ballot(valid && dv < top);
+        while (b) {
+          const int src = __builtin_ctzll(b);
+          lane_heap_push_root(hd, hi, lane, k, lane_value(dv, src),
+                              static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(row), src)));
+          top = lane_value(hd, 0);
+          b &= b - 1;
+          b &= __ballot(valid && dv < top);
+        }
+      }
+    }
+    __syncthreads();
+  }
+  if (tid < 64) {
+    if (lane == 0) atomicAdd(total_cand, static_cast<unsigned long long>(total));
+    lane_heap_store(hd, hi, lane, k, out_idx + qi * k, out_dist + qi * k, out_count + qi);
+  }
+}
+
+template <typename T>
+int run_f64(const sc_index* index, const T* d_queries, int64_t q, int k, int64_t* d_idx,
+            double* d_dist, uint32_t* d_count, hipStream_t s, sc_stats* stats) {
+  const int64_t n = static_cast<int64_t>(index->n);
+  const int ld = static_cast<int>(index->ld), d = static_cast<int>(index->d);
+  const T* rows = static_cast<const T*>(index->rows);
+  const Bound64 bd = bound64<T>(ld);
+  DevBuf local;
+  const double* y2m = nullptr;
+  if (int rc = ensure_norms64(const_cast<sc_index*>(index), local, &y2m, s)) return rc;
+
+  // Levels: the dense prefix, then m ranges growing by the same factor (at
+  // most 16: k (factor - 1) candidates per query and level against one scan
+  // and one selection launch for a further level).
+  const int64_t cols = std::min<int64_t>(kDenseRows, (n + kMR - 1) / kMR * kMR);
+  std::vector<int64_t> edge{cols};
+  if (n > cols) {
+    const double span = static_cast<double>(n) / static_cast<double>(cols);
+    const int m = std::max(1, std::min(kMaxLevels, static_cast<int>(std::ceil(std::log(span) / std::log(16.0)))));
+    for (int i = 1; i < m; ++i)
+      edge.push_back(std::max<int64_t>(
+          edge.back() + kMR, static_cast<int64_t>(cols * std::pow(span, double(i) / m)) / kMR * kMR));
+    edge.push_back(n);
+  }
+  const int nlev = static_cast<int>(edge.size()) - 1;
+  auto expect = [&](double len) { return k * (1.0 + std::log(std::max(1.0, len / k))); };
+  const int pre_cap = static_cast<int>(std::min<int64_t>(cols, static_cast<int64_t>(3.0 * expect(cols)) + 64));
+  auto plan = [&](int64_t qn, Level (&lv)[kMaxLevels], ScanOut& o) {
+    const int64_t nqt = (qn + kMQ - 1) / kMQ;
+    o.entries = o.lists = 0;
+    for (int i = 0; i < nlev; ++i) {
+      Level& v = lv[i];
+      v.row0 = edge[i];
+      v.tiles = (edge[i + 1] - edge[i] + kMR - 1) / kMR;
+      const int64_t items = nqt * v.tiles;
+      // two workgroups per CU fit (LDS and registers)
+      v.per = std::max<int64_t>(1, (items + 511) / 512);
+      v.groups = (items + v.per - 1) / v.per;
+      v.lists = static_cast<int>(std::min<int64_t>((v.tiles + v.per - 1) / v.per + 1, v.tiles));
+      const int64_t len = std::min<int64_t>(v.per * kMR, v.tiles * kMR);
+      // a tile that passes whole, one look's growth, and the running-k-th
+      // improvements after it with room to spare
+      v.cap = static_cast<int>(std::min<int64_t>(
+          len, kMR + std::max(2 * k, 32) + static_cast<int64_t>(4.0 * expect(static_cast<double>(len)))));
+      v.entry0 = o.entries;
+      v.list0 = o.lists;
+      o.entries += static_cast<int64_t>(v.lists) * v.cap;
+      o.lists += v.lists;
+    }
+  };
+  Lists ls{};
+  ls.nlevels = nlev;
+  ls.pre_cap = pre_cap;
+  // the candidate store of a call is bounded by batches of queries (whole
+  // query tiles); a smaller batch has longer lists per query, so the size is
+  // found by halving
+  int64_t qb = q;
+  for (;;) {
+    plan(qb, ls.lv, ls.out);
+    const double bytes = static_cast<double>(qb) * (12.0 * ls.out.entries + 4.0 * ls.out.lists +
+                                                    4.0 * pre_cap + 8.0 * (cols + k + 1));
+    if (bytes <= 1.5 * 1024.0 * 1024.0 * 1024.0 || qb <= kMQ) break;
+    qb = std::max<int64_t>(kMQ, (qb / 2 + kMQ - 1) / kMQ * kMQ);
+  }
+  DevBuf flags, olist, x2m, dense, pidx, pcnt, cidx, cu, ccnt, seed;
+  SC_HIP(flags.alloc(64, s));  // [0] listed queries, [2..3] candidate total (u64)
+  SC_HIP(olist.alloc(sizeof(uint32_t) * qb, s));
+  SC_HIP(x2m.alloc(sizeof(double) * qb, s));
+  SC_HIP(dense.alloc(sizeof(double) * qb * cols, s));
+  SC_HIP(pidx.alloc(sizeof(uint32_t) * qb * pre_cap, s));
+  SC_HIP(pcnt.alloc(sizeof(uint32_t) * qb, s));
+  SC_HIP(seed.alloc(sizeof(double) * qb * k, s));
+  SC_HIP(cidx.alloc(sizeof(uint32_t) * qb * ls.out.entries, s));
+  SC_HIP(cu.alloc(sizeof(double) * qb * ls.out.entries, s));
+  SC_HIP(ccnt.alloc(sizeof(uint32_t) * qb * ls.out.lists, s));
+  uint32_t* list_n = flags.as<uint32_t>();
+  unsigned long long* total = reinterpret_cast<unsigned long long*>(flags.as<char>() + 8);
+  hipLaunchKernelGGL(zero_words_kernel, dim3(1), dim3(64), 0, s, flags.as<uint32_t>(), int64_t{16});
+  for (int64_t b0 = 0; b0 < q; b0 += qb) {
+    const int64_t qn = std::min(qb, q - b0);
+    const T* qs = d_queries + b0 * ld;
+    if (qn != qb) plan(qn, ls.lv, ls.out);
+    if (ls.out.entries > 0 && qn != qb && (ls.out.entries * qn > static_cast<int64_t>(cidx.cap / 4) ||
+                                           ls.out.lists * qn > static_cast<int64_t>(ccnt.cap / 4))) {
+      // a short last batch spreads over more pieces
+      SC_HIP(cidx.alloc(sizeof(uint32_t) * qn * ls.out.entries, s));
+      SC_HIP(cu.alloc(sizeof(double) * qn * ls.out.entries, s));
+      SC_HIP(ccnt.alloc(sizeof(uint32_t) * qn * ls.out.lists, s));
+    }
+    ls.pre_idx = pidx.as<uint32_t>();
+    ls.pre_count = pcnt.as<uint32_t>();
+    ls.out.idx = cidx.as<uint32_t>();
+    ls.out.u = cu.as<double>();
+    ls.out.count = ccnt.as<uint32_t>();
+    hipLaunchKernelGGL(zero_words_kernel, dim3(1), dim3(64), 0, s, list_n, int64_t{1});
+    if (int rc = query_norms64<T>(qs, qn, ld, x2m.as<double>(), olist.as<uint32_t>(), list_n, s)) return rc;
+    const unsigned nqt = static_cast<unsigned>((qn + kMQ - 1) / kMQ);
+    const unsigned sel = static_cast<unsigned>((qn + kSelectWaves - 1) / kSelectWaves);
+    {
+      ProfScope ps("knn_scan", s);
+      hipLaunchKernelGGL(dense_kernel<T>, dim3(nqt, static_cast<unsigned>(cols / kMR)), dim3(kMT), 0,
+                         s, rows, n, ld, d, y2m, qs, qn, x2m.as<double>(), cols, dense.as<double>());
+      hipLaunchKernelGGL(select_dense_kernel, dim3(sel), dim3(64 * kSelectWaves), 0, s,
+                         dense.as<double>(), cols, y2m, x2m.as<double>(), qn, k, bd, pre_cap,
+                         pidx.as<uint32_t>(), pcnt.as<uint32_t>(), seed.as<double>());
+      SC_HIP(hipGetLastError());
+      if (nlev > 0) {
+        // pieces that a level does not have leave empty lists
+        const int64_t w = qn * ls.out.lists;
+        hipLaunchKernelGGL(zero_words_kernel, dim3(static_cast<unsigned>(std::min<int64_t>(1024, (w + 255) / 256))),
+                           dim3(256), 0, s, ls.out.count, w);
+      }
+      for (int i = 0; i < nlev; ++i) {
+        hipLaunchKernelGGL(scan_kernel<T>, dim3(static_cast<unsigned>(ls.lv[i].groups)), dim3(kMT), 0,
+                           s, rows, n, ld, d, y2m, qs, qn, x2m.as<double>(), seed.as<double>(), k, bd,
+                           ls.lv[i], ls.out);
+        if (i + 1 < nlev)
+          hipLaunchKernelGGL(select_level_kernel, dim3(sel), dim3(64 * kSelectWaves), 0, s, ls.lv[i],
+                             ls.out, qn, k, seed.as<double>());
+        SC_HIP(hipGetLastError());
+      }
+    }
+    {
+      ProfScope ps("knn_replay", s);
+      hipLaunchKernelGGL(finish_kernel<T>, dim3(static_cast<unsigned>(qn)), dim3(kFinishThreads),
+                         sizeof(uint32_t) * (ls.out.lists + 2), s, rows, ld, qs, qn, k, ls,
+                         d_idx + b0 * k, d_dist + b0 * k, d_count + b0, olist.as<uint32_t>(), list_n,
+                         total);
+      SC_HIP(hipGetLastError());
+    }
+    if (int rc = launch_serial_exact(index, qs, k, olist.as<uint32_t>(), list_n, d_idx + b0 * k,
+                                     d_dist + b0 * k, d_count + b0, s))
+      return rc;
+    if (stats) {
+      uint64_t h[2] = {0, 0};
+      SC_HIP(hipMemcpyAsync(h, flags.p, 16, hipMemcpyDeviceToHost, s));
+      SC_HIP(hipStreamSynchronize(s));
+      stats->overflow_queries += static_cast<uint32_t>(h[0]);
+      if (b0 + qn >= q) stats->candidates += h[1];
+    }
+  }
+  if (stats) stats->queries += static_cast<uint64_t>(q);
+  return SC_OK;
+}
+
+}  // namespace
+
+int ensure_norms64(sc_index* ix, DevBuf& local, const double** y2m, hipStream_t s) {
+  const int64_t n = static_cast<int64_t>(ix->n);
+  const int64_t npad = std::max<int64_t>(kMR, (n + kMR - 1) / kMR * kMR);
+  const int ld = static_cast<int>(ix->ld);
+  const double shrink = 1.0 - norm_gap(ld);
+  auto launch = [&](double* out) -> int {
+    const dim3 grid(static_cast<unsigned>((npad * 16 + 255) / 256));
+    if (ix->dtype == SC_F64)
+      hipLaunchKernelGGL(row_norms_kernel<double>, grid, dim3(256), 0, s,
+                         static_cast<const double*>(ix->rows), n, npad, ld, shrink, out);
+    else
+      hipLaunchKernelGGL(row_norms_kernel<float>, grid, dim3(256), 0, s,
+                         static_cast<const float*>(ix->rows), n, npad, ld, shrink, out);
+    SC_HIP(hipGetLastError());
+    return SC_OK;
+  };
+  std::lock_guard<std::mutex> lk(*static_cast<std::mutex*>(ix->mu));
+  if (ix->norms64) {
+    *y2m = ix->norms64;
+    return SC_OK;
+  }
+  if (stream_capturing(s)) {
+    SC_HIP(local.alloc(sizeof(double) * npad, s));
+    if (int rc = launch(local.as<double>())) return rc;
+    *y2m = local.as<double>();
+    return SC_OK;
+  }
+  double* p = nullptr;
+  SC_HIP(hipMalloc(reinterpret_cast<void**>(&p), sizeof(double) * npad));
+  int rc = launch(p);
+  if (rc == SC_OK) {
+    // calls on other streams may follow at once
+    const hipError_t e = hipStreamSynchronize(s);
+    if (e != hipSuccess) rc = hip_fail(e, "row norms");
+  }
+  if (rc != SC_OK) {
+    (void)hipFree(p);
+    return rc;
+  }
+  ix->norms64 = p;
+  *y2m = p;
+  return SC_OK;
+}
+
+template <typename T>
+int query_norms64(const T* queries, int64_t q, int ld, double* x2m, uint32_t* list,
+                  uint32_t* list_n, hipStream_t s) {
+  hipLaunchKernelGGL(query_norms_kernel<T>, dim3(static_cast<unsigned>((q * 16 + 255) / 256)), dim3(256),
+                     0, s, queries, q, ld, 1.0 - norm_gap(ld), x2m, list, list_n);
+  SC_HIP(hipGetLastError());
+  return SC_OK;
+}
+template int query_norms64<double>(const double*, int64_t, int, double*, uint32_t*, uint32_t*, hipStream_t);
+template int query_norms64<float>(const float*, int64_t, int, double*, uint32_t*, uint32_t*, hipStream_t);
+
+int knn_f64_device(const sc_index* index, const void* d_queries, int64_t q, int k, int64_t* d_idx,
+                   double* d_dist, uint32_t* d_count, hipStream_t stream, sc_stats* stats) {
+  if (index->dtype == SC_F64)
+    return run_f64(index, static_cast<const double*>(d_queries), q, k, d_idx, d_dist, d_count,
+                   stream, stats);
+  return run_f64(index, static_cast<const float*>(d_queries), q, k, d_idx, d_dist, d_count, stream,
+                 stats);
+}
+
+}  // namespace sc

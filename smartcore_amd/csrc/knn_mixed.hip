@@ -66,14 +66,15 @@
 #include <vector>
 
 #include "common.hpp"
+#include "heap.hpp"
 #include "metric.hpp"
 
 namespace sc {
 
 // from knn_exact.hip
-int launch_serial_exact_f32(const sc_index* index, const float* d_queries, int k,
-                            const uint32_t* list, const uint32_t* list_n, int64_t* d_idx,
-                            double* d_dist, uint32_t* d_count, hipStream_t stream);
+int launch_serial_exact(const sc_index* index, const void* d_queries, int k, const uint32_t* list,
+                        const uint32_t* list_n, int64_t* d_idx, double* d_dist, uint32_t* d_count,
+                        hipStream_t stream);
 
 namespace {
 
@@ -854,16 +855,6 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
-__device__ __forceinline__ double lane_value(double v, int l) {
-  const int lo = __builtin_amdgcn_readlane(static_cast<int>(__double_as_longlong(v)), l);
-  const int hi = __builtin_amdgcn_readlane(static_cast<int>(__double_as_longlong(v) >> 32), l);
-  return __longlong_as_double((static_cast<long long>(hi) << 32) |
-                              static_cast<unsigned long long>(static_cast<uint32_t>(lo)));
-}
-__device__ __forceinline__ float lane_value(float v, int l) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
-}
-
 // The k smallest of a seed (null: +inf) and the exact distances, rounded
 // up to f32, of the entries in lists [l0, l0 + nl) (candidates of rows after
 // the seed's rows, distinct): the next seed, ascending.  Entries past a
@@ -901,45 +892,6 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void select_seed_kernel(
     }
   }
   if (lane < k) seed_out[qi * k + lane] = b;
-}
-
-// The reference heap (heap_select.rs) held across a wave's lanes: lane j < k
-// holds entry j (distance hd, row hi).  Replacing the root and sifting it
-// down follows HeapSelection::sift_down (heap_select.rs:71-86: the children
-// of kk are 2kk and 2kk + 1; stop on Equal or Greater) with the node values
-// read by readlane and the swap done by a select in every lane, so an
-// insertion costs a few instructions per level and no memory traffic.
-__device__ __forceinline__ void lane_heap_push_root(double& hd, uint32_t& hi, int lane, int k,
-                                                    double d, uint32_t row) {
-  if (lane == 0) {
-    hd = d;
-    hi = row;
-  }
-  const int n = k - 1;
-  int kk = 0;
-  double vk = d;
-  while (2 * kk <= n) {
-    int j = 2 * kk;
-    double vj = lane_value(hd, j);
-    if (j < n) {
-      const double vj1 = lane_value(hd, j + 1);
-      if (vj < vj1) {
-        j += 1;
-        vj = vj1;
-      }
-    }
-    if (vk == vj || vk > vj) break;
-    const uint32_t ij = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(hi), j));
-    const uint32_t ik = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(hi), kk));
-    if (lane == kk) {
-      hd = vj;
-      hi = ij;
-    } else if (lane == j) {
-      hd = vk;
-      hi = ik;
-    }
-    kk = j;
-  }
 }
 
 // Pass 2a: the exact s of every stored candidate (the reference's
@@ -1110,20 +1062,7 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void mixed_replay_kernel(
     atomicAdd(&counters[0], seen);
     atomicAdd(&counters[1], seen);
   }
-  // the heap array without its empty slots, in heap order
-  const bool full = lane < k && hi != 0xffffffffu;
-  const uint64_t fm = __ballot(full);
-  const int c = __popcll(fm);
-  if (full) {
-    const int pos = __popcll(fm & ((uint64_t(1) << lane) - 1));
-    out_idx[qi * k + pos] = static_cast<int64_t>(hi);
-    out_dist[qi * k + pos] = hd;
-  }
-  if (lane >= c && lane < k) {
-    out_idx[qi * k + lane] = -1;
-    out_dist[qi * k + lane] = NAN;
-  }
-  if (lane == 0) out_count[qi] = static_cast<uint32_t>(c);
+  lane_heap_store(hd, hi, lane, k, out_idx + qi * k, out_dist + qi * k, out_count + qi);
 }
 
 // Builds the BF16 copy and row terms of an f32 index once.  ldb (the BF16
@@ -1414,7 +1353,7 @@ int knn_mixed_device(const sc_index* cix, const void* d_queries, size_t q_, size
                        lst.as<uint32_t>(), list_n, counters);
     SC_HIP(hipGetLastError());
   }
-  if (int rc = launch_serial_exact_f32(ix, qf, k, lst.as<uint32_t>(), list_n, d_idx, d_dist,
+  if (int rc = launch_serial_exact(ix, qf, k, lst.as<uint32_t>(), list_n, d_idx, d_dist,
                                        d_count, stream))
     return rc;
   if (stats) {

@@ -1,0 +1,225 @@
+// FP64 MFMA tile sweep shared by the Euclidian searches.
+//
+// A 256-thread workgroup sweeps 128-row tiles of the index against 128
+// queries.  Wave (wr, wq) of the 2 x 2 arrangement owns 64 rows x 64 queries
+// as 4 x 4 v_mfma_f64_16x16x4_f64 accumulators (128 VGPRs), so a K step of
+// four dimensions costs 8 LDS reads for 16 MFMAs and the kernel is bound by
+// the matrix pipe (64 cycles per MFMA and SIMD): the vector form needs
+// three FP64 instructions per element (subtract, multiply, add) where the
+// MFMA needs one fused multiply-add.  Dimension chunks of 16 go through two
+// LDS buffers: chunk c + 1 is stored and chunk c + 2 requested while chunk
+// c's MFMAs run, with one barrier per chunk; the chunk stream runs on across
+// tiles, so a tile's first chunk is as early as any other.  f32 rows are
+// widened (exactly) when they are stored to LDS.
+//
+// The accumulators start at y2m, a lower bound of the row's ||y||^2, and the
+// queries are staged as -2x, so a tile ends with acc = y2m - 2 x.y.
+//
+// Bound.  With D = ||x - y||^2 exactly, u = 2^-53 and any order of the
+// accumulation, the MFMA chain's error is at most 2 ld u (x2 + y2) for the
+// products' sum plus the same for the running sum that contains y2m, and the
+// norms carry (ld + 1) u each.  norm_gap(ld) = g = (4 ld + 32) 2^-52 is above
+// all of it, so with x2m = (1 - g) x2 and y2m = (1 - g) y2
+//   L = x2m + acc <= D <= L + 2.5 g (x2m + y2m).
+// The reference's sum S (euclidian.rs:57-62) is within sum_eps of D in
+// relative terms and sum_tiny absolutely (f32 squares may underflow), so
+//   S < T  implies  acc < T (1 + 3 eps) + 2 tiny - x2m.
+// Rows with a non-finite value never enter the reference heap or pass a
+// radius test (their S is inf or NaN); they carry y2m = +inf and are left
+// out.  Rows whose squared norm reaches kNorm64Limit carry NaN: comparisons
+// are written so that NaN is always a candidate, and exact arithmetic
+// decides.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "common.hpp"
+
+namespace sc {
+
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kMQ = 128;       // queries per workgroup tile
+constexpr int kMR = 128;       // rows per tile
+constexpr int kMD = 16;        // dimensions per chunk
+constexpr int kMT = 256;       // threads
+// LDS row stride of a chunk: 16 values + 2, so the 16 rows x 4 dimensions a
+// wave reads with one ds_read_b64 fall on every bank exactly twice
+constexpr int kMStride = kMD + 2;
+constexpr double kNorm64Limit = 1e290;
+
+inline double norm_gap(int ld) { return (4.0 * ld + 32.0) * 2.220446049250313e-16; }
+template <typename T>
+inline double sum_eps(int ld) {
+  // f64: three roundings per term and ld adds; f32: two f32 roundings of
+  // the difference (squared) and one of the square, then the f64 fold
+  return sizeof(T) == 8 ? (ld + 8.0) * 2.220446049250313e-16
+                        : 2.384185791015625e-07 + (ld + 8.0) * 2.220446049250313e-16;
+}
+template <typename T>
+inline double sum_tiny(int ld) {
+  return sizeof(T) == 8 ? 1e-300 : ld * 2.802596928649634e-45;
+}
+// Above this a sum may overflow in the reference's own type.
+template <typename T>
+inline double sum_limit() {
+  return sizeof(T) == 8 ? 1e300 : 1e38;
+}
+// The bound's constants as the kernels take them.
+struct Bound64 {
+  double gap25;   // 2.5 g
+  double up;      // 1 + 3 eps
+  double tiny;    // 2 tiny
+  double limit;
+};
+template <typename T>
+inline Bound64 bound64(int ld) {
+  return Bound64{2.5 * norm_gap(ld), 1.0 + 3.0 * sum_eps<T>(ld), 2.0 * sum_tiny<T>(ld),
+                 sum_limit<T>()};
+}
+// The accumulator threshold that every row with S < t is below.
+__device__ __forceinline__ double acc_threshold(const Bound64& b, double t, double x2m) {
+  return t < INFINITY ? t * b.up + b.tiny - x2m : INFINITY;
+}
+// An upper bound on S of a pair whose lower bound on D is L.
+__device__ __forceinline__ double sum_upper(const Bound64& b, double L, double norms) {
+  const double u = (L + b.gap25 * norms) * b.up + b.tiny;
+  return u < b.limit ? u : INFINITY;  // NaN too
+}
+
+struct MSmem {
+  double R[2][kMR][kMStride];
+  double Q[2][kMQ][kMStride];
+  double y2[2][kMR];  // y2m of the tile, by tile parity
+};
+
+// Sweeps tiles tb .. te - 1 (row = row0 + 128 tile) against queries
+// q0 .. q0 + 127; epi(t, acc, parity) runs on all threads at each tile's
+// end (it may synchronise).  Out-of-range rows and queries are read clamped:
+// y2m carries +inf past the last row.  SWAP: the accumulators hold
+// (query, row) transposed -- lane column = row -- and start at zero.
+template <typename T, bool SWAP, typename Epi>
+__device__ __forceinline__ void mfma64_sweep(MSmem& sm, const T* __restrict__ rows, int64_t n,
+                                             int ld, int d, const double* __restrict__ y2m,
+                                             const T* __restrict__ queries, int64_t q, int64_t q0,
+                                             int64_t row0, int64_t tb, int64_t te, Epi epi) {
+  constexpr int PV = 16 / sizeof(T);            // values per 16-byte piece
+  constexpr int PR = kMD / PV;                  // pieces per row of a chunk
+  constexpr int NP = kMR * PR / kMT;            // pieces per thread (rows and queries each)
+  typedef T Piece __attribute__((ext_vector_type(PV)));
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = tid >> 6;
+  const int wr = wave & 1, wq = wave >> 1;
+  const int lr = lane & 15, lg = lane >> 4;
+  const int nch = d > kMD ? (d + kMD - 1) / kMD : 1;
+  const int64_t total = (te - tb) * nch;
+  if (total <= 0) return;
+
+  // this thread's pieces: row (or query) pr + p * (kMT / PR), values pc ..
+  const int pr = tid / PR, pc = (tid % PR) * PV;
+  // (32-bit offsets from the query tile's first row)
+  const T* qbase = queries + q0 * ld;
+  const int qleft = static_cast<int>(min<int64_t>(kMQ, q - q0)) - 1;
+  Piece vr[NP], vq[NP];
+  double vy = 0.0;
+  int64_t lt = tb;  // load cursor: tile and chunk
+  int lk = 0;
+  auto gload = [&]() {
+    const int64_t t0 = row0 + lt * kMR;
+    const T* rbase = rows + t0 * ld + lk * kMD;
+    const T* cbase = qbase + lk * kMD;
+    const int left = static_cast<int>(min<int64_t>(kMR, n - t0)) - 1;
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      const int r = pr + p * (kMT / PR);
+      vr[p] = *reinterpret_cast<const Piece*>(rbase + min(r, left) * ld + pc);
+      vq[p] = *reinterpret_cast<const Piece*>(cbase + min(r, qleft) * ld + pc);
+    }
+    if (lk == 0 && tid < kMR) vy = y2m[t0 + tid];
+  };
+  auto swrite = [&](int buf) {
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      const int r = pr + p * (kMT / PR);
+#pragma unroll
+      for (int c = 0; c < PV; ++c) {
+        sm.R[buf][r][pc + c] = static_cast<double>(vr[p][c]);
+        sm.Q[buf][r][pc + c] = -2.0 * static_cast<double>(vq[p][c]);
+      }
+    }
+    if (lk == 0 && tid < kMR) sm.y2[(lt - tb) & 1][tid] = vy;
+  };
+  auto advance = [&]() {
+    if (++lk == nch) {
+      lk = 0;
+      ++lt;
+    }
+  };
+  gload();
+  swrite(0);
+  advance();
+  if (total > 1) gload();
+  __syncthreads();
+
+  f64x4 acc[4][4];
+  int kc = 0;
+  int64_t t = tb;
+  for (int64_t c = 0; c < total; ++c) {
+    const int buf = static_cast<int>(c & 1);
+    const int par = static_cast<int>((t - tb) & 1);
+    if (c + 1 < total) {
+      swrite(buf ^ 1);
+      advance();
+      if (c + 2 < total) gload();
+    }
+    if (kc == 0) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        f64x4 y = {0.0, 0.0, 0.0, 0.0};
+        if (!SWAP) {
+#pragma unroll
+          for (int v = 0; v < 4; ++v) y[v] = sm.y2[par][wr * 64 + 16 * i + 4 * v + lg];
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = y;
+      }
+    }
+    // K step s covers dimensions 4s .. 4s + 3 of the chunk; the last chunk
+    // stops at the row's true dimension (the padding is zeros)
+    const int steps = min(4, (d - kc * kMD + 3) / 4);
+#pragma unroll 1
+    for (int s = 0; s < steps; ++s) {
+      double a[4], b[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) a[i] = sm.R[buf][wr * 64 + 16 * i + lr][4 * s + lg];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) b[j] = sm.Q[buf][wq * 64 + 16 * j + lr][4 * s + lg];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          acc[i][j] = SWAP ? __builtin_amdgcn_mfma_f64_16x16x4f64(b[j], a[i], acc[i][j], 0, 0, 0)
+                           : __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
+    }
+    __syncthreads();
+    if (++kc == nch) {
+      epi(t, acc, par);
+      kc = 0;
+      ++t;
+    }
+  }
+}
+
+// y2m of every row of an index (kMR rows of padding past the last, +inf),
+// built once per index; on a capturing stream, where nothing may be kept or
+// waited for, into `local` for the call.
+int ensure_norms64(sc_index* ix, DevBuf& local, const double** y2m, hipStream_t s);
+// The same for a call's queries (no padding).  Queries with a finite but too
+// large norm are appended to list (their x2m is +inf, like that of the
+// non-finite ones).
+template <typename T>
+int query_norms64(const T* queries, int64_t q, int ld, double* x2m, uint32_t* list,
+                  uint32_t* list_n, hipStream_t s);
+
+}  // namespace sc
