@@ -31,9 +31,9 @@
 // hardly a row is tested in vain.
 //
 // Bound by the FP64 matrix rate (72 TFLOP/s in a large matrix product on
-// this card): 4,096 queries x 200,000 x 64 f64 rows take 2.83 ms (12.8 ms
+// this card): 4,096 queries x 200,000 x 64 f64 rows take 2.56 ms (12.8 ms
 // with a tile of vector subtract, multiply, add), 3,001 x 750,000 x 100 f32
-// 8.5 ms (42.1), 54 TFLOP/s.  The prefix is 1,024 rows because its selection
+// 8.2 ms (42.0), 56 TFLOP/s.  The prefix is 1,024 rows because its selection
 // is a walk per query; two levels then leave about 250 candidates per query
 // at k = 10, and one more level would cost two launches to save 100.
 #include <hip/hip_runtime.h>
@@ -134,18 +134,17 @@ __global__ __launch_bounds__(kMT, 2) void dense_kernel(const T* __restrict__ row
   const int tid = threadIdx.x;
   if (tid < kMQ) sx[tid] = x2m[min(q0 + tid, q - 1)];
   mfma64_sweep<T, true>(sm, rows, n, ld, d, y2m, queries, q, q0, 0, tile, tile + 1,
-                        [&](int64_t t, f64x4(&acc)[4][4], int par) {
-    const int lane = tid & 63, wave = tid >> 6;
-    const int wr = wave & 1, wq = wave >> 1, lr = lane & 15, lg = lane >> 4;
+                        [&](int64_t t, MAcc& acc, int par) {
+    const MLane ml;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int rl = wr * 64 + 16 * i + lr;
+    for (int i = 0; i < 8; ++i) {
+      const int rl = 16 * i + ml.lr;
       const double y = sm.y2[par][rl];
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-          const int ql = wq * 64 + 16 * j + 4 * v + lg;
+          const int ql = ml.wave * 32 + 16 * j + 4 * v + ml.lg;
           if (q0 + ql < q) out[(q0 + ql) * cols + t * kMR + rl] = acc[i][j][v] + (sx[ql] + y);
         }
     }
@@ -242,12 +241,7 @@ __global__ __launch_bounds__(kMT, 2) void scan_kernel(
     const T* __restrict__ queries, int64_t q, const double* __restrict__ x2m,
     const double* __restrict__ seed, int k, Bound64 bd, Level lv, ScanOut out) {
   __shared__ MSmem sm;
-  __shared__ double sx[kMQ], sth[kMQ];
-  __shared__ uint32_t mask[kMQ][kMR / 32];
-  __shared__ uint32_t cnt[kMQ], mark[kMQ];
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
-  const int wr = wave & 1, wq = wave >> 1, lr = lane & 15, lg = lane >> 4;
+  const MLane ml;
   const int64_t nqt = (q + kMQ - 1) / kMQ;
   const uint32_t grow = static_cast<uint32_t>(max(2 * k, 32));
   int64_t pos = static_cast<int64_t>(blockIdx.x) * lv.per;
@@ -258,126 +252,73 @@ __global__ __launch_bounds__(kMT, 2) void scan_kernel(
     const int64_t te = min(lv.tiles, tb + (end - pos));
     const int list = static_cast<int>(blockIdx.x - qt * lv.tiles / lv.per);
     const int64_t q0 = qt * kMQ;
-    __syncthreads();  // the previous piece's last reads
-    if (tid < kMQ) {
-      const int64_t qi = q0 + tid;
-      const double x2 = qi < q ? x2m[qi] : INFINITY;
-      sx[tid] = x2;
-      // queries that take no part: nothing is below -inf
-      sth[tid] = x2 < INFINITY ? acc_threshold(bd, seed[qi * k + k - 1], x2) : -INFINITY;
-      cnt[tid] = 0u;
-      mark[tid] = 0u;
+    // the lane's two queries: norm, threshold, entries so far and at the
+    // last look (the same in all four lanes of a column)
+    double x2[2], th[2];
+    uint32_t cnt[2] = {0u, 0u}, mark[2] = {0u, 0u};
 #pragma unroll
-      for (int w = 0; w < kMR / 32; ++w) mask[tid][w] = 0u;
+    for (int j = 0; j < 2; ++j) {
+      const int64_t qi = q0 + ml.query_of(j);
+      x2[j] = qi < q ? x2m[qi] : INFINITY;
+      // queries that take no part: nothing is below -inf
+      th[j] = x2[j] < INFINITY ? acc_threshold(bd, seed[qi * k + k - 1], x2[j]) : -INFINITY;
     }
     auto slot_of = [&](int ql, uint32_t c) {
       return (q0 + ql) * out.entries + lv.entry0 + static_cast<int64_t>(list) * lv.cap + c;
     };
     mfma64_sweep<T, false>(sm, rows, n, ld, d, y2m, queries, q, q0, lv.row0, tb, te,
-                           [&](int64_t t, f64x4(&acc)[4][4], int par) {
-      // acc[i][j][v]: row wr 64 + 16 i + 4 v + lg, query wq 64 + 16 j + lr
-      uint32_t hm[4];
-      bool any = false;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const double th = sth[wq * 64 + 16 * j + lr];
-        hm[j] = 0u;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int v = 0; v < 4; ++v)
-            hm[j] |= static_cast<uint32_t>(!(acc[i][j][v] >= th)) << (4 * i + v);
-        if (!(th > -INFINITY)) hm[j] = 0u;
-        any = any || hm[j] != 0u;
-      }
-      if (any) {
-        // rows left out (padding, non-finite) drop; the others mark their bit
-        any = false;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          uint32_t m = hm[j];
-          while (m) {
-            const int b = __builtin_ctz(m);
-            m &= m - 1;
-            const int rl = wr * 64 + 16 * (b >> 2) + 4 * (b & 3) + lg;
-            if (sm.y2[par][rl] == INFINITY)
-              hm[j] &= ~(1u << b);
-            else
-              atomicOr(&mask[wq * 64 + 16 * j + lr][rl >> 5], 1u << (rl & 31));
-          }
-          any = any || hm[j] != 0u;
-        }
-      }
-      if (!__syncthreads_or(any)) return;
+                           [&](int64_t t, MAcc& acc, int par) {
       const int64_t r0 = lv.row0 + t * kMR;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if (hm[j] == 0u) continue;
-        const int ql = wq * 64 + 16 * j + lr;
-        const uint32_t base = cnt[ql];
-        const double x2 = sx[ql];
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            if (!((hm[j] >> (4 * i + v)) & 1u)) continue;
-            const int rl = wr * 64 + 16 * i + 4 * v + lg;
-            // the place in row order: the marked rows before this one
-            uint32_t c = base + __popc(mask[ql][rl >> 5] & ((1u << (rl & 31)) - 1u));
-            for (int w = 0; w < (rl >> 5); ++w) c += __popc(mask[ql][w]);
-            if (c < static_cast<uint32_t>(lv.cap)) {
-              const int64_t s = slot_of(ql, c);
-              out.idx[s] = static_cast<uint32_t>(r0 + rl);
-              out.u[s] = sum_upper(bd, acc[i][j][v] + x2, x2 + sm.y2[par][rl]);
-            }
-          }
-      }
-      __syncthreads();
-      bool grown = false;
-      if (tid < kMQ) {
-        uint32_t c = 0;
-#pragma unroll
-        for (int w = 0; w < kMR / 32; ++w) {
-          c += __popc(mask[tid][w]);
-          mask[tid][w] = 0u;
+      tile_hits(ml, acc, th, sm.y2[par], [&](int i, int j, int v, int rl, bool hit, uint64_t m) {
+        m &= ml.column();
+        const uint32_t c = cnt[j] + __popcll(m & ml.below());
+        if (hit && c < static_cast<uint32_t>(lv.cap)) {
+          const int64_t s = slot_of(ml.query_of(j), c);
+          out.idx[s] = static_cast<uint32_t>(r0 + rl);
+          out.u[s] = sum_upper(bd, acc[i][j][v] + x2[j], x2[j] + sm.y2[par][rl]);
         }
-        if (c) {
-          c += cnt[tid];
-          cnt[tid] = c;
-          grown = c - mark[tid] >= grow;
-        }
-      }
-      if (!__syncthreads_or(grown)) return;
+        cnt[j] += __popcll(m);
+      });
       // lists that grew by `grow` since they were last looked at: their own
       // k-th U is a threshold too
-      for (int ql = wave; ql < kMQ; ql += kMT / 64) {
-        const uint32_t c = cnt[ql];
-        if (c - mark[ql] < grow) continue;  // the same for the whole wave
-        const uint32_t m = min(c, static_cast<uint32_t>(lv.cap));
-        KSmallest ks;
-        ks.clear();
-        const double* u = out.u + slot_of(ql, 0);
-        for (uint32_t c0 = 0; c0 < m; c0 += 64) {
-          const double x = c0 + lane < m ? u[c0 + lane] : INFINITY;
-          uint64_t b = __ballot(x < ks.kth);
-          while (b) {
-            const int src = __builtin_ctzll(b);
-            ks.insert(lane_value(x, src), lane, k);
-            b &= b - 1;
-            b &= __ballot(x < ks.kth);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        uint64_t g = __ballot(cnt[j] - mark[j] >= grow) & 0xffffu;
+        while (g) {
+          const int src = __builtin_ctzll(g);  // the column
+          g &= g - 1;
+          const uint32_t c = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(cnt[j]), src));
+          const uint32_t m = min(c, static_cast<uint32_t>(lv.cap));
+          const double* u = out.u + slot_of(ml.wave * 32 + 16 * j + src, 0);
+          // entries that other lanes of this wavefront stored
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+          KSmallest ks;
+          ks.clear();
+          for (uint32_t c0 = 0; c0 < m; c0 += 64) {
+            const double x = c0 + ml.lane < m ? u[c0 + ml.lane] : INFINITY;
+            uint64_t b = __ballot(x < ks.kth);
+            while (b) {
+              const int s2 = __builtin_ctzll(b);
+              ks.insert(lane_value(x, s2), ml.lane, k);
+              b &= b - 1;
+              b &= __ballot(x < ks.kth);
+            }
+          }
+          if (ml.lr == src) {
+            const double lower = acc_threshold(bd, ks.kth, x2[j]);
+            if (lower < th[j]) th[j] = lower;
+            mark[j] = c;
           }
         }
-        if (lane == 0) {
-          const double th = acc_threshold(bd, ks.kth, sx[ql]);
-          if (th < sth[ql]) sth[ql] = th;
-          mark[ql] = c;
-        }
       }
-      __syncthreads();
     });
-    __syncthreads();
-    if (tid < kMQ && q0 + tid < q) out.count[(q0 + tid) * out.lists + lv.list0 + list] = cnt[tid];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int64_t qi = q0 + ml.query_of(j);
+      if (ml.lg == 0 && qi < q) out.count[qi * out.lists + lv.list0 + list] = cnt[j];
+    }
     pos += te - tb;
+    __syncthreads();  // the sweep's LDS is staged anew
   }
 }
 
@@ -439,8 +380,6 @@ __global__ __launch_bounds__(kFinishThreads) void finish_kernel(
     int64_t* __restrict__ out_idx, double* __restrict__ out_dist, uint32_t* __restrict__ out_count,
     uint32_t* __restrict__ list, uint32_t* __restrict__ list_n,
     unsigned long long* __restrict__ total_cand) {
-  constexpr int PV = 16 / sizeof(T);
-  typedef T Piece __attribute__((ext_vector_type(PV)));
   extern __shared__ __align__(16) uint32_t start[];  // nl + 1
   __shared__ double s_S[kFinishBatch];
   __shared__ uint32_t s_row[kFinishBatch];
@@ -510,21 +449,7 @@ __global__ __launch_bounds__(kFinishThreads) void finish_kernel(
         row = ls.out.idx[qi * ls.out.entries + ls.lv[v].entry0 +
                          (lo - 1 - ls.lv[v].list0) * ls.lv[v].cap + at];
       }
-      const Piece* r = reinterpret_cast<const Piece*>(rows + static_cast<int64_t>(row) * ld);
-      const Piece* x = reinterpret_cast<const Piece*>(qrow);
-      double s = 0.0;
-      for (int j = 0; j < ld / PV; j += 16 / PV) {
-        Piece rv[16 / PV], xv[16 / PV];
-#pragma unroll
-        for (int c = 0; c < 16 / PV; ++c) {
-          rv[c] = r[j + c];
-          xv[c] = x[j + c];
-        }
-#pragma unroll
-        for (int c = 0; c < 16 / PV; ++c)
-#pragma unroll
-          for (int w = 0; w < PV; ++w) s = s + Term<T, kEuclid>::f(xv[c][w], rv[c][w], 2.0);
-      }
+      const double s = exact_sum(qrow, rows + static_cast<int64_t>(row) * ld, ld);
       s_S[e] = s;
       s_row[e] = row;
     }

@@ -1,16 +1,21 @@
 // FP64 MFMA tile sweep shared by the Euclidian searches.
 //
 // A 256-thread workgroup sweeps 128-row tiles of the index against 128
-// queries.  Wave (wr, wq) of the 2 x 2 arrangement owns 64 rows x 64 queries
-// as 4 x 4 v_mfma_f64_16x16x4_f64 accumulators (128 VGPRs), so a K step of
-// four dimensions costs 8 LDS reads for 16 MFMAs and the kernel is bound by
-// the matrix pipe (64 cycles per MFMA and SIMD): the vector form needs
-// three FP64 instructions per element (subtract, multiply, add) where the
-// MFMA needs one fused multiply-add.  Dimension chunks of 16 go through two
-// LDS buffers: chunk c + 1 is stored and chunk c + 2 requested while chunk
-// c's MFMAs run, with one barrier per chunk; the chunk stream runs on across
-// tiles, so a tile's first chunk is as early as any other.  f32 rows are
-// widened (exactly) when they are stored to LDS.
+// queries.  Wave w owns queries 32 w .. 32 w + 31 against all 128 rows, as
+// 8 x 2 v_mfma_f64_16x16x4_f64 accumulators (128 VGPRs): a K step of four
+// dimensions costs 10 LDS reads for 16 MFMAs, and because a query's rows
+// never leave its wavefront, results are filtered and appended in row order
+// without a barrier (a 2 x 2 arrangement of 64 x 64 needs 8 reads, but two
+// barriers per tile to order a query's rows across two wavefronts: 4,096
+// queries x 200,000 x 64 took 2.91 ms with it and 2.56 ms without, 5,000 x
+// 100,000 x 16 within a radius 0.91 and 0.84).  The kernel is bound by the matrix pipe (64 cycles per
+// MFMA and SIMD): the vector form needs three FP64 instructions per element
+// (subtract, multiply, add) where the MFMA needs one fused multiply-add.
+// Dimension chunks of 16 go through two LDS buffers: chunk c + 1 is stored
+// and chunk c + 2 requested while chunk c's MFMAs run, with one barrier per
+// chunk; the chunk stream runs on across tiles, so a tile's first chunk is
+// as early as any other.  Queries of one chunk are staged once.  f32 rows
+// are widened (exactly) when they are stored to LDS.
 //
 // The accumulators start at y2m, a lower bound of the row's ||y||^2, and the
 // queries are staged as -2x, so a tile ends with acc = y2m - 2 x.y.
@@ -34,6 +39,7 @@
 #include <hip/hip_runtime.h>
 
 #include "common.hpp"
+#include "metric.hpp"
 
 namespace sc {
 
@@ -87,17 +93,64 @@ __device__ __forceinline__ double sum_upper(const Bound64& b, double L, double n
   return u < b.limit ? u : INFINITY;  // NaN too
 }
 
+// The reference's sum of one (query, row) pair: terms in dimension order,
+// 16 values of both requested before they are folded (rows are padded to
+// multiples of 16 values).
+template <typename T>
+__device__ __forceinline__ double exact_sum(const T* __restrict__ x, const T* __restrict__ y, int ld) {
+  constexpr int PV = 16 / sizeof(T);
+  typedef T Piece __attribute__((ext_vector_type(PV)));
+  const Piece* xp = reinterpret_cast<const Piece*>(x);
+  const Piece* yp = reinterpret_cast<const Piece*>(y);
+  double s = 0.0;
+  for (int j = 0; j < ld / PV; j += 16 / PV) {
+    Piece xv[16 / PV], yv[16 / PV];
+#pragma unroll
+    for (int c = 0; c < 16 / PV; ++c) {
+      xv[c] = xp[j + c];
+      yv[c] = yp[j + c];
+    }
+#pragma unroll
+    for (int c = 0; c < 16 / PV; ++c)
+#pragma unroll
+      for (int w = 0; w < PV; ++w) s = s + Term<T, kEuclid>::f(xv[c][w], yv[c][w], 2.0);
+  }
+  return s;
+}
+
 struct MSmem {
   double R[2][kMR][kMStride];
   double Q[2][kMQ][kMStride];
-  double y2[2][kMR];  // y2m of the tile, by tile parity
+  // y2m by tile modulo 4: a wavefront may still read a tile's while the
+  // others, at most one barrier ahead, store the next but one's
+  double y2[4][kMR];
 };
 
+// Where a lane's accumulators lie: acc[i][j][v] is row row_of(i, v), query
+// query_of(j) of the tile.  The four lanes of a query's column hold four
+// consecutive rows.
+struct MLane {
+  int lane, wave, lr, lg;
+  __device__ __forceinline__ MLane() {
+    lane = threadIdx.x & 63;
+    wave = threadIdx.x >> 6;
+    lr = lane & 15;
+    lg = lane >> 4;
+  }
+  __device__ __forceinline__ int row_of(int i, int v) const { return 16 * i + 4 * v + lg; }
+  __device__ __forceinline__ int query_of(int j) const { return wave * 32 + 16 * j + lr; }
+  // the lanes of this lane's column
+  __device__ __forceinline__ uint64_t column() const { return uint64_t(0x0001000100010001) << lr; }
+  __device__ __forceinline__ uint64_t below() const { return (uint64_t(1) << lane) - 1; }
+};
+typedef f64x4 MAcc[8][2];
+
 // Sweeps tiles tb .. te - 1 (row = row0 + 128 tile) against queries
-// q0 .. q0 + 127; epi(t, acc, parity) runs on all threads at each tile's
-// end (it may synchronise).  Out-of-range rows and queries are read clamped:
-// y2m carries +inf past the last row.  SWAP: the accumulators hold
-// (query, row) transposed -- lane column = row -- and start at zero.
+// q0 .. q0 + 127; epi(t, acc, slot) runs at each tile's end, without a
+// barrier of its own (sm.y2[slot] holds the tile's y2m).  Out-of-range rows and
+// queries are read clamped: y2m carries +inf past the last row.  SWAP: the
+// accumulators hold (query, row) transposed -- acc[i][j][v] of a lane is row
+// 16 i + lr, query 32 wave + 16 j + 4 v + lg -- and start at zero.
 template <typename T, bool SWAP, typename Epi>
 __device__ __forceinline__ void mfma64_sweep(MSmem& sm, const T* __restrict__ rows, int64_t n,
                                              int ld, int d, const double* __restrict__ y2m,
@@ -108,10 +161,7 @@ __device__ __forceinline__ void mfma64_sweep(MSmem& sm, const T* __restrict__ ro
   constexpr int NP = kMR * PR / kMT;            // pieces per thread (rows and queries each)
   typedef T Piece __attribute__((ext_vector_type(PV)));
   const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int wr = wave & 1, wq = wave >> 1;
-  const int lr = lane & 15, lg = lane >> 4;
+  const MLane ml;
   const int nch = d > kMD ? (d + kMD - 1) / kMD : 1;
   const int64_t total = (te - tb) * nch;
   if (total <= 0) return;
@@ -125,30 +175,37 @@ __device__ __forceinline__ void mfma64_sweep(MSmem& sm, const T* __restrict__ ro
   double vy = 0.0;
   int64_t lt = tb;  // load cursor: tile and chunk
   int lk = 0;
+  auto gload_q = [&]() {
+    const T* cbase = qbase + lk * kMD;
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+      vq[p] = *reinterpret_cast<const Piece*>(cbase + min(pr + p * (kMT / PR), qleft) * ld + pc);
+  };
   auto gload = [&]() {
     const int64_t t0 = row0 + lt * kMR;
     const T* rbase = rows + t0 * ld + lk * kMD;
-    const T* cbase = qbase + lk * kMD;
     const int left = static_cast<int>(min<int64_t>(kMR, n - t0)) - 1;
 #pragma unroll
-    for (int p = 0; p < NP; ++p) {
-      const int r = pr + p * (kMT / PR);
-      vr[p] = *reinterpret_cast<const Piece*>(rbase + min(r, left) * ld + pc);
-      vq[p] = *reinterpret_cast<const Piece*>(cbase + min(r, qleft) * ld + pc);
-    }
+    for (int p = 0; p < NP; ++p)
+      vr[p] = *reinterpret_cast<const Piece*>(rbase + min(pr + p * (kMT / PR), left) * ld + pc);
+    if (nch > 1) gload_q();
     if (lk == 0 && tid < kMR) vy = y2m[t0 + tid];
+  };
+  auto swrite_q = [&](int buf) {
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+#pragma unroll
+      for (int c = 0; c < PV; ++c)
+        sm.Q[buf][pr + p * (kMT / PR)][pc + c] = -2.0 * static_cast<double>(vq[p][c]);
   };
   auto swrite = [&](int buf) {
 #pragma unroll
-    for (int p = 0; p < NP; ++p) {
-      const int r = pr + p * (kMT / PR);
+    for (int p = 0; p < NP; ++p)
 #pragma unroll
-      for (int c = 0; c < PV; ++c) {
-        sm.R[buf][r][pc + c] = static_cast<double>(vr[p][c]);
-        sm.Q[buf][r][pc + c] = -2.0 * static_cast<double>(vq[p][c]);
-      }
-    }
-    if (lk == 0 && tid < kMR) sm.y2[(lt - tb) & 1][tid] = vy;
+      for (int c = 0; c < PV; ++c)
+        sm.R[buf][pr + p * (kMT / PR)][pc + c] = static_cast<double>(vr[p][c]);
+    if (nch > 1) swrite_q(buf);
+    if (lk == 0 && tid < kMR) sm.y2[(lt - tb) & 3][tid] = vy;
   };
   auto advance = [&]() {
     if (++lk == nch) {
@@ -156,18 +213,23 @@ __device__ __forceinline__ void mfma64_sweep(MSmem& sm, const T* __restrict__ ro
       ++lt;
     }
   };
+  if (nch == 1) {  // the queries' only chunk: staged for the whole sweep
+    gload_q();
+    swrite_q(0);
+  }
   gload();
   swrite(0);
   advance();
   if (total > 1) gload();
   __syncthreads();
 
-  f64x4 acc[4][4];
+  MAcc acc;
   int kc = 0;
   int64_t t = tb;
   for (int64_t c = 0; c < total; ++c) {
     const int buf = static_cast<int>(c & 1);
-    const int par = static_cast<int>((t - tb) & 1);
+    const int qbuf = nch > 1 ? buf : 0;
+    const int par = static_cast<int>((t - tb) & 3);
     if (c + 1 < total) {
       swrite(buf ^ 1);
       advance();
@@ -175,14 +237,14 @@ __device__ __forceinline__ void mfma64_sweep(MSmem& sm, const T* __restrict__ ro
     }
     if (kc == 0) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
+      for (int i = 0; i < 8; ++i) {
         f64x4 y = {0.0, 0.0, 0.0, 0.0};
         if (!SWAP) {
 #pragma unroll
-          for (int v = 0; v < 4; ++v) y[v] = sm.y2[par][wr * 64 + 16 * i + 4 * v + lg];
+          for (int v = 0; v < 4; ++v) y[v] = sm.y2[par][ml.row_of(i, v)];
         }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = y;
+        acc[i][0] = y;
+        acc[i][1] = y;
       }
     }
     // K step s covers dimensions 4s .. 4s + 3 of the chunk; the last chunk
@@ -190,15 +252,15 @@ __device__ __forceinline__ void mfma64_sweep(MSmem& sm, const T* __restrict__ ro
     const int steps = min(4, (d - kc * kMD + 3) / 4);
 #pragma unroll 1
     for (int s = 0; s < steps; ++s) {
-      double a[4], b[4];
+      double a[8], b[2];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = sm.R[buf][wr * 64 + 16 * i + lr][4 * s + lg];
+      for (int j = 0; j < 2; ++j) b[j] = sm.Q[qbuf][ml.wave * 32 + 16 * j + ml.lr][4 * s + ml.lg];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) b[j] = sm.Q[buf][wq * 64 + 16 * j + lr][4 * s + lg];
+      for (int i = 0; i < 8; ++i) a[i] = sm.R[buf][16 * i + ml.lr][4 * s + ml.lg];
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < 8; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < 2; ++j)
           acc[i][j] = SWAP ? __builtin_amdgcn_mfma_f64_16x16x4f64(b[j], a[i], acc[i][j], 0, 0, 0)
                            : __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
     }
@@ -208,6 +270,41 @@ __device__ __forceinline__ void mfma64_sweep(MSmem& sm, const T* __restrict__ ro
       kc = 0;
       ++t;
     }
+  }
+}
+
+// Calls f(i, j, v, row, hit, mask) for every accumulator register of the
+// wavefront that holds values below their query's threshold th[j] (-inf: a
+// query that takes no part), rows ascending for each query; hit: this lane
+// is one of the lanes in mask.  Rows that y2 leaves out are dropped.  The
+// first test of a query block is one compare per register, or-ed in scalar
+// registers.
+template <typename F>
+__device__ __forceinline__ void tile_hits(const MLane& ml, const MAcc& acc, const double (&th)[2],
+                                          const double* y2, F f) {
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    uint64_t some = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) some |= __ballot(!(acc[i][j][v] >= th[j]));
+    if (some == 0) continue;  // the whole wavefront
+    // compared anew: 32 kept compare masks would not fit the scalar registers
+    double t = th[j];
+    asm volatile("" : "+v"(t));
+    const bool part = !(t == -INFINITY);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        bool hit = !(acc[i][j][v] >= t);
+        if (__ballot(hit) == 0) continue;
+        const int rl = ml.row_of(i, v);
+        hit = hit && part && y2[rl] != INFINITY;
+        const uint64_t m = __ballot(hit);
+        if (m) f(i, j, v, rl, hit, m);
+      }
   }
 }
 
