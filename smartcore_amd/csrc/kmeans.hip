@@ -7,11 +7,11 @@
 //             the reference's element order; argmin with strict < so the
 //             lowest index wins ties (kmeans.rs:343-346).  64 rows x 64
 //             centroids per tile, 4x4 register micro-tiles.
-//   partial   One workgroup per block of kBlockRows rows.  Rows are staged
-//             through LDS 128 at a time; wave w owns the clusters c with
-//             c % 4 == w and adds each owned row into an f64 LDS accumulator
-//             (lane = dimension, ds_add_f64), in row order.  One owner per
-//             cluster makes the sums deterministic.
+//   partial   One workgroup per block of kBlockRows rows adds each cluster's
+//             rows in row order: the MFMA form's kernel (kmeans_mixed.hip:
+//             labels sorted in LDS) for k and ld up to 128, else LDS
+//             accumulators or ballots over the labels.  One owner wave per cluster makes the sums
+//             deterministic.
 //   reduce    Two kernels shared by every form and by the batched form.
 //             group: block sums added in groups of 16 blocks, in block
 //             order.  final: one workgroup per cluster adds the groups in
@@ -142,6 +142,62 @@ __global__ __launch_bounds__(NT) void kmeans_assign_kernel(const T* __restrict__
   }
 }
 
+// Rows of up to 64 values: one thread per row, its values in registers, the
+// centroids read through the scalar cache (their address is the same in all
+// lanes), four of them at a time so that four folds are in flight.  Three
+// FP64 instructions per row, centroid and dimension is what the reference's
+// arithmetic costs, and nothing else is issued; the tile above also moves
+// every operand through LDS and computes its 64 centroids whatever k is
+// (100,000 x 16, k = 10: 18.4 us with the tile, 6.8 here).
+template <typename T, int L>
+__global__ __launch_bounds__(NT) void kmeans_assign_rows_kernel(const T* __restrict__ rows,
+                                                                int64_t n, int d,
+                                                                const double* __restrict__ cent,
+                                                                int k, uint32_t* __restrict__ labels,
+                                                                const KmState* __restrict__ st) {
+  if (st && st->done) return;
+  constexpr int LD = 16 * L;
+  constexpr int PV = 16 / sizeof(T);
+  typedef T Piece __attribute__((ext_vector_type(PV)));
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * NT + threadIdx.x;
+  if (i >= n) return;
+  double x[LD];
+  const Piece* r = reinterpret_cast<const Piece*>(rows + i * LD);
+#pragma unroll
+  for (int p = 0; p < LD / PV; ++p) {
+    const Piece v = r[p];
+#pragma unroll
+    for (int w = 0; w < PV; ++w) x[PV * p + w] = static_cast<double>(v[w]);
+  }
+  double bv = INFINITY;
+  uint32_t bi = 0xffffffffu;
+  for (int c0 = 0; c0 < k; c0 += 4) {
+    const double* cp[4];
+    double s[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int u = 0; u < 4; ++u) cp[u] = cent + static_cast<int64_t>(min(c0 + u, k - 1)) * LD;
+#pragma unroll
+    for (int j0 = 0; j0 < LD; j0 += 4) {
+      if (j0 < d) {  // the padding would add exact zeros
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+          for (int j = j0; j < j0 + 4; ++j) s[u] = s[u] + Term<double, kEuclid>::f(x[j], cp[u][j], 2.0);
+      }
+    }
+    // strict <, lowest index first (kmeans.rs:343-346); a repeated last
+    // centroid is not below itself
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (s[u] < bv) {
+        bv = s[u];
+        bi = static_cast<uint32_t>(min(c0 + u, k - 1));
+      }
+  }
+  // kmeans.rs:334-347: min starts at f64::MAX; nothing below it keeps 0
+  labels[i] = bv < DBL_MAX ? bi : 0u;
+}
+
 // The shift mu of the distortion sums: the first row, widened to f64, with
 // non-finite values replaced by 0.
 template <typename T>
@@ -181,7 +237,9 @@ __global__ void x2_total_kernel(const double* __restrict__ x2block, int64_t nb, 
   st->x2total = s;
 }
 
-// Partial sums with one owner wave per cluster (see the file comment).
+// Partial sums for more clusters than the sorted kernel takes, as long as
+// their accumulators fit LDS: rows are staged 128 at a time; wave w owns the
+// clusters c with c % 4 == w and adds each owned row in row order.
 // Dynamic LDS: acc[k*d] f64 | stage[kChunkRows*ld] T | lab[kChunkRows] | cnt[k].
 template <typename T>
 __global__ __launch_bounds__(NT) void kmeans_partial_lds_kernel(
@@ -234,8 +292,8 @@ __global__ __launch_bounds__(NT) void kmeans_partial_lds_kernel(
   for (int e = tid; e < k; e += NT) pcount[b * k + e] = cnt[e];
 }
 
-// Fallback when the accumulators do not fit LDS: one wave per cluster,
-// ballots over the labels, rows added in row order.
+// Partial sums of the remaining shapes: one wave per
+// cluster, ballots over the labels, rows added in row order.
 template <typename T>
 __global__ __launch_bounds__(NT) void kmeans_partial_ballot_kernel(
     const T* __restrict__ rows, int64_t n, int ld, int d, const uint32_t* __restrict__ labels,
@@ -624,23 +682,163 @@ __global__ void kmeans_state_init_kernel(KmState* st) {
   st->fallback = 0;
 }
 
-// One k-means++ round (kmeans.rs:367-379 and the final pass :399-410):
-// d_i = min(d_i, squared_distance(row_i, centroid)) in the rows' own type
-// (the reference calls Euclidian::squared_distance on TX rows here), and the
-// label of a row that improves becomes `label`.
+// ---- k-means++ on the device (kmeans.rs:354-413) ----
+//
+// Each round updates every row's squared distance to its nearest centre so
+// far (the reference calls Euclidian::squared_distance on TX rows here, so
+// the terms are the rows' own type) and the label of the rows that improve;
+// then the next centre is the first row whose running sum of distances, added
+// in row order, reaches cutoff = u * sum.  The reference's sums are
+// sequential folds, a chain of n dependent adds; any order of adding is
+// within n 2^-53 of them in relative terms, so a parallel prefix sum decides
+// the row unless it ends within delta = 4 (n + 64) 2^-53 sum of the cutoff
+// on either side of that row (about one round in 10^4 at a million rows):
+// then, and when a sum is not finite, the round is left to the host, which
+// folds in row order.  The draws u do not depend on the data, so all rounds
+// are queued without a host round trip.  (100,000 x 16, k = 10: 0.25 ms, and
+// 1,000,000 x 64, k = 64: 4.0; downloading and folding every round took 1.24
+// and 119.)
+constexpr int kPPRows = 1024;  // rows per partial sum
+
+struct PPState {
+  uint32_t round;  // the round the host has to decide, or 0
+};
+
 template <typename T>
-__global__ void kmeanspp_round_kernel(const T* __restrict__ rows, int64_t n, int ld,
-                                      const T* __restrict__ centroid, double* __restrict__ dmin,
-                                      uint32_t* __restrict__ y, uint32_t label) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const T* r = rows + i * ld;
-  double s = 0.0;
-  for (int j = 0; j < ld; ++j) s = s + Term<T, kEuclid>::f(r[j], centroid[j], 2.0);
-  if (s < dmin[i]) {
-    dmin[i] = s;
-    y[i] = label;
+__global__ __launch_bounds__(kPPRows) void kmeanspp_round_kernel(
+    const T* __restrict__ rows, int64_t n, int ld, const int64_t* __restrict__ pick,
+    double* __restrict__ dmin, uint32_t* __restrict__ y, uint32_t label, double* __restrict__ part,
+    const PPState* __restrict__ st) {
+  if (st->round) return;
+  constexpr int PV = 16 / sizeof(T);
+  typedef T Piece __attribute__((ext_vector_type(PV)));
+  __shared__ double s_wave[kPPRows / 64];
+  const Piece* cen = reinterpret_cast<const Piece*>(rows + pick[label] * ld);
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * kPPRows + threadIdx.x;
+  double best = 0.0;
+  if (i < n) {
+    const Piece* r = reinterpret_cast<const Piece*>(rows + i * ld);
+    double s = 0.0;
+    for (int p = 0; p < ld / PV; p += 16 / PV) {  // ld is a multiple of 16
+      Piece a[16 / PV], b[16 / PV];
+#pragma unroll
+      for (int c = 0; c < 16 / PV; ++c) {
+        a[c] = r[p + c];
+        b[c] = cen[p + c];
+      }
+#pragma unroll
+      for (int c = 0; c < 16 / PV; ++c)
+#pragma unroll
+        for (int w = 0; w < PV; ++w) s = s + Term<T, kEuclid>::f(a[c][w], b[c][w], 2.0);
+    }
+    best = label ? dmin[i] : DBL_MAX;
+    if (s < best) {
+      best = s;
+      y[i] = label;
+    }
+    dmin[i] = best;
   }
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) best += __shfl_xor(best, o);
+  if ((threadIdx.x & 63) == 0) s_wave[threadIdx.x >> 6] = best;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double sum = 0.0;
+    for (int w = 0; w < kPPRows / 64; ++w) sum += s_wave[w];
+    part[blockIdx.x] = sum;
+  }
+}
+
+// The row of pick[round] (see above); one workgroup.
+__global__ __launch_bounds__(kPPRows) void kmeanspp_pick_kernel(const double* __restrict__ dmin,
+                                                                int64_t n,
+                                                                const double* __restrict__ part,
+                                                                int64_t nb,
+                                                                const double* __restrict__ draws,
+                                                                uint32_t round,
+                                                                int64_t* __restrict__ pick,
+                                                                PPState* __restrict__ st) {
+  if (st->round) return;
+  __shared__ double s_wave[kPPRows / 64];
+  __shared__ double s_total, s_before, s_cut, s_delta;
+  __shared__ int64_t s_block;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // inclusive prefix over the workgroup's values
+  auto scan = [&](double v) {
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const double up = __shfl_up(v, o);
+      if (lane >= o) v += up;
+    }
+    __syncthreads();  // earlier readers of s_wave
+    if (lane == 63) s_wave[wave] = v;
+    __syncthreads();
+    double base = 0.0;
+    for (int w = 0; w < wave; ++w) base += s_wave[w];
+    return v + base;
+  };
+  double total = 0.0;
+  for (int64_t b0 = 0; b0 < nb; b0 += kPPRows) {
+    const double p = scan(b0 + tid < nb ? part[b0 + tid] : 0.0);
+    if (tid == kPPRows - 1) s_total = total + p;
+    __syncthreads();
+    total = s_total;
+    __syncthreads();
+  }
+  if (tid == 0) {
+    s_cut = draws[round] * total;
+    s_delta = 4.0 * (static_cast<double>(n) + 64.0) * 1.1102230246251565e-16 * total;
+    s_block = -1;
+  }
+  __syncthreads();
+  const double cut = s_cut, delta = s_delta;
+  // the block in which the running sum reaches the cutoff
+  double before = 0.0;
+  for (int64_t b0 = 0; b0 < nb && s_block < 0; b0 += kPPRows) {
+    const double own = b0 + tid < nb ? part[b0 + tid] : 0.0;
+    const double p = before + scan(own);
+    const bool here = b0 + tid < nb && p >= cut;
+    const uint64_t m = __ballot(here);
+    __shared__ int s_first[kPPRows / 64];
+    if (lane == 0) s_first[wave] = m ? __builtin_ctzll(m) : 64;
+    if (tid == kPPRows - 1) s_total = p;
+    __syncthreads();
+    int first = -1;
+    for (int w = 0; w < kPPRows / 64 && first < 0; ++w)
+      if (s_first[w] < 64) first = 64 * w + s_first[w];
+    if (first == tid) {
+      s_block = b0 + tid;
+      s_before = p - own;  // (rounding: inside delta)
+    }
+    before = s_total;
+    __syncthreads();
+  }
+  const int64_t block = s_block;
+  bool sure = block >= 0 && total < INFINITY;
+  if (sure) {
+    const int64_t i = block * kPPRows + tid;
+    const double own = i < n ? dmin[i] : 0.0;
+    const double p = s_before + scan(own);
+    const bool here = i < n && p >= cut;
+    const uint64_t m = __ballot(here);
+    __shared__ int s_at[kPPRows / 64];
+    if (lane == 0) s_at[wave] = m ? __builtin_ctzll(m) : 64;
+    __syncthreads();
+    int first = -1;
+    for (int w = 0; w < kPPRows / 64 && first < 0; ++w)
+      if (s_at[w] < 64) first = 64 * w + s_at[w];
+    sure = first >= 0;
+    if (first == tid) {
+      // row i's sum reaches the cutoff and the sum before it does not, by
+      // more than any order of adding can move them
+      const bool certain = p >= cut + delta && (i == 0 || p - own < cut - delta);
+      if (certain)
+        pick[round] = i;
+      else
+        st->round = round;
+    }
+  }
+  if (!sure && tid == 0) st->round = round;
 }
 
 __global__ void fill_kernel(double* p, int64_t n, double v) {
@@ -661,6 +859,31 @@ int kmeans_assign_launch(const sc_index* ix, const void* rows, int64_t n, const 
   const unsigned grid = static_cast<unsigned>((n + PT - 1) / PT);
   if (grid == 0) return SC_OK;
   ProfScope ps("kmeans_assign", s);
+  const int d = static_cast<int>(ix->d);
+  const dim3 rgrid(static_cast<unsigned>((n + NT - 1) / NT));
+#define SC_ASSIGN_ROWS(L)                                                                         \
+  if (ix->ld == 16 * L) {                                                                         \
+    if (ix->dtype == SC_F64)                                                                      \
+      hipLaunchKernelGGL((kmeans_assign_rows_kernel<double, L>), rgrid, dim3(NT), 0, s,           \
+                         static_cast<const double*>(rows), n, d, d_cent, k, d_labels, st);        \
+    else                                                                                          \
+      hipLaunchKernelGGL((kmeans_assign_rows_kernel<float, L>), rgrid, dim3(NT), 0, s,            \
+                         static_cast<const float*>(rows), n, d, d_cent, k, d_labels, st);         \
+    SC_HIP(hipGetLastError());                                                                    \
+    return SC_OK;                                                                                 \
+  }
+  // One thread per row where it is the faster form: rows of up to 48 values
+  // (200,000 x 40, k = 32: 48 against 89 us), or 64 with few centroids for
+  // the tile's 64 (1,000,000 x 64, k = 64: 605 against 462 us; its cost goes
+  // with k, the tile's with ceil(k / 64)), and enough rows for the chip
+  // (20,000 x 6, k = 130: 35 against 26 us).
+  if (n >= 65536 || k <= 32) {
+    SC_ASSIGN_ROWS(1) SC_ASSIGN_ROWS(2) SC_ASSIGN_ROWS(3)
+    if (k <= 32) {
+      SC_ASSIGN_ROWS(4)
+    }
+  }
+#undef SC_ASSIGN_ROWS
   if (ix->dtype == SC_F64)
     hipLaunchKernelGGL(kmeans_assign_kernel<double>, dim3(grid), dim3(NT), 0, s,
                        static_cast<const double*>(rows), n, static_cast<int>(ix->ld), d_cent, k,
@@ -708,8 +931,13 @@ int kmeans_partial_launch(const sc_index* ix, KmWork& w, int k, const KmState* s
   const int ld = static_cast<int>(ix->ld);
   if (w.p.nb == 0) return SC_OK;
   ProfScope ps("kmeans_partial", s);
-  const size_t lds = partial_lds_bytes(ix, k);
+  // Sorting the labels first turns each cluster's rows into one run that is
+  // read 16 or 32 rows at a time; walking them through LDS atomics took 147
+  // us for 100,000 x 16 f64 rows and 10 clusters, the sorted runs take 17
+  // (1,000,000 x 64 f32, 64 clusters: 306 and 55).
+  if (kmeans_sorted_sums_supported(k, ld)) return kmeans_sorted_sums_launch(ix, w, s);
   const dim3 grid(static_cast<unsigned>(w.p.nb));
+  const size_t lds = partial_lds_bytes(ix, k);
   if (static_cast<int64_t>(k) * d <= kMaxLdsAcc && lds <= 96 * 1024) {
     if (ix->dtype == SC_F64)
       hipLaunchKernelGGL(kmeans_partial_lds_kernel<double>, grid, dim3(NT), lds, s,
@@ -719,16 +947,17 @@ int kmeans_partial_launch(const sc_index* ix, KmWork& w, int k, const KmState* s
       hipLaunchKernelGGL(kmeans_partial_lds_kernel<float>, grid, dim3(NT), lds, s,
                          static_cast<const float*>(ix->rows), n, ld, d, w.p.labels, k, w.p.psum,
                          w.p.pcount, st);
-  } else {
-    if (ix->dtype == SC_F64)
-      hipLaunchKernelGGL(kmeans_partial_ballot_kernel<double>, grid, dim3(NT), 0, s,
-                         static_cast<const double*>(ix->rows), n, ld, d, w.p.labels, k, w.p.psum,
-                         w.p.pcount, st);
-    else
-      hipLaunchKernelGGL(kmeans_partial_ballot_kernel<float>, grid, dim3(NT), 0, s,
-                         static_cast<const float*>(ix->rows), n, ld, d, w.p.labels, k, w.p.psum,
-                         w.p.pcount, st);
+    SC_HIP(hipGetLastError());
+    return SC_OK;
   }
+  if (ix->dtype == SC_F64)
+    hipLaunchKernelGGL(kmeans_partial_ballot_kernel<double>, grid, dim3(NT), 0, s,
+                       static_cast<const double*>(ix->rows), n, ld, d, w.p.labels, k, w.p.psum,
+                       w.p.pcount, st);
+  else
+    hipLaunchKernelGGL(kmeans_partial_ballot_kernel<float>, grid, dim3(NT), 0, s,
+                       static_cast<const float*>(ix->rows), n, ld, d, w.p.labels, k, w.p.psum,
+                       w.p.pcount, st);
   SC_HIP(hipGetLastError());
   return SC_OK;
 }
@@ -1059,57 +1288,75 @@ int sc_kmeans_plus_plus(const sc_index* index, size_t k, int has_seed, uint64_t 
   hipStream_t s = stream_for(index);
   // rand_custom.rs:8-33: Some(seed) -> seed_from_u64(seed); None -> 0
   SmallRng rng(has_seed ? seed : 0);
-  const size_t es = elem_size(index->dtype);
-  const size_t row_bytes = index->ld * es;
-  DevBuf cen, dmin, dy;
-  SC_HIP(cen.alloc(row_bytes, s));
+  // kmeans.rs:358-362: first centre is a uniformly drawn row; then one draw
+  // per further centre
+  std::vector<double> draws(k, 0.0);
+  const int64_t pick0 = static_cast<int64_t>(rng.gen_range(static_cast<uint64_t>(n)));
+  for (size_t j = 1; j < k; ++j) draws[j] = rng.gen_f64();
+  const int64_t nb = (n + kPPRows - 1) / kPPRows;
+  DevBuf ddraw, dpick, dmin, dy, part, dst;
+  SC_HIP(ddraw.alloc(sizeof(double) * k, s));
+  SC_HIP(dpick.alloc(sizeof(int64_t) * k, s));
   SC_HIP(dmin.alloc(sizeof(double) * n, s));
   SC_HIP(dy.alloc(sizeof(uint32_t) * n, s));
+  SC_HIP(part.alloc(sizeof(double) * nb, s));
+  SC_HIP(dst.alloc(sizeof(PPState), s));
   SC_HIP(hipMemsetAsync(dy.p, 0, sizeof(uint32_t) * n, s));
-  const unsigned grid = static_cast<unsigned>((n + 255) / 256);
-  hipLaunchKernelGGL(fill_kernel, dim3(grid), dim3(256), 0, s, dmin.as<double>(), n, DBL_MAX);
-  SC_HIP(hipGetLastError());
-  const char* base = static_cast<const char*>(index->rows);
-  // kmeans.rs:358-362: first centre is a uniformly drawn row
-  const uint64_t pick = rng.gen_range(static_cast<uint64_t>(n));
-  SC_HIP(hipMemcpyAsync(cen.p, base + pick * row_bytes, row_bytes, hipMemcpyDeviceToDevice, s));
-  std::vector<double> hd(static_cast<size_t>(n));
-  auto round = [&](uint32_t label) -> int {
+  SC_HIP(hipMemsetAsync(dst.p, 0, sizeof(PPState), s));
+  if (int rc = upload_staged(ddraw.p, draws.data(), sizeof(double) * k, s)) return rc;
+  if (int rc = upload_staged(dpick.p, &pick0, sizeof(int64_t), s)) return rc;
+  auto round = [&](size_t label) -> int {
     if (index->dtype == SC_F64)
-      hipLaunchKernelGGL(kmeanspp_round_kernel<double>, dim3(grid), dim3(256), 0, s,
-                         static_cast<const double*>(index->rows), n, static_cast<int>(index->ld),
-                         cen.as<double>(), dmin.as<double>(), dy.as<uint32_t>(), label);
+      hipLaunchKernelGGL(kmeanspp_round_kernel<double>, dim3(static_cast<unsigned>(nb)), dim3(kPPRows), 0,
+                         s, static_cast<const double*>(index->rows), n, static_cast<int>(index->ld),
+                         dpick.as<int64_t>(), dmin.as<double>(), dy.as<uint32_t>(),
+                         static_cast<uint32_t>(label), part.as<double>(), dst.as<PPState>());
     else
-      hipLaunchKernelGGL(kmeanspp_round_kernel<float>, dim3(grid), dim3(256), 0, s,
-                         static_cast<const float*>(index->rows), n, static_cast<int>(index->ld),
-                         cen.as<float>(), dmin.as<double>(), dy.as<uint32_t>(), label);
+      hipLaunchKernelGGL(kmeanspp_round_kernel<float>, dim3(static_cast<unsigned>(nb)), dim3(kPPRows), 0,
+                         s, static_cast<const float*>(index->rows), n, static_cast<int>(index->ld),
+                         dpick.as<int64_t>(), dmin.as<double>(), dy.as<uint32_t>(),
+                         static_cast<uint32_t>(label), part.as<double>(), dst.as<PPState>());
     SC_HIP(hipGetLastError());
     return SC_OK;
   };
-  for (size_t j = 1; j < k; ++j) {
-    if (int rc = round(static_cast<uint32_t>(j - 1))) return rc;
-    SC_HIP(hipMemcpyAsync(hd.data(), dmin.p, sizeof(double) * n, hipMemcpyDeviceToHost, s));
+  // rounds first .. k: round j labels rows against centre j - 1 and picks
+  // centre j; the last only labels
+  for (size_t first = 1;;) {
+    for (size_t j = first; j <= k; ++j) {
+      if (int rc = round(j - 1)) return rc;
+      if (j < k) {
+        hipLaunchKernelGGL(kmeanspp_pick_kernel, dim3(1), dim3(kPPRows), 0, s, dmin.as<double>(), n,
+                           part.as<double>(), nb, ddraw.as<double>(), static_cast<uint32_t>(j),
+                           dpick.as<int64_t>(), dst.as<PPState>());
+        SC_HIP(hipGetLastError());
+      }
+    }
+    PPState hs{};
+    SC_HIP(hipMemcpyAsync(&hs, dst.p, sizeof(hs), hipMemcpyDeviceToHost, s));
     SC_HIP(hipStreamSynchronize(s));
+    if (hs.round == 0) break;
+    // the host decides this centre as the reference does
+    std::vector<double> hd(static_cast<size_t>(n));
+    if (int rc = download_staged(hd.data(), dmin.p, sizeof(double) * n, s)) return rc;
     // kmeans.rs:381-394: sequential sum, cutoff, linear cumulative scan
     double sum = 0.0;
     for (int64_t i = 0; i < n; ++i) sum += hd[i];
-    const double cutoff = rng.gen_f64() * sum;
+    const double cutoff = draws[hs.round] * sum;
     double cost = 0.0;
-    int64_t index_i = 0;
-    while (index_i < n) {
-      cost += hd[index_i];
+    int64_t at = 0;
+    while (at < n) {
+      cost += hd[at];
       if (cost >= cutoff) break;
-      index_i += 1;
+      at += 1;
     }
     // the reference would index past the end here (only reachable with a
     // NaN sum); stay on the last row instead
-    if (index_i >= n) index_i = n - 1;
-    SC_HIP(hipMemcpyAsync(cen.p, base + index_i * row_bytes, row_bytes, hipMemcpyDeviceToDevice, s));
+    if (at >= n) at = n - 1;
+    if (int rc = upload_staged(dpick.as<int64_t>() + hs.round, &at, sizeof(int64_t), s)) return rc;
+    SC_HIP(hipMemsetAsync(dst.p, 0, sizeof(PPState), s));
+    first = hs.round + 1;
   }
-  if (int rc = round(static_cast<uint32_t>(k - 1))) return rc;
-  SC_HIP(hipMemcpyAsync(labels, dy.p, sizeof(uint32_t) * n, hipMemcpyDeviceToHost, s));
-  SC_HIP(hipStreamSynchronize(s));
-  return SC_OK;
+  return download_staged(labels, dy.p, sizeof(uint32_t) * n, s);
 }
 
 }  // extern "C"

@@ -156,5 +156,9 @@ int kmeans_tables_launch(const KmProb* d_probs, size_t count, hipStream_t s);
 // partial of the FP64 form).
 int kmeans_mixed_step_launch(const sc_index* ix, KmWork& w, hipStream_t s);
 bool kmeans_mixed_supported(const sc_index* ix, int k);
+// The block partial sums alone, from labels sorted in LDS (f64 or f32 rows):
+// the same partials as the FP64 form's partial kernels.
+bool kmeans_sorted_sums_supported(int k, int ld);
+int kmeans_sorted_sums_launch(const sc_index* ix, KmWork& w, hipStream_t s);
 
 }  // namespace sc

@@ -551,14 +551,71 @@ __global__ __launch_bounds__((Cfg<KBM, KSM, W>::NTH), (Cfg<KBM, KSM, W>::label_w
 // partials bit for bit.
 constexpr int kSumWaves = 8;
 constexpr int kSumThreads = 64 * kSumWaves;
-constexpr int kSumBatch = 32;
+// rows of a run in flight (registers: half as many of f64)
+template <typename T>
+constexpr int kSumBatch = sizeof(T) == 4 ? 32 : 16;
 constexpr int kSumMaxK = 128;
 constexpr int kSumGroups = kBlockRows / 64 / kSumWaves;  // 64-row groups per wave
 
-// DPL: dimensions per lane (2 when some row is wider than 64 values).
-template <int DPL>
-__global__ __launch_bounds__(kSumThreads, DPL == 1 ? 4 : 2) void km_sums_kernel(
+// The runs of rows of up to 64 / G values: a load takes G rows at once (lane
+// group g of 64 / G lanes holds row G t + g), so NB loads keep G NB rows in
+// flight, and they go through the wavefront's LDS tile to be added in row
+// order, one LDS read per row and dimension.  Rows past the run's end are
+// stored as +0.0, which changes no bit of a sum that starts at +0.0 (it is
+// never -0.0), so the adds need no test.  One row per load leaves most lanes
+// idle and a run's chain bound by latency: 100,000 x 16 f64 rows in 10
+// clusters took 40 us a step that way and take 17 (22 with the rows brought
+// across the lanes by shuffles).
+constexpr int kPackLoads = 16;
+template <typename T, int G, typename Rows, typename Sums, typename Counts>
+__device__ __forceinline__ void sum_runs_packed(Rows rows, int ld, int d, int k, int wave, int lane,
+                                                const uint16_t* perm, const uint32_t* start, T* tile,
+                                                Sums psum, Counts pcount) {
+  constexpr int LW = 64 / G;
+  constexpr int NR = G * kPackLoads;  // rows of a batch
+  const int g = lane / LW, jl = lane % LW;
+  const int j = min(jl, ld - 1);  // (past ld: a value that is never stored)
+  for (int c = wave; c < k; c += kSumWaves) {
+    const int e0 = static_cast<int>(start[c]), e1 = static_cast<int>(start[c + 1]);
+    double acc = 0.0;
+    for (int e = e0; e < e1; e += NR) {
+      const int nv = e1 - e;
+      T x[kPackLoads];
+#pragma unroll
+      for (int t = 0; t < kPackLoads; ++t)
+        x[t] = rows[static_cast<int64_t>(perm[min(e + t * G + g, e1 - 1)]) * ld + j];
+#pragma unroll
+      for (int t = 0; t < kPackLoads; ++t)
+        tile[(t * G + g) * LW + jl] = t * G + g < nv ? x[t] : T(0);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int t0 = 0; t0 < NR; t0 += 16) {
+        if (t0 < nv) {
+          T v[16];
+#pragma unroll
+          for (int t = 0; t < 16; ++t) v[t] = tile[(t0 + t) * LW + jl];
+#pragma unroll
+          for (int t = 0; t < 16; ++t) acc = acc + static_cast<double>(v[t]);
+        }
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
+    if (lane < d) psum[static_cast<int64_t>(c) * d + lane] = acc;
+    if (lane == 0) pcount[c] = static_cast<uint32_t>(e1 - e0);
+  }
+}
+
+// T: the rows' type.  DPL: dimensions per lane (2 when some row is wider than
+// 64 values).  PACK: narrow rows in few clusters take the packed runs (whose
+// tiles cost LDS): a block's runs average at least 64 rows there.
+constexpr int kPackMaxK = 32;
+constexpr int kPackTile = 64 * kPackLoads;  // values: NR rows of LW
+template <typename T, int DPL, bool PACK>
+__global__ __launch_bounds__(kSumThreads, DPL == 1 && !(PACK && sizeof(T) == 8) ? 4 : 2) void km_sums_kernel(
     const KmProb* __restrict__ P, const uint2* __restrict__ items, int64_t nitems) {
+  __shared__ T tiles[PACK ? kSumWaves * kPackTile : 1];
   __shared__ uint32_t lab[kBlockRows];
   __shared__ uint16_t perm[kBlockRows];
   __shared__ uint32_t pos[kSumWaves][kSumMaxK];
@@ -645,7 +702,14 @@ __global__ __launch_bounds__(kSumThreads, DPL == 1 ? 4 : 2) void km_sums_kernel(
     // the runs
     const int64_t kd = static_cast<int64_t>(k) * d;
     const auto psum = to_global(p.psum) + b * kd;
-    const auto rows = to_global(static_cast<const float*>(p.rows)) + r0 * ld;
+    const auto rows = to_global(static_cast<const T*>(p.rows)) + r0 * ld;
+    if constexpr (PACK) {
+      T* tile = tiles + wave * kPackTile;
+      if (ld <= 16)
+        sum_runs_packed<T, 4>(rows, ld, d, k, wave, lane, perm, start, tile, psum, to_global(p.pcount) + b * k);
+      else
+        sum_runs_packed<T, 2>(rows, ld, d, k, wave, lane, perm, start, tile, psum, to_global(p.pcount) + b * k);
+    } else {
     // two runs at a time: clusters c and c + kSumWaves, kSumBatch rows of
     // each requested before either is added
     const int j0 = min(lane, ld - 1), j1 = min(lane + 64, ld - 1);
@@ -660,14 +724,14 @@ __global__ __launch_bounds__(kSumThreads, DPL == 1 ? 4 : 2) void km_sums_kernel(
       }
       while (e[0] < e1[0] || e[1] < e1[1]) {
         int nv[2];
-        float x[2][kSumBatch][DPL];
+        T x[2][kSumBatch<T>][DPL];
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-          nv[u] = max(0, min(kSumBatch, e1[u] - e[u]));
+          nv[u] = max(0, min(kSumBatch<T>, e1[u] - e[u]));
           const uint32_t mine = lane < nv[u] ? perm[e[u] + lane] : 0u;
           // lanes at or past ld read an in-row value that is never stored
 #pragma unroll
-          for (int t = 0; t < kSumBatch; ++t) {
+          for (int t = 0; t < kSumBatch<T>; ++t) {
             const uint32_t r = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(mine), t));
             x[u][t][0] = rows[static_cast<int64_t>(r) * ld + j0];
             if (DPL > 1) x[u][t][1] = rows[static_cast<int64_t>(r) * ld + j1];
@@ -676,11 +740,11 @@ __global__ __launch_bounds__(kSumThreads, DPL == 1 ? 4 : 2) void km_sums_kernel(
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
 #pragma unroll
-          for (int t = 0; t < kSumBatch; ++t)
-            if (t < nv[u]) {
-              acc[u][0] = acc[u][0] + static_cast<double>(x[u][t][0]);
-              if (DPL > 1) acc[u][1] = acc[u][1] + static_cast<double>(x[u][t][1]);
-            }
+          for (int t = 0; t < kSumBatch<T>; ++t) {
+            // (+0.0 past the run's end, see sum_runs_packed)
+            acc[u][0] = acc[u][0] + static_cast<double>(t < nv[u] ? x[u][t][0] : T(0));
+            if (DPL > 1) acc[u][1] = acc[u][1] + static_cast<double>(t < nv[u] ? x[u][t][1] : T(0));
+          }
           e[u] += nv[u];
         }
       }
@@ -692,6 +756,7 @@ __global__ __launch_bounds__(kSumThreads, DPL == 1 ? 4 : 2) void km_sums_kernel(
           if (lane == 0)
             to_global(p.pcount)[b * k + cc[u]] = start[cc[u] + 1] - start[cc[u]];
         }
+    }
     }
     __syncthreads();  // LDS is rewritten by the next item
   }
@@ -770,13 +835,18 @@ int launch_label(int kbm, int ksm, int mult, const KmProb* dP, const uint2* item
 }
 
 // ldmax: the widest padded row among the items' problems.
-int launch_sums(const KmProb* dP, const uint2* items, int64_t nitems, int ldmax, int cus,
+template <typename T>
+int launch_sums(const KmProb* dP, const uint2* items, int64_t nitems, int ldmax, int k, int cus,
                 hipStream_t s) {
   const unsigned grid = static_cast<unsigned>(std::max<int64_t>(1, std::min<int64_t>(nitems, 4 * cus)));
+  // the packed form for a single problem only: a batch's launch holds every
+  // shape, and the tiles' LDS would cost its many-cluster problems occupancy
   if (ldmax > 64)
-    hipLaunchKernelGGL(km_sums_kernel<2>, dim3(grid), dim3(kSumThreads), 0, s, dP, items, nitems);
+    hipLaunchKernelGGL((km_sums_kernel<T, 2, false>), dim3(grid), dim3(kSumThreads), 0, s, dP, items, nitems);
+  else if (!items && ldmax <= 32 && k <= kPackMaxK)
+    hipLaunchKernelGGL((km_sums_kernel<T, 1, true>), dim3(grid), dim3(kSumThreads), 0, s, dP, items, nitems);
   else
-    hipLaunchKernelGGL(km_sums_kernel<1>, dim3(grid), dim3(kSumThreads), 0, s, dP, items, nitems);
+    hipLaunchKernelGGL((km_sums_kernel<T, 1, false>), dim3(grid), dim3(kSumThreads), 0, s, dP, items, nitems);
   SC_HIP(hipGetLastError());
   return SC_OK;
 }
@@ -800,6 +870,14 @@ bool kmeans_mixed_supported(const sc_index* ix, int k) {
   return ix->dtype == SC_F32 && class_fits(k, static_cast<int>(ix->ld));
 }
 
+bool kmeans_sorted_sums_supported(int k, int ld) { return k <= kSumMaxK && ld <= 128; }
+
+int kmeans_sorted_sums_launch(const sc_index* ix, KmWork& w, hipStream_t s) {
+  const int ld = w.p.ld, cus = device_cus();
+  return ix->dtype == SC_F64 ? launch_sums<double>(w.dprob, nullptr, w.p.nb, ld, w.p.k, cus, s)
+                             : launch_sums<float>(w.dprob, nullptr, w.p.nb, ld, w.p.k, cus, s);
+}
+
 int kmeans_mixed_step_launch(const sc_index* ix, KmWork& w, hipStream_t s) {
   if (w.p.nb == 0) return SC_OK;
   const int k = w.p.k, ld = w.p.ld;
@@ -809,7 +887,7 @@ int kmeans_mixed_step_launch(const sc_index* ix, KmWork& w, hipStream_t s) {
   const int64_t nseg = (w.p.n + kSegRows - 1) / kSegRows;
   ProfScope ps("kmeans_mixed_assign", s);
   if (int rc = launch_label(kbm, ksm, 0, w.dprob, nullptr, nseg, exact, cus, s)) return rc;
-  return launch_sums(w.dprob, nullptr, w.p.nb, ld, cus, s);
+  return launch_sums<float>(w.dprob, nullptr, w.p.nb, ld, w.p.k, cus, s);
 }
 
 // ------------------------------------------------------------------ batch
@@ -1211,7 +1289,7 @@ extern "C" int sc_kmeans_batch_run(const sc_kmeans_problem* problems, size_t cou
         if (int rc = launch_label(K->kbm, K->ksm, mult, dG, bItems.as<uint2>() + K->at,
                                   static_cast<int64_t>(K->items.size()), K->exact, cus, s))
           return rc;
-      if (int rc = launch_sums(dG, d_all, nall, G.ldmax, cus, s)) return rc;
+      if (int rc = launch_sums<float>(dG, d_all, nall, G.ldmax, kSumMaxK, cus, s)) return rc;
       return kmeans_reduce_launch(dG, G.red, true, true, s);
     };
 
