@@ -254,6 +254,12 @@ int knn_l1_mixed_device(const sc_index* index, const void* d_queries, size_t q, 
                         int64_t* d_idx, double* d_dist, uint32_t* d_count, hipStream_t stream,
                         sc_stats* stats);
 
+// The 16-bit coded form of the same (coded: whether the index's values allow
+// it; k <= 64).
+int ensure_q16(sc_index* ix, bool* coded, hipStream_t s);
+int knn_l1q_device(const sc_index* index, const float* d_queries, int64_t q, int k, int64_t* d_idx,
+                   double* d_dist, uint32_t* d_count, hipStream_t stream, sc_stats* stats);
+
 int knn_mixed_device(const sc_index* index, const void* d_queries, size_t q, size_t k,
                      int64_t* d_idx, double* d_dist, uint32_t* d_count, hipStream_t stream,
                      sc_stats* stats);

@@ -201,7 +201,7 @@ __global__ __launch_bounds__(256) void dbscan_verify_kernel(const T* __restrict_
   for (unsigned long long e = static_cast<unsigned long long>(blockIdx.x) * blockDim.x + threadIdx.x;
        e < m; e += static_cast<unsigned long long>(gridDim.x) * blockDim.x) {
     const uint2 p = pairs[e];
-    const double s = exact_sum(rows + static_cast<int64_t>(p.x) * ld, rows + static_cast<int64_t>(p.y) * ld, ld);
+    const double s = exact_sum<T, kEuclid>(rows + static_cast<int64_t>(p.x) * ld, rows + static_cast<int64_t>(p.y) * ld, ld);
     if (__builtin_sqrt(s) <= radius) {
       atomicAdd(&degree[p.x], 1u);
       atomicAdd(&degree[p.y], 1u);

@@ -31,7 +31,7 @@
 // hardly a row is tested in vain.
 //
 // Bound by the FP64 matrix rate (72 TFLOP/s in a large matrix product on
-// this card): 4,096 queries x 200,000 x 64 f64 rows take 2.56 ms (12.8 ms
+// this card): 4,096 queries x 200,000 x 64 f64 rows take 2.49 ms (12.8 ms
 // with a tile of vector subtract, multiply, add), 3,001 x 750,000 x 100 f32
 // 8.2 ms (42.0), 56 TFLOP/s.  The prefix is 1,024 rows because its selection
 // is a walk per query; two levels then leave about 250 candidates per query
@@ -46,6 +46,7 @@
 #include "common.hpp"
 #include "heap.hpp"
 #include "metric.hpp"
+#include "knn_lists.hpp"
 #include "mfma64.hpp"
 
 namespace sc {
@@ -57,11 +58,6 @@ int launch_serial_exact(const sc_index* index, const void* d_queries, int k, con
 
 namespace {
 
-constexpr int64_t kDenseRows = 1024;
-constexpr int kFinishThreads = 128;
-constexpr int kFinishBatch = 1024;   // candidates rescored and replayed at a time
-constexpr int kSelectWaves = 4;
-constexpr int kMaxLevels = 8;
 
 // Sixteen lanes per row: the squared norm (any order: the gap covers it).
 template <typename T>
@@ -112,12 +108,6 @@ __global__ void query_norms_kernel(const T* __restrict__ qs, int64_t q, int ld, 
   if (finite && !in) list[atomicAdd(list_n, 1u)] = static_cast<uint32_t>(i);
 }
 
-__global__ void zero_words_kernel(uint32_t* p, int64_t n) {
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
-       i += static_cast<int64_t>(gridDim.x) * blockDim.x)
-    p[i] = 0u;
-}
-
 // L of queries x the first `cols` rows (a multiple of kMR, rows past the
 // index +inf), row-major by query.  One workgroup per (query tile, row tile).
 template <typename T>
@@ -151,28 +141,6 @@ __global__ __launch_bounds__(kMT, 2) void dense_kernel(const T* __restrict__ row
   });
 }
 
-// The k smallest values a wavefront has seen, ascending in lanes 0 .. k-1.
-struct KSmallest {
-  double b;    // lane's entry
-  double kth;
-  // "none seen".  The compiler keeps a uniform f64 in a scalar register pair
-  // and writes the constant +inf there with one s_mov_b64, whose literal
-  // holds the low half only (it reads back as 0.0); the empty asm keeps the
-  // value in vector registers.
-  __device__ __forceinline__ void clear() {
-    double inf = INFINITY;
-    asm volatile("" : "+v"(inf));
-    b = inf;
-    kth = inf;
-  }
-  __device__ __forceinline__ void insert(double x, int lane, int k) {
-    double prev = __shfl_up(b, 1);
-    if (lane == 0) prev = -INFINITY;
-    if (lane < k && x < b) b = x < prev ? prev : x;
-    kth = lane_value(b, k - 1);
-  }
-};
-
 __global__ __launch_bounds__(64 * kSelectWaves) void select_dense_kernel(
     const double* __restrict__ L, int64_t cols, const double* __restrict__ y2m,
     const double* __restrict__ x2m, int64_t q, int k, Bound64 bd, int cap,
@@ -181,7 +149,7 @@ __global__ __launch_bounds__(64 * kSelectWaves) void select_dense_kernel(
   const int64_t qi = static_cast<int64_t>(blockIdx.x) * kSelectWaves + (threadIdx.x >> 6);
   if (qi >= q) return;  // the whole wave
   const double x2 = x2m[qi];
-  KSmallest ks;
+  KSmallest<double> ks;
   ks.clear();
   uint32_t cnt = 0;
   const double* l = L + qi * cols;
@@ -217,29 +185,11 @@ __global__ __launch_bounds__(64 * kSelectWaves) void select_dense_kernel(
   if (lane == 0) cand_count[qi] = cnt;
 }
 
-// One level of the scan.  Its (query tile, row tile) pairs, query tiles
-// outermost, are dealt to the workgroups in contiguous runs of `per`, so all
-// end together; the part of a run inside one query tile is a piece, with one
-// candidate list per query.  The pieces of query tile qt are the workgroups
-// from qt * tiles / per on.
-struct Level {
-  int64_t row0, tiles, per, groups;
-  int lists;  // per query
-  int cap;    // entries per list
-  int64_t entry0, list0;  // where the level's lists begin (per query)
-};
-struct ScanOut {
-  uint32_t* idx;    // q x entries
-  double* u;        // q x entries
-  uint32_t* count;  // q x lists
-  int64_t entries, lists;  // per query, all levels
-};
-
 template <typename T>
 __global__ __launch_bounds__(kMT, 2) void scan_kernel(
     const T* __restrict__ rows, int64_t n, int ld, int d, const double* __restrict__ y2m,
     const T* __restrict__ queries, int64_t q, const double* __restrict__ x2m,
-    const double* __restrict__ seed, int k, Bound64 bd, Level lv, ScanOut out) {
+    const double* __restrict__ seed, int k, Bound64 bd, Level lv, ScanOut<double> out) {
   __shared__ MSmem sm;
   const MLane ml;
   const int64_t nqt = (q + kMQ - 1) / kMQ;
@@ -292,18 +242,9 @@ __global__ __launch_bounds__(kMT, 2) void scan_kernel(
           const double* u = out.u + slot_of(ml.wave * 32 + 16 * j + src, 0);
           // entries that other lanes of this wavefront stored
           __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
-          KSmallest ks;
+          KSmallest<double> ks;
           ks.clear();
-          for (uint32_t c0 = 0; c0 < m; c0 += 64) {
-            const double x = c0 + ml.lane < m ? u[c0 + ml.lane] : INFINITY;
-            uint64_t b = __ballot(x < ks.kth);
-            while (b) {
-              const int s2 = __builtin_ctzll(b);
-              ks.insert(lane_value(x, s2), ml.lane, k);
-              b &= b - 1;
-              b &= __ballot(x < ks.kth);
-            }
-          }
+          ks.take(u, m, ml.lane, k);
           if (ml.lr == src) {
             const double lower = acc_threshold(bd, ks.kth, x2[j]);
             if (lower < th[j]) th[j] = lower;
@@ -322,162 +263,6 @@ __global__ __launch_bounds__(kMT, 2) void scan_kernel(
   }
 }
 
-// The k smallest U of the earlier levels (seed) and the entries of one
-// level's lists, in place.
-__global__ __launch_bounds__(64 * kSelectWaves) void select_level_kernel(Level lv, ScanOut in,
-                                                                         int64_t q, int k,
-                                                                         double* __restrict__ seed) {
-  const int lane = threadIdx.x & 63;
-  const int64_t qi = static_cast<int64_t>(blockIdx.x) * kSelectWaves + (threadIdx.x >> 6);
-  if (qi >= q) return;  // the whole wave
-  KSmallest ks;
-  ks.b = lane < k ? seed[qi * k + lane] : INFINITY;
-  ks.kth = lane_value(ks.b, k - 1);
-  const uint32_t* cc = in.count + qi * in.lists + lv.list0;
-  const double* u = in.u + qi * in.entries + lv.entry0;
-  for (int l0 = 0; l0 < lv.lists; l0 += 64) {
-    // 64 counts at once, then the non-empty lists one by one
-    const uint32_t cl = l0 + lane < lv.lists ? min(cc[l0 + lane], static_cast<uint32_t>(lv.cap)) : 0u;
-    uint64_t some = __ballot(cl != 0u);
-    while (some) {
-      const int li = __builtin_ctzll(some);
-      some &= some - 1;
-      const uint32_t c = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(cl), li));
-      const double* ul = u + static_cast<int64_t>(l0 + li) * lv.cap;
-      for (uint32_t c0 = 0; c0 < c; c0 += 64) {
-        const double x = c0 + lane < c ? ul[c0 + lane] : INFINITY;
-        uint64_t m = __ballot(x < ks.kth);
-        while (m) {
-          const int src = __builtin_ctzll(m);
-          ks.insert(lane_value(x, src), lane, k);
-          m &= m - 1;
-          m &= __ballot(x < ks.kth);
-        }
-      }
-    }
-  }
-  if (lane < k) seed[qi * k + lane] = ks.b;
-}
-
-// Where the lists of a query lie: list 0 is the dense prefix's (its own
-// array), then each level's.
-struct Lists {
-  const uint32_t* pre_idx;
-  const uint32_t* pre_count;
-  int pre_cap;
-  ScanOut out;
-  int nlevels;
-  Level lv[kMaxLevels];
-};
-
-// S of every candidate and the heap replay (see the file comment).  The
-// candidates are numbered across the lists by a prefix sum of the counts and
-// taken kFinishBatch at a time: all threads compute their S, then the first
-// wavefront replays the batch from LDS, 64 entries at a time.
-template <typename T>
-__global__ __launch_bounds__(kFinishThreads) void finish_kernel(
-    const T* __restrict__ rows, int ld, const T* __restrict__ queries, int64_t q, int k, Lists ls,
-    int64_t* __restrict__ out_idx, double* __restrict__ out_dist, uint32_t* __restrict__ out_count,
-    uint32_t* __restrict__ list, uint32_t* __restrict__ list_n,
-    unsigned long long* __restrict__ total_cand) {
-  extern __shared__ __align__(16) uint32_t start[];  // nl + 1
-  __shared__ double s_S[kFinishBatch];
-  __shared__ uint32_t s_row[kFinishBatch];
-  __shared__ uint32_t s_over;
-  const int64_t qi = blockIdx.x;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int nl = 1 + static_cast<int>(ls.out.lists);
-  if (tid == 0) s_over = 0u;
-  __syncthreads();
-  if (tid < 64) {
-    uint32_t acc = 0;
-    bool over = false;
-    for (int l0 = 0; l0 < nl; l0 += 64) {
-      const int l = l0 + lane;
-      uint32_t c = 0;
-      if (l < nl) {
-        c = l == 0 ? ls.pre_count[qi] : ls.out.count[qi * ls.out.lists + l - 1];
-        int cap = ls.pre_cap;
-        if (l > 0) {
-          cap = ls.lv[0].cap;
-          for (int v = 1; v < ls.nlevels; ++v)
-            if (l - 1 >= ls.lv[v].list0) cap = ls.lv[v].cap;
-        }
-        over = over || c > static_cast<uint32_t>(cap);
-      }
-      uint32_t inc = c;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t up = __shfl_up(inc, o);
-        if (lane >= o) inc += up;
-      }
-      if (l < nl) start[l] = acc + inc - c;
-      acc += __shfl(inc, 63);
-    }
-    if (lane == 0) start[nl] = acc;
-    if (__ballot(over) != 0 && lane == 0) {
-      s_over = 1u;
-      list[atomicAdd(list_n, 1u)] = static_cast<uint32_t>(qi);
-      out_count[qi] = 0u;
-    }
-  }
-  __syncthreads();
-  if (s_over) return;
-  const uint32_t total = start[nl];
-  const T* qrow = queries + qi * ld;
-  double hd = INFINITY, top = INFINITY;
-  uint32_t hi = 0xffffffffu;
-  for (uint32_t e0 = 0; e0 < total; e0 += kFinishBatch) {
-    const uint32_t m = min(total - e0, static_cast<uint32_t>(kFinishBatch));
-    for (uint32_t e = tid; e < m; e += kFinishThreads) {
-      // the list of candidate e0 + e: the last whose start is at or below it
-      int lo = 0, hi_l = nl;
-      while (hi_l - lo > 1) {
-        const int mid = (lo + hi_l) >> 1;
-        if (start[mid] <= e0 + e)
-          lo = mid;
-        else
-          hi_l = mid;
-      }
-      const uint32_t at = e0 + e - start[lo];
-      uint32_t row;
-      if (lo == 0) {
-        row = ls.pre_idx[qi * ls.pre_cap + at];
-      } else {
-        int v = 0;
-        while (v + 1 < ls.nlevels && lo - 1 >= ls.lv[v + 1].list0) ++v;
-        row = ls.out.idx[qi * ls.out.entries + ls.lv[v].entry0 +
-                         (lo - 1 - ls.lv[v].list0) * ls.lv[v].cap + at];
-      }
-      const double s = exact_sum(qrow, rows + static_cast<int64_t>(row) * ld, ld);
-      s_S[e] = s;
-      s_row[e] = row;
-    }
-    __syncthreads();
-    if (tid < 64) {
-      for (uint32_t c0 = 0; c0 < m; c0 += 64) {
-        const bool valid = c0 + lane < m;
-        const double dv = valid ? __builtin_sqrt(s_S[c0 + lane]) : 0.0;
-        const uint32_t row = valid ? s_row[c0 + lane] : 0u;
-        uint64_t b = __ballot(valid && dv < top);
-        while (b) {
-          const int src = __builtin_ctzll(b);
-          lane_heap_push_root(hd, hi, lane, k, lane_value(dv, src),
-                              static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(row), src)));
-          top = lane_value(hd, 0);
-          b &= b - 1;
-          b &= __ballot(valid && dv < top);
-        }
-      }
-    }
-    __syncthreads();
-  }
-  if (tid < 64) {
-    if (lane == 0) atomicAdd(total_cand, static_cast<unsigned long long>(total));
-    lane_heap_store(hd, hi, lane, k, out_idx + qi * k, out_dist + qi * k, out_count + qi);
-  }
-}
-
 template <typename T>
 int run_f64(const sc_index* index, const T* d_queries, int64_t q, int k, int64_t* d_idx,
             double* d_dist, uint32_t* d_count, hipStream_t s, sc_stats* stats) {
@@ -489,46 +274,16 @@ int run_f64(const sc_index* index, const T* d_queries, int64_t q, int k, int64_t
   const double* y2m = nullptr;
   if (int rc = ensure_norms64(const_cast<sc_index*>(index), local, &y2m, s)) return rc;
 
-  // Levels: the dense prefix, then m ranges growing by the same factor (at
-  // most 16: k (factor - 1) candidates per query and level against one scan
-  // and one selection launch for a further level).
   const int64_t cols = std::min<int64_t>(kDenseRows, (n + kMR - 1) / kMR * kMR);
-  std::vector<int64_t> edge{cols};
-  if (n > cols) {
-    const double span = static_cast<double>(n) / static_cast<double>(cols);
-    const int m = std::max(1, std::min(kMaxLevels, static_cast<int>(std::ceil(std::log(span) / std::log(16.0)))));
-    for (int i = 1; i < m; ++i)
-      edge.push_back(std::max<int64_t>(
-          edge.back() + kMR, static_cast<int64_t>(cols * std::pow(span, double(i) / m)) / kMR * kMR));
-    edge.push_back(n);
-  }
+  const std::vector<int64_t> edge = level_edges(n, cols);
   const int nlev = static_cast<int>(edge.size()) - 1;
-  auto expect = [&](double len) { return k * (1.0 + std::log(std::max(1.0, len / k))); };
-  const int pre_cap = static_cast<int>(std::min<int64_t>(cols, static_cast<int64_t>(3.0 * expect(cols)) + 64));
-  auto plan = [&](int64_t qn, Level (&lv)[kMaxLevels], ScanOut& o) {
-    const int64_t nqt = (qn + kMQ - 1) / kMQ;
-    o.entries = o.lists = 0;
-    for (int i = 0; i < nlev; ++i) {
-      Level& v = lv[i];
-      v.row0 = edge[i];
-      v.tiles = (edge[i + 1] - edge[i] + kMR - 1) / kMR;
-      const int64_t items = nqt * v.tiles;
-      // two workgroups per CU fit (LDS and registers)
-      v.per = std::max<int64_t>(1, (items + 511) / 512);
-      v.groups = (items + v.per - 1) / v.per;
-      v.lists = static_cast<int>(std::min<int64_t>((v.tiles + v.per - 1) / v.per + 1, v.tiles));
-      const int64_t len = std::min<int64_t>(v.per * kMR, v.tiles * kMR);
-      // a tile that passes whole, one look's growth, and the running-k-th
-      // improvements after it with room to spare
-      v.cap = static_cast<int>(std::min<int64_t>(
-          len, kMR + std::max(2 * k, 32) + static_cast<int64_t>(4.0 * expect(static_cast<double>(len)))));
-      v.entry0 = o.entries;
-      v.list0 = o.lists;
-      o.entries += static_cast<int64_t>(v.lists) * v.cap;
-      o.lists += v.lists;
-    }
+  const int pre_cap = static_cast<int>(std::min<int64_t>(
+      cols, static_cast<int64_t>(3.0 * expected_entrants(k, static_cast<double>(cols))) + 64));
+  // two workgroups per CU fit (LDS and registers)
+  auto plan = [&](int64_t qn, Level (&lv)[kMaxLevels], ScanOut<double>& o) {
+    plan_levels(edge, qn, kMQ, 512, k, lv, o);
   };
-  Lists ls{};
+  Lists<double> ls{};
   ls.nlevels = nlev;
   ls.pre_cap = pre_cap;
   // the candidate store of a call is bounded by batches of queries (whole
@@ -595,17 +350,17 @@ int run_f64(const sc_index* index, const T* d_queries, int64_t q, int k, int64_t
                            s, rows, n, ld, d, y2m, qs, qn, x2m.as<double>(), seed.as<double>(), k, bd,
                            ls.lv[i], ls.out);
         if (i + 1 < nlev)
-          hipLaunchKernelGGL(select_level_kernel, dim3(sel), dim3(64 * kSelectWaves), 0, s, ls.lv[i],
+          hipLaunchKernelGGL(select_level_kernel<double>, dim3(sel), dim3(64 * kSelectWaves), 0, s, ls.lv[i],
                              ls.out, qn, k, seed.as<double>());
         SC_HIP(hipGetLastError());
       }
     }
     {
       ProfScope ps("knn_replay", s);
-      hipLaunchKernelGGL(finish_kernel<T>, dim3(static_cast<unsigned>(qn)), dim3(kFinishThreads),
-                         sizeof(uint32_t) * (ls.out.lists + 2), s, rows, ld, qs, qn, k, ls,
+      hipLaunchKernelGGL((finish_kernel<T, kEuclid, double>), dim3(static_cast<unsigned>(qn)), dim3(kFinishThreads),
+                         finish_lds<T>(ld, ls.out.lists), s, rows, ld, qs, qn, k, ls,
                          d_idx + b0 * k, d_dist + b0 * k, d_count + b0, olist.as<uint32_t>(), list_n,
-                         total);
+                         stats ? total : nullptr);
       SC_HIP(hipGetLastError());
     }
     if (int rc = launch_serial_exact(index, qs, k, olist.as<uint32_t>(), list_n, d_idx + b0 * k,

@@ -93,31 +93,6 @@ __device__ __forceinline__ double sum_upper(const Bound64& b, double L, double n
   return u < b.limit ? u : INFINITY;  // NaN too
 }
 
-// The reference's sum of one (query, row) pair: terms in dimension order,
-// 16 values of both requested before they are folded (rows are padded to
-// multiples of 16 values).
-template <typename T>
-__device__ __forceinline__ double exact_sum(const T* __restrict__ x, const T* __restrict__ y, int ld) {
-  constexpr int PV = 16 / sizeof(T);
-  typedef T Piece __attribute__((ext_vector_type(PV)));
-  const Piece* xp = reinterpret_cast<const Piece*>(x);
-  const Piece* yp = reinterpret_cast<const Piece*>(y);
-  double s = 0.0;
-  for (int j = 0; j < ld / PV; j += 16 / PV) {
-    Piece xv[16 / PV], yv[16 / PV];
-#pragma unroll
-    for (int c = 0; c < 16 / PV; ++c) {
-      xv[c] = xp[j + c];
-      yv[c] = yp[j + c];
-    }
-#pragma unroll
-    for (int c = 0; c < 16 / PV; ++c)
-#pragma unroll
-      for (int w = 0; w < PV; ++w) s = s + Term<T, kEuclid>::f(xv[c][w], yv[c][w], 2.0);
-  }
-  return s;
-}
-
 struct MSmem {
   double R[2][kMR][kMStride];
   double Q[2][kMQ][kMStride];

@@ -262,7 +262,7 @@ __global__ __launch_bounds__(64) void radius_resolve_kernel(
           hi = mid;
       }
       row = mine[lo * cap + (e - start[lo])];
-      match = __builtin_sqrt(exact_sum(queries + qi * ld, rows + static_cast<int64_t>(row) * ld, ld)) <= radius;
+      match = __builtin_sqrt(exact_sum<T, kEuclid>(queries + qi * ld, rows + static_cast<int64_t>(row) * ld, ld)) <= radius;
     }
     // to the front: entry e lies at or past offset e, so no entry that is
     // still to be read is overwritten
@@ -298,7 +298,7 @@ __global__ __launch_bounds__(256) void radius_emit_kernel(
     out_idx[o + j] = row;
     if (out_dist)
       out_dist[o + j] =
-          __builtin_sqrt(exact_sum(queries + qi * ld, rows + static_cast<int64_t>(row) * ld, ld));
+          __builtin_sqrt(exact_sum<T, kEuclid>(queries + qi * ld, rows + static_cast<int64_t>(row) * ld, ld));
   }
 }
 
