@@ -36,7 +36,7 @@
 // Levels.  Small indexes run one such launch.  For indexes of at least
 // kSeedMinRows rows the first launch covers only the first kPrefixRows
 // rows; then fixed-threshold launches cover row ranges growing kLevelRatio
-// times.  The candidates of each level get their exact s (Pass 2a) as the
+// times.  The candidates of each level get their exact s (Pass 2) as the
 // level ends; the next level tests every row against T, the k-th smallest
 // s among the candidates of all earlier levels rounded up to f32, and
 // appends the rows with L < T.  The candidates are a subset of the earlier
@@ -49,10 +49,11 @@
 // the width of the bound, and fewer rows pass.)
 // Candidates are kept only if the per-row bound, which uses the stored
 // norms of y - bf16(y) and x - bf16(x), also has L below the threshold.
-// Pass 2 (replay, FP64).  Every candidate's exact s is computed in
-// parallel (a workgroup per query); then one wavefront per query walks its
-// lists in index order, 64 entries at a time, and applies the heap rule to
-// the entries below the heap's top, one after another.  Rows that would not
+// Pass 2 (replay, FP64).  As a level ends, a workgroup per query computes
+// the exact s of the level's candidates, all lists' entries taken together,
+// and brings them into row order; after the last level one wavefront per
+// query walks them, 64 at a time, and applies the heap rule to the entries
+// below the heap's top, one after another.  Rows that would not
 // enter the reference heap are no-ops, so the final heap array equals the
 // reference's.  Queries whose lists overflow, or whose rows are not finite
 // / too large for the bound, are recomputed by the sequential exact kernel.
@@ -98,7 +99,6 @@ constexpr int64_t kPrefixRows = 16384;    // rows of the seeding launch
 constexpr int64_t kSeedMinRows = 524288;  // indexes this large are seeded
 constexpr int64_t kLevelRatio = 8;        // row-range growth of the fixed-threshold levels
 constexpr int64_t kScanPadRows = 1024;    // padding rows past the index read by fixed launches
-constexpr int kMaxLists = 64 + 2 * 64 * 8;  // running lists + fixed pairs, any plan
 constexpr double kC1 = 0.0078125 + 1.52587890625e-05 + 128.0 * 2.384185791015625e-07;
 constexpr double kLoMargin = 3.814697265625e-06;   // 2^-18
 constexpr double kHiMargin = 1.52587890625e-05;    // 2^-16
@@ -846,222 +846,233 @@ __global__ __launch_bounds__(kNT, 2) void fixed_scan_kernel(const ScanArgs a) {
   }
 }
 
-// One wavefront per query for the sequential passes below; four per
-// workgroup.  LDS traffic of a wave is ordered by the hardware; the fence
-// keeps the compiler from moving it across the exchange points.
-constexpr int kWavesPerBlock = 4;
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-// The k smallest of a seed (null: +inf) and the exact distances, rounded
-// up to f32, of the entries in lists [l0, l0 + nl) (candidates of rows after
-// the seed's rows, distinct): the next seed, ascending.  Entries past a
-// list's cap were not stored; leaving them out keeps a valid seed.  Lanes
-// 0 .. k-1 hold the current k smallest in ascending order; a value enters
-// by one shift across the lanes.
-__global__ __launch_bounds__(64 * kWavesPerBlock) void select_seed_kernel(
-    const float* __restrict__ seed_in, const double* __restrict__ cand_S,
-    const uint32_t* __restrict__ cand_count, ListLayout lay, int l0, int nl, int64_t q, int k,
-    float* __restrict__ seed_out) {
-  const int lane = threadIdx.x & 63;
-  const int64_t qi = static_cast<int64_t>(blockIdx.x) * kWavesPerBlock + (threadIdx.x >> 6);
-  if (qi >= q) return;  // the whole wave
-  float b = (lane < k && seed_in) ? seed_in[qi * k + lane] : INFINITY;
-  if (lane >= k) b = INFINITY;
-  float kth = lane_value(b, k - 1);
-  const int64_t perq = lay.per_query();
-  for (int l = l0; l < l0 + nl; ++l) {
-    const uint32_t c = min(cand_count[static_cast<size_t>(qi) * lay.nlists() + l],
-                           static_cast<uint32_t>(lay.cap(l)));
-    const double* sv = cand_S + static_cast<size_t>(qi) * perq + lay.offset(l);
-    for (uint32_t c0 = 0; c0 < c; c0 += 64) {
-      const float v = c0 + lane < c ? __double2float_ru(sv[c0 + lane]) : INFINITY;
-      uint64_t m = __ballot(v < kth);
-      while (m) {
-        const int src = __builtin_ctzll(m);
-        const float x = lane_value(v, src);
-        float prev = __shfl_up(b, 1);
-        if (lane == 0) prev = -INFINITY;
-        if (lane < k && x < b) b = x < prev ? prev : x;
-        kth = lane_value(b, k - 1);
-        m &= m - 1;
-        m &= __ballot(v < kth);
-      }
-    }
-  }
-  if (lane < k) seed_out[qi * k + lane] = b;
-}
+// ---- rescoring, seeds and replay (Pass 2) ----
+// A level's lists are cut into units: a running launch's list, or a fixed
+// launch's pair (the two halves of its tiles, each in row order).
+constexpr int kLevelThreads = 128;
+constexpr int kLevelBatch = 1024;  // candidates ranked and rescored at a time
+constexpr int kMaxSegs = 64;       // units of a level
+constexpr int kReplayWaves = 4;
 
-// Pass 2a: the exact s of every stored candidate (the reference's
-// arithmetic: f32 differences and squares, f64 sum in dimension order).
-// One workgroup per query; its threads take the candidates in turn.
-constexpr int kRescoreThreads = 128;
-__global__ __launch_bounds__(kRescoreThreads) void mixed_rescore_kernel(
-    const float* __restrict__ rows, const float* __restrict__ qs, int ld, int64_t q, ListLayout lay,
-    int l_lo, int l_hi, const uint32_t* __restrict__ cand_idx,
-    const uint32_t* __restrict__ cand_count, const float* __restrict__ x2m,
-    double* __restrict__ cand_S) {
+// A level's end, one workgroup per query: the exact s of its candidates (the
+// reference's arithmetic: f32 differences and squares, f64 sum in dimension
+// order), each pair's entries brought into row order across its two lists
+// (the first list keeps its length), and the next seed: the k smallest of the
+// current seed (null: none) and those distances rounded up to f32.  The
+// candidates are numbered across the units by a prefix sum of the counts and
+// taken up to kLevelBatch at a time, so that all threads work whatever the
+// lists' lengths: small batches of queries have hundreds of lists of a few
+// entries each, and walking those one after another cost more than the scans
+// (a burst of 10,000 queries on 2,000,000 x 96 rows, k = 20: 12.7 ms, 8.6 with
+// these kernels and the heap's one-step sift).  Entries past a list's cap were
+// not stored; leaving them out keeps a valid seed.
+__global__ __launch_bounds__(kLevelThreads) void mixed_level_kernel(
+    const float* __restrict__ rows, const float* __restrict__ qs, int ld, ListLayout lay, int l_lo,
+    int l_hi, uint32_t* __restrict__ cand_idx, const uint32_t* __restrict__ cand_count,
+    const float* __restrict__ x2m, double* __restrict__ cand_S, int k,
+    const float* __restrict__ seed_in, float* __restrict__ seed_out) {
+  __shared__ __align__(16) float qrow[16 * kMaxKS];
+  __shared__ uint32_t start[kMaxSegs + 1], first[kMaxSegs];
+  __shared__ uint32_t s_row[kLevelBatch];
+  __shared__ float s_v[kLevelBatch];
+  __shared__ __align__(16) unsigned char tiles[kLevelThreads / 64][kSumTileBytes];
   const int64_t qi = blockIdx.x;
-  if (qi >= q || !(x2m[qi] < INFINITY)) return;  // uniform: listed for the exact kernel
-  __shared__ float qrow[16 * kMaxKS];
-  __shared__ uint32_t start[kMaxLists + 1];
-  const int nl = lay.nlists();
-  for (int j = threadIdx.x; j < ld; j += kRescoreThreads) qrow[j] = qs[qi * ld + j];
-  const int nr = l_hi - l_lo;  // lists l_lo .. l_hi - 1
-  if (threadIdx.x == 0) {
-    uint32_t acc = 0;
-    for (int i = 0; i < nr; ++i) {
-      start[i] = acc;
-      acc += min(cand_count[static_cast<size_t>(qi) * nl + l_lo + i],
-                 static_cast<uint32_t>(lay.cap(l_lo + i)));
+  const int tid = threadIdx.x, lane = tid & 63;
+  float b = INFINITY;
+  if (tid < k && seed_in) b = seed_in[qi * k + tid];
+  if (!(x2m[qi] < INFINITY)) {  // uniform: listed for the exact kernel
+    if (tid < k && seed_out) seed_out[qi * k + tid] = b;
+    return;
+  }
+  for (int j = tid; j < ld; j += kLevelThreads) qrow[j] = qs[qi * ld + j];
+  const bool pairs = l_lo >= lay.nrun;
+  const int nu = pairs ? (l_hi - l_lo) / 2 : l_hi - l_lo;  // at most kMaxSegs
+  if (tid < 64) {
+    uint32_t a = 0, o = 0;
+    if (lane < nu) {
+      const uint32_t* cc = cand_count + qi * lay.nlists() + l_lo;
+      const uint32_t cap = static_cast<uint32_t>(lay.cap(l_lo));
+      a = min(cc[pairs ? 2 * lane : lane], cap);
+      o = pairs ? min(cc[2 * lane + 1], cap) : 0u;
+      first[lane] = a;
     }
-    start[nr] = acc;
+    uint32_t inc = a + o;
+#pragma unroll
+    for (int w = 1; w < 64; w <<= 1) {
+      const uint32_t up = __shfl_up(inc, w);
+      if (lane >= w) inc += up;
+    }
+    if (lane < nu) start[lane] = inc - a - o;
+    if (lane == 63) start[nu] = inc;
   }
   __syncthreads();
-  const size_t qbase = static_cast<size_t>(qi) * lay.per_query();
-  for (uint32_t e = threadIdx.x; e < start[nr]; e += kRescoreThreads) {
-    int i = 0;
-    while (start[i + 1] <= e) ++i;
-    const size_t slot = qbase + lay.offset(l_lo + i) + (e - start[i]);
-    // the row read 16 values at a time (ld is a multiple of 16, rows are
-    // 64-byte aligned), the terms added in dimension order
-    const f32x4* r4 = reinterpret_cast<const f32x4*>(rows + static_cast<int64_t>(cand_idx[slot]) * ld);
-    double sum = 0.0;
-    for (int j = 0; j < ld; j += 16) {
-      f32x4 v[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = r4[j / 4 + i];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-          sum = sum + Term<float, kEuclid>::f(qrow[j + 4 * i + c], v[i][c], 2.0);
+  const int64_t base = qi * lay.per_query() + lay.offset(l_lo);
+  const int64_t cap = lay.cap(l_lo);
+  // the unit of candidate e: the last that starts at or below it
+  auto unit_of = [&](uint32_t e) {
+    int lo = 0, hi = nu;
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (start[mid] <= e)
+        lo = mid;
+      else
+        hi = mid;
     }
-    cand_S[slot] = sum;
+    return lo;
+  };
+  // the slot of place `at` of unit u
+  auto slot_of = [&](int u, uint32_t at) {
+    if (!pairs) return base + u * cap + at;
+    return at < first[u] ? base + 2 * u * cap + at : base + (2 * u + 1) * cap + (at - first[u]);
+  };
+  float kth = tid < 64 ? lane_value(b, k - 1) : 0.0f;
+  const uint32_t total = start[nu];
+  for (uint32_t e0 = 0; e0 < total;) {
+    // whole pairs while they fit (a longer one is left unmerged: its query
+    // goes to the serial kernel)
+    uint32_t m = min(total - e0, static_cast<uint32_t>(kLevelBatch));
+    if (pairs && e0 + m < total) {
+      const int u = unit_of(e0 + m);
+      if (start[u] > e0) m = start[u] - e0;
+    }
+    for (uint32_t e = tid; e < m; e += kLevelThreads) {
+      const int u = unit_of(e0 + e);
+      s_row[e] = cand_idx[slot_of(u, e0 + e - start[u])];
+    }
+    __syncthreads();
+    for (uint32_t b0 = tid & ~63u; b0 < m; b0 += kLevelThreads) {  // a wavefront's 64
+      const uint32_t e = min(b0 + lane, m - 1);
+      const uint32_t row = s_row[e];
+      const double s = wave_exact_sums<float, kEuclid>(qrow, rows, row, ld, tiles[tid >> 6]);
+      if (b0 + lane >= m) continue;
+      const int u = unit_of(e0 + e);
+      const uint32_t at = e0 + e - start[u], a = first[u], len = start[u + 1] - start[u];
+      uint32_t place = at;
+      if (pairs && a != 0u && a != len && start[u] >= e0 && start[u] + len <= e0 + m) {
+        // its own place plus the other half's entries before this row
+        const uint32_t ob = start[u] - e0 + (at < a ? a : 0u);
+        uint32_t lo = 0, up = at < a ? len - a : a;
+        while (lo < up) {
+          const uint32_t mid = (lo + up) >> 1;
+          if (s_row[ob + mid] < row)
+            lo = mid + 1;
+          else
+            up = mid;
+        }
+        place = (at < a ? at : at - a) + lo;
+      }
+      const int64_t slot = slot_of(u, place);
+      cand_idx[slot] = row;
+      cand_S[slot] = s;
+      s_v[e] = __double2float_ru(s);
+    }
+    __syncthreads();
+    if (seed_out && tid < 64) {
+      for (uint32_t c0 = 0; c0 < m; c0 += 64) {
+        const float v = c0 + lane < m ? s_v[c0 + lane] : INFINITY;
+        uint64_t w = __ballot(v < kth);
+        while (w) {
+          const float x = lane_value(v, __builtin_ctzll(w));
+          const float prev = __shfl_up(b, 1);
+          if (lane < k && x < b) b = (lane > 0 && x < prev) ? prev : x;
+          kth = lane_value(b, k - 1);
+          w &= w - 1;
+          w &= __ballot(v < kth);
+        }
+      }
+    }
+    __syncthreads();
+    e0 += m;
   }
+  if (tid < k && seed_out) seed_out[qi * k + tid] = b;
 }
 
-// Pass 2b: replay of the heap rule over the candidates in row order, one
-// wavefront per query.  Entries are taken 64 at a time (lane = entry); the
-// lanes whose distance is below the heap's largest (the reference's strict
-// <) enter one after another, in row order, by a sift-down of the heap
-// held across the lanes, and the rest are tested again against the new top.  A
-// fixed launch's list pair is merged by row 64 entries at a time: an entry's
-// place is its lane plus the count of smaller rows in the other list's
-// window, and the places below 64 are the next 64 rows of the merge.
-// Queries whose lists overflowed go to the serial exact kernel's list.
-__global__ __launch_bounds__(64 * kWavesPerBlock) void mixed_replay_kernel(
+// The replay, one wavefront per query (the heap lives across its lanes): the
+// candidates of all lists, in row order by now, 64 at a time across the
+// lists; the next 64 are requested before the current ones go through the
+// heap.  Queries whose lists overflowed, or a pair of whose lists could not
+// be merged, go to the serial exact kernel's list.
+__global__ __launch_bounds__(64 * kReplayWaves) void mixed_replay_kernel(
     int64_t q, int k, ListLayout lay, const uint32_t* __restrict__ cand_idx,
     const double* __restrict__ cand_S, const uint32_t* __restrict__ cand_count,
     const float* __restrict__ x2m, int64_t* __restrict__ out_idx, double* __restrict__ out_dist,
     uint32_t* __restrict__ out_count, uint32_t* __restrict__ list, uint32_t* __restrict__ list_n,
     unsigned long long* __restrict__ counters) {
-  __shared__ uint32_t s_win[kWavesPerBlock][2][64];
-  __shared__ uint32_t s_mrow[kWavesPerBlock][64];
-  __shared__ double s_mS[kWavesPerBlock][64];
+  extern __shared__ __align__(16) uint32_t replay_smem[];  // per wavefront: nlists + 1 starts
   const int lane = threadIdx.x & 63;
   const int w = threadIdx.x >> 6;
-  const int64_t qi = static_cast<int64_t>(blockIdx.x) * kWavesPerBlock + w;
+  const int64_t qi = static_cast<int64_t>(blockIdx.x) * kReplayWaves + w;
   if (qi >= q) return;                     // the whole wave
   if (!(x2m[qi] < INFINITY)) return;       // listed for the exact kernel already
   const int nl = lay.nlists();
-  const uint32_t* cc = cand_count + static_cast<size_t>(qi) * nl;
+  uint32_t* start = replay_smem + w * (nl + 1);
+  const uint32_t* cc = cand_count + qi * nl;
   bool over = false;
-  for (int l = lane; l < nl; l += 64) over = over || cc[l] > static_cast<uint32_t>(lay.cap(l));
-  if (__ballot(over) != 0) {
-    if (lane == 0) {
-      const uint32_t slot = atomicAdd(list_n, 1u);
-      list[slot] = static_cast<uint32_t>(qi);
+  uint32_t total = 0;
+  for (int l0 = 0; l0 < nl; l0 += 64) {
+    const int l = l0 + lane;
+    const uint32_t c = l < nl ? cc[l] : 0u;
+    if (l < nl) {
+      over = over || c > static_cast<uint32_t>(lay.cap(l));
+      if (l >= lay.nrun) {
+        const uint32_t o = cc[lay.nrun + ((l - lay.nrun) ^ 1)];
+        over = over || (c != 0u && o != 0u && c + o > static_cast<uint32_t>(kLevelBatch));
+      }
     }
+    uint32_t inc = c;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t up = __shfl_up(inc, o);
+      if (lane >= o) inc += up;
+    }
+    if (l < nl) start[l] = total + inc - c;
+    total += __shfl(inc, 63);
+  }
+  if (__ballot(over) != 0) {
+    if (lane == 0) list[atomicAdd(list_n, 1u)] = static_cast<uint32_t>(qi);
     return;
   }
+  if (lane == 0) start[nl] = total;
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  const int64_t qbase = qi * lay.per_query();
+  uint32_t row = 0, row_n = 0;
+  double s = 0.0, s_n = 0.0;
+  auto load = [&](uint32_t e, uint32_t& r, double& v) {
+    if (e >= total) return;
+    int lo = 0, hi = nl;  // the last list that starts at or below e
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (start[mid] <= e)
+        lo = mid;
+      else
+        hi = mid;
+    }
+    const int64_t slot = qbase + lay.offset(lo) + (e - start[lo]);
+    r = cand_idx[slot];
+    v = cand_S[slot];
+  };
+  load(lane, row, s);
   // the heap in lanes 0 .. k-1 (the reference seeds it with k x {inf, None})
-  double hd = INFINITY;
+  double hd = INFINITY, top = INFINITY;
   uint32_t hi = 0xffffffffu;
-  double top = INFINITY;
-  // entries of one chunk, in row order over the lanes (valid lanes first)
-  auto consume = [&](double S, uint32_t row, bool valid) {
-    const double d = __builtin_sqrt(S);
+  for (uint32_t e0 = 0; e0 < total; e0 += 64) {
+    load(e0 + 64 + lane, row_n, s_n);
+    const bool valid = e0 + lane < total;
+    const double d = __builtin_sqrt(s);
     uint64_t m = __ballot(valid && d < top);
     while (m) {
       const int src = __builtin_ctzll(m);
-      const double dl = lane_value(d, src);
-      const uint32_t rl = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(row), src));
-      lane_heap_push_root(hd, hi, lane, k, dl, rl);
+      lane_heap_push_root(hd, hi, lane, k, lane_value(d, src), lane_value(row, src));
       top = lane_value(hd, 0);
       m &= m - 1;
       m &= __ballot(valid && d < top);
     }
-  };
-  const size_t qbase = static_cast<size_t>(qi) * lay.per_query();
-  unsigned long long seen = 0;
-  for (int l = 0; l < lay.nrun; ++l) {
-    const size_t base = qbase + lay.offset(l);
-    const uint32_t n = cc[l];
-    seen += n;
-    for (uint32_t c0 = 0; c0 < n; c0 += 64) {
-      const bool valid = c0 + lane < n;
-      const double S = valid ? cand_S[base + c0 + lane] : 0.0;
-      const uint32_t row = valid ? cand_idx[base + c0 + lane] : 0u;
-      consume(S, row, valid);
-    }
+    row = row_n;
+    s = s_n;
   }
-  uint32_t* winA = s_win[w][0];
-  uint32_t* winB = s_win[w][1];
-  uint32_t* mrow = s_mrow[w];
-  double* mS = s_mS[w];
-  // count of entries below v in a window of 64 ascending rows (absent
-  // entries are 0xffffffff)
-  auto rank_in = [&](const uint32_t* win, uint32_t v) {
-    int lo = 0;
-#pragma unroll
-    for (int step = 64; step > 0; step >>= 1)
-      if (lo + step <= 64 && win[lo + step - 1] < v) lo += step;
-    return lo;
-  };
-  for (int l = lay.nrun; l < nl; l += 2) {
-    const size_t bA = qbase + lay.offset(l), bB = qbase + lay.offset(l + 1);
-    const uint32_t nA = cc[l], nB = cc[l + 1];
-    seen += nA + nB;
-    uint32_t ia = 0, ib = 0;
-    while (ia < nA || ib < nB) {
-      const bool okA = ia + lane < nA, okB = ib + lane < nB;
-      const uint32_t ra = okA ? cand_idx[bA + ia + lane] : 0xffffffffu;
-      const uint32_t rb = okB ? cand_idx[bB + ib + lane] : 0xffffffffu;
-      const double Sa = okA ? cand_S[bA + ia + lane] : 0.0;
-      const double Sb = okB ? cand_S[bB + ib + lane] : 0.0;
-      winA[lane] = ra;
-      winB[lane] = rb;
-      wave_sync();
-      const int pa = lane + rank_in(winB, ra);
-      const int pb = lane + rank_in(winA, rb);
-      const bool takeA = okA && pa < 64, takeB = okB && pb < 64;
-      if (takeA) {
-        mrow[pa] = ra;
-        mS[pa] = Sa;
-      }
-      if (takeB) {
-        mrow[pb] = rb;
-        mS[pb] = Sb;
-      }
-      const uint32_t cA = static_cast<uint32_t>(__popcll(__ballot(takeA)));
-      const uint32_t cB = static_cast<uint32_t>(__popcll(__ballot(takeB)));
-      wave_sync();
-      const bool valid = static_cast<uint32_t>(lane) < cA + cB;
-      const double S = valid ? mS[lane] : 0.0;
-      const uint32_t row = valid ? mrow[lane] : 0u;
-      wave_sync();  // the window and merge slots are rewritten next round
-      consume(S, row, valid);
-      ia += cA;
-      ib += cB;
-    }
-  }
-  if (lane == 0) {
-    atomicAdd(&counters[0], seen);
-    atomicAdd(&counters[1], seen);
-  }
+  // (only when asked for: one address for all queries)
+  if (counters && lane == 0) atomicAdd(counters, static_cast<unsigned long long>(total));
   lane_heap_store(hd, hi, lane, k, out_idx + qi * k, out_dist + qi * k, out_count + qi);
 }
 
@@ -1287,20 +1298,14 @@ int knn_mixed_device(const sc_index* cix, const void* d_queries, size_t q_, size
   sa.cand_count = ccnt.as<uint32_t>();
   float* seed_cur = seedA.as<float>();
   float* seed_next = seedB.as<float>();
-  // exact distances of the candidates in lists [l_lo, l_hi)
-  auto rescore = [&](int l_lo, int l_hi) -> int {
-    hipLaunchKernelGGL(mixed_rescore_kernel, dim3(static_cast<unsigned>(q)), dim3(kRescoreThreads),
-                       0, stream, static_cast<const float*>(ix->rows), qf, ld, q, lay, l_lo, l_hi,
-                       cidx.as<uint32_t>(), ccnt.as<uint32_t>(), x2.as<float>(), cS.as<double>());
-    SC_HIP(hipGetLastError());
-    return SC_OK;
-  };
-  // the next seed from the current one (null: none yet) and lists [l0, l0 + nl)
-  auto select = [&](const float* in, int l0, int nl) -> int {
-    hipLaunchKernelGGL(select_seed_kernel,
-                       dim3(static_cast<unsigned>((q + kWavesPerBlock - 1) / kWavesPerBlock)),
-                       dim3(64 * kWavesPerBlock), 0, stream, in, cS.as<double>(), ccnt.as<uint32_t>(), lay, l0, nl, q, k,
-                       seed_next);
+  // the end of a level whose candidates are lists [l_lo, l_hi): their exact
+  // distances and order, and (not after the last) the next seed (in: the
+  // current one, null: none yet)
+  auto level_end = [&](const float* in, int l_lo, int l_hi, bool last) -> int {
+    hipLaunchKernelGGL(mixed_level_kernel, dim3(static_cast<unsigned>(q)), dim3(kLevelThreads), 0, stream,
+                       static_cast<const float*>(ix->rows), qf, ld, lay, l_lo, l_hi,
+                       cidx.as<uint32_t>(), ccnt.as<uint32_t>(), x2.as<float>(), cS.as<double>(), k,
+                       last ? nullptr : in, last ? nullptr : seed_next);
     SC_HIP(hipGetLastError());
     std::swap(seed_cur, seed_next);
     return SC_OK;
@@ -1315,8 +1320,7 @@ int knn_mixed_device(const sc_index* cix, const void* d_queries, size_t q_, size
     la.lbase = 0;
     if (int rc = launch_scan(ld / 16, 0, la, stream)) return rc;
     if (nfix_levels > 0) {
-      if (int rc = rescore(0, nseg)) return rc;
-      if (int rc = select(nullptr, 0, nseg)) return rc;
+      if (int rc = level_end(nullptr, 0, nseg, false)) return rc;
     }
     for (int i = 1; i < nfix_levels; ++i) {
       ScanArgs fa = sa;
@@ -1326,8 +1330,7 @@ int knn_mixed_device(const sc_index* cix, const void* d_queries, size_t q_, size
       fa.lbase = nseg + 2 * nseg * (i - 1);
       fa.seed = seed_cur;
       if (int rc = launch_scan(ld / 16, 2, fa, stream)) return rc;
-      if (int rc = rescore(fa.lbase, fa.lbase + 2 * nseg)) return rc;
-      if (int rc = select(seed_cur, fa.lbase, 2 * nseg)) return rc;
+      if (int rc = level_end(seed_cur, fa.lbase, fa.lbase + 2 * nseg, false)) return rc;
     }
   }
   int l_last = 0;  // first list of the last scan
@@ -1345,25 +1348,25 @@ int knn_mixed_device(const sc_index* cix, const void* d_queries, size_t q_, size
   }
   {
     ProfScope ps("knn_mixed_rescore", stream);
-    if (int rc = rescore(l_last, lay.nlists())) return rc;
+    if (int rc = level_end(nullptr, l_last, lay.nlists(), true)) return rc;
     hipLaunchKernelGGL(mixed_replay_kernel,
-                       dim3(static_cast<unsigned>((q + kWavesPerBlock - 1) / kWavesPerBlock)),
-                       dim3(64 * kWavesPerBlock), 0, stream, q, k, lay, cidx.as<uint32_t>(),
-                       cS.as<double>(), ccnt.as<uint32_t>(), x2.as<float>(), d_idx, d_dist, d_count,
-                       lst.as<uint32_t>(), list_n, counters);
+                       dim3(static_cast<unsigned>((q + kReplayWaves - 1) / kReplayWaves)),
+                       dim3(64 * kReplayWaves), sizeof(uint32_t) * kReplayWaves * (lay.nlists() + 1),
+                       stream, q, k, lay, cidx.as<uint32_t>(), cS.as<double>(), ccnt.as<uint32_t>(),
+                       x2.as<float>(), d_idx, d_dist, d_count, lst.as<uint32_t>(), list_n,
+                       stats ? counters : nullptr);
     SC_HIP(hipGetLastError());
   }
   if (int rc = launch_serial_exact(ix, qf, k, lst.as<uint32_t>(), list_n, d_idx, d_dist,
                                        d_count, stream))
     return rc;
   if (stats) {
-    uint64_t h[2] = {0, 0};
-    uint32_t ln = 0;
-    SC_HIP(hipMemcpyAsync(&ln, list_n, 4, hipMemcpyDeviceToHost, stream));
-    SC_HIP(hipMemcpyAsync(h, counters, 16, hipMemcpyDeviceToHost, stream));
+    uint64_t h[2] = {0, 0};  // listed queries, candidates
+    SC_HIP(hipMemcpyAsync(h, flags.p, 16, hipMemcpyDeviceToHost, stream));
     SC_HIP(hipStreamSynchronize(stream));
+    const uint32_t ln = static_cast<uint32_t>(h[0]);
     stats->queries += static_cast<uint64_t>(q);
-    stats->candidates += h[0];
+    stats->candidates += h[1];
     stats->shortlist_rescored += h[1];
     stats->overflow_queries += ln;
     stats->uncertified += ln;
