@@ -120,17 +120,17 @@ struct MLane {
 };
 typedef f64x4 MAcc[8][2];
 
-// Sweeps tiles tb .. te - 1 (row = row0 + 128 tile) against queries
-// q0 .. q0 + 127; epi(t, acc, slot) runs at each tile's end, without a
+// Sweeps tiles at(tb) .. at(te - 1) (row = row0 + 128 tile) against queries
+// q0 .. q0 + 127; epi(t, acc, slot) runs at the end of tile at(t), without a
 // barrier of its own (sm.y2[slot] holds the tile's y2m).  Out-of-range rows and
 // queries are read clamped: y2m carries +inf past the last row.  SWAP: the
 // accumulators hold (query, row) transposed -- acc[i][j][v] of a lane is row
 // 16 i + lr, query 32 wave + 16 j + 4 v + lg -- and start at zero.
-template <typename T, bool SWAP, typename Epi>
+template <typename T, bool SWAP, typename Epi, typename At>
 __device__ __forceinline__ void mfma64_sweep(MSmem& sm, const T* __restrict__ rows, int64_t n,
                                              int ld, int d, const double* __restrict__ y2m,
                                              const T* __restrict__ queries, int64_t q, int64_t q0,
-                                             int64_t row0, int64_t tb, int64_t te, Epi epi) {
+                                             int64_t row0, int64_t tb, int64_t te, Epi epi, At at) {
   constexpr int PV = 16 / sizeof(T);            // values per 16-byte piece
   constexpr int PR = kMD / PV;                  // pieces per row of a chunk
   constexpr int NP = kMR * PR / kMT;            // pieces per thread (rows and queries each)
@@ -157,7 +157,7 @@ __device__ __forceinline__ void mfma64_sweep(MSmem& sm, const T* __restrict__ ro
       vq[p] = *reinterpret_cast<const Piece*>(cbase + min(pr + p * (kMT / PR), qleft) * ld + pc);
   };
   auto gload = [&]() {
-    const int64_t t0 = row0 + lt * kMR;
+    const int64_t t0 = row0 + at(lt) * kMR;
     const T* rbase = rows + t0 * ld + lk * kMD;
     const int left = static_cast<int>(min<int64_t>(kMR, n - t0)) - 1;
 #pragma unroll
@@ -246,6 +246,16 @@ __device__ __forceinline__ void mfma64_sweep(MSmem& sm, const T* __restrict__ ro
       ++t;
     }
   }
+}
+
+// The tiles tb .. te - 1 themselves.
+template <typename T, bool SWAP, typename Epi>
+__device__ __forceinline__ void mfma64_sweep(MSmem& sm, const T* __restrict__ rows, int64_t n,
+                                             int ld, int d, const double* __restrict__ y2m,
+                                             const T* __restrict__ queries, int64_t q, int64_t q0,
+                                             int64_t row0, int64_t tb, int64_t te, Epi epi) {
+  mfma64_sweep<T, SWAP>(sm, rows, n, ld, d, y2m, queries, q, q0, row0, tb, te, epi,
+                        [](int64_t t) { return t; });
 }
 
 // Calls f(i, j, v, row, hit, mask) for every accumulator register of the
