@@ -210,18 +210,36 @@ class DenseMatrix {
   static DenseMatrix from_row_major(size_t nrows, size_t ncols, const T* data) {
     return DenseMatrix(nrows, ncols, std::vector<T>(data, data + nrows * ncols), false);
   }
+  // The same without a copy: the caller keeps `data` alive and unchanged as
+  // long as this matrix, and any copy of it, is used.
+  static DenseMatrix view_row_major(size_t nrows, size_t ncols, const T* data) {
+    DenseMatrix m;
+    m.nrows_ = nrows;
+    m.ncols_ = ncols;
+    m.view_ = data;
+    m.column_major_ = false;
+    return m;
+  }
   std::pair<size_t, size_t> shape() const { return {nrows_, ncols_}; }
   // matrix.rs:367-380
   const T& get(size_t r, size_t c) const {
-    return column_major_ ? values_[c * nrows_ + r] : values_[r * ncols_ + c];
+    return column_major_ ? values_[c * nrows_ + r] : row_values()[r * ncols_ + c];
   }
   std::vector<T> get_row(size_t r) const {
     std::vector<T> row(ncols_);
     for (size_t c = 0; c < ncols_; ++c) row[c] = get(r, c);
     return row;
   }
+  // The rows in row-major order: this matrix's own values where they lie so,
+  // else a copy in `scratch` (100,000 x 16 f64 rows copied twice on the way
+  // to the device took about 1 ms of a 6.3 ms KMeans::fit).
+  const T* row_major_data(std::vector<T>& scratch) const {
+    if (!column_major_) return row_values();
+    scratch = row_major();
+    return scratch.data();
+  }
   std::vector<T> row_major() const {
-    if (!column_major_) return values_;
+    if (!column_major_) return std::vector<T>(row_values(), row_values() + nrows_ * ncols_);
     std::vector<T> out(nrows_ * ncols_);
     for (size_t r = 0; r < nrows_; ++r)
       for (size_t c = 0; c < ncols_; ++c) out[r * ncols_ + c] = values_[c * nrows_ + r];
@@ -229,8 +247,11 @@ class DenseMatrix {
   }
 
  private:
+  const T* row_values() const { return view_ ? view_ : values_.data(); }
+
   size_t nrows_ = 0, ncols_ = 0;
   std::vector<T> values_;
+  const T* view_ = nullptr;  // view_row_major's data
   bool column_major_ = true;
 };
 
@@ -338,10 +359,19 @@ class LinearKNNSearch {
     return LinearKNNSearch(std::move(data), std::move(distance));
   }
   LinearKNNSearch(std::vector<std::vector<T>> data, D distance)
-      : data_(std::move(data)), distance_(std::move(distance)), dev_(std::make_shared<Device>()) {
-    dim_ = data_.empty() ? 0 : data_[0].size();
-    for (const auto& r : data_)
+      : distance_(std::move(distance)), store_(std::make_shared<Store>()) {
+    n_ = data.size();
+    dim_ = data.empty() ? 0 : data[0].size();
+    for (const auto& r : data)
       if (r.size() != dim_) throw Panic("Input vector sizes are different.");
+    store_->rows = std::move(data);
+    store_->has_rows = true;
+  }
+  // n rows of dim values in one row-major block.  find()'s row vectors are
+  // made when they are first asked for, which the estimators never do.
+  LinearKNNSearch(std::vector<T> packed, size_t n, size_t dim, D distance)
+      : distance_(std::move(distance)), store_(std::make_shared<Store>()), n_(n), dim_(n ? dim : 0) {
+    store_->packed = std::move(packed);
   }
 
   using Neighbour = std::tuple<size_t, double, const std::vector<T>*>;
@@ -354,27 +384,44 @@ class LinearKNNSearch {
   // The loop of KNNClassifier::predict batched into one device call.
   std::vector<std::vector<Neighbour>> find_batch(const std::vector<std::vector<T>>& from, size_t k,
                                                  SearchMode mode = SearchMode::PlainFp64) const {
-    const auto dm = distance_.device_metric();
-    if (!dm) throw Failed::because(FailedError::FindFailed, "metric has no device kernel");
+    if (!distance_.device_metric())
+      throw Failed::because(FailedError::FindFailed, "metric has no device kernel");
     std::vector<T> q(from.size() * dim_);
     for (size_t i = 0; i < from.size(); ++i) {
       if (from[i].size() != dim_) throw Panic("Input vector sizes are different.");
       std::copy(from[i].begin(), from[i].end(), q.begin() + i * dim_);
     }
-    std::vector<int64_t> idx(from.size() * std::max<size_t>(k, 1));
-    std::vector<double> dist(idx.size());
-    std::vector<uint32_t> cnt(std::max<size_t>(from.size(), 1));
-    detail::check(sc_knn_search(index(), q.data(), from.size(), k, dm->metric, dm->p,
-                                static_cast<sc_mode>(mode), idx.data(), dist.data(), cnt.data()));
+    const Found f = find_packed(q.data(), from.size(), dim_, k, mode);
+    const auto& data = rows();
     std::vector<std::vector<Neighbour>> out(from.size());
     for (size_t i = 0; i < from.size(); ++i) {
-      out[i].reserve(cnt[i]);
-      for (size_t j = 0; j < cnt[i]; ++j) {
-        const size_t r = static_cast<size_t>(idx[i * k + j]);
-        out[i].emplace_back(r, dist[i * k + j], &data_[r]);
+      out[i].reserve(f.count[i]);
+      for (size_t j = 0; j < f.count[i]; ++j) {
+        const size_t r = static_cast<size_t>(f.idx[i * k + j]);
+        out[i].emplace_back(r, f.dist[i * k + j], &data[r]);
       }
     }
     return out;
+  }
+
+  // The same for nq row-major queries, as arrays: query i's neighbours are
+  // entries i k .. i k + count[i] - 1.
+  struct Found {
+    std::vector<int64_t> idx;
+    std::vector<double> dist;
+    std::vector<uint32_t> count;
+  };
+  Found find_packed(const T* q, size_t nq, size_t ncols, size_t k, SearchMode mode) const {
+    const auto dm = distance_.device_metric();
+    if (!dm) throw Failed::because(FailedError::FindFailed, "metric has no device kernel");
+    if (nq > 0 && ncols != dim_) throw Panic("Input vector sizes are different.");
+    Found f;
+    f.idx.resize(nq * std::max<size_t>(k, 1));
+    f.dist.resize(f.idx.size());
+    f.count.resize(std::max<size_t>(nq, 1));
+    detail::check(sc_knn_search(index(), q, nq, k, dm->metric, dm->p, static_cast<sc_mode>(mode),
+                                f.idx.data(), f.dist.data(), f.count.data()));
+    return f;
   }
 
   // linear_search.rs:89-108
@@ -390,29 +437,35 @@ class LinearKNNSearch {
     std::vector<double> dist(idx.size());
     sc_radius_result_copy(r, off.data(), idx.data(), dist.data());
     sc_radius_result_free(r);
+    const auto& data = rows();
     std::vector<Neighbour> out;
     for (size_t j = 0; j < total; ++j)
-      out.emplace_back(static_cast<size_t>(idx[j]), dist[j], &data_[static_cast<size_t>(idx[j])]);
+      out.emplace_back(static_cast<size_t>(idx[j]), dist[j], &data[static_cast<size_t>(idx[j])]);
     return out;
   }
 
-  size_t len() const { return data_.size(); }
+  size_t len() const { return n_; }
   // The device-resident rows (uploaded on first use).
   const sc_index* index() const {
-    std::lock_guard<std::mutex> lk(dev_->mu);
-    if (!dev_->ix) {
-      std::vector<T> packed(data_.size() * dim_);
-      for (size_t i = 0; i < data_.size(); ++i)
-        std::copy(data_[i].begin(), data_[i].end(), packed.begin() + i * dim_);
+    std::lock_guard<std::mutex> lk(store_->mu);
+    if (!store_->ix) {
+      std::vector<T> scratch;
+      const T* rows = store_->packed.data();
+      if (store_->packed.size() != n_ * dim_) {
+        scratch.resize(n_ * dim_);
+        for (size_t i = 0; i < n_; ++i)
+          std::copy(store_->rows[i].begin(), store_->rows[i].end(), scratch.begin() + i * dim_);
+        rows = scratch.data();
+      }
       sc_index* ix = nullptr;
-      detail::check(sc_index_create(packed.data(), detail::dtype_of<T>(), data_.size(), dim_, &ix));
-      dev_->ix = ix;
+      detail::check(sc_index_create(rows, detail::dtype_of<T>(), n_, dim_, &ix));
+      store_->ix = ix;
     }
-    return dev_->ix;
+    return store_->ix;
   }
   bool on_device() const {
-    std::lock_guard<std::mutex> lk(dev_->mu);
-    return dev_->ix != nullptr;
+    std::lock_guard<std::mutex> lk(store_->mu);
+    return store_->ix != nullptr;
   }
 
   // The rows and the distance (serde's view of LinearKNNSearch,
@@ -422,10 +475,10 @@ class LinearKNNSearch {
     w.u8(static_cast<uint8_t>(detail::dtype_of<T>()));
     w.u8(static_cast<uint8_t>(dm ? dm->metric : SC_EUCLIDIAN));
     w.u16(dm ? dm->p : 2);
-    w.u64(data_.size());
+    w.u64(n_);
     w.u64(dim_);
-    for (const auto& r : data_)
-      for (const T& v : r) w.num<T>(v);
+    for (size_t i = 0; i < n_; ++i)
+      for (size_t j = 0; j < dim_; ++j) w.num<T>(row(i)[j]);
   }
   static LinearKNNSearch load(detail::ByteReader& r) {
     if (r.u8() != static_cast<uint8_t>(detail::dtype_of<T>()))
@@ -443,22 +496,46 @@ class LinearKNNSearch {
   }
   bool operator==(const LinearKNNSearch& o) const {
     const auto a = distance_.device_metric(), b = o.distance_.device_metric();
-    return data_ == o.data_ && a.has_value() == b.has_value() &&
+    if (n_ != o.n_ || dim_ != o.dim_) return false;
+    for (size_t i = 0; i < n_; ++i)
+      if (!std::equal(row(i), row(i) + dim_, o.row(i))) return false;
+    return a.has_value() == b.has_value() &&
            (!a || (a->metric == b->metric && a->p == b->p));
   }
 
  private:
-  struct Device {
+  // The rows (as one block, as vectors, or both) and their device copy,
+  // shared by the copies of a search.
+  struct Store {
     std::mutex mu;
     sc_index* ix = nullptr;
-    ~Device() {
+    std::vector<T> packed;
+    std::vector<std::vector<T>> rows;
+    bool has_rows = false;
+    ~Store() {
       if (ix) sc_index_destroy(ix);
     }
   };
-  std::vector<std::vector<T>> data_;
+  const T* row(size_t i) const {
+    // (the form a search was made with never changes)
+    return store_->packed.size() == n_ * dim_ ? store_->packed.data() + i * dim_ : store_->rows[i].data();
+  }
+  const std::vector<std::vector<T>>& rows() const {
+    std::lock_guard<std::mutex> lk(store_->mu);
+    if (!store_->has_rows) {
+      store_->rows.reserve(n_);
+      for (size_t i = 0; i < n_; ++i) {
+        const T* r = store_->packed.data() + i * dim_;
+        store_->rows.emplace_back(r, r + dim_);
+      }
+      store_->has_rows = true;
+    }
+    return store_->rows;
+  }
+
   D distance_;
-  std::shared_ptr<Device> dev_;
-  size_t dim_ = 0;
+  std::shared_ptr<Store> store_;
+  size_t n_ = 0, dim_ = 0;
 };
 
 // ---------------------------------------------------------------- neighbors
@@ -501,12 +578,44 @@ struct KNNClassifierParameters {
   KNNClassifierParameters with_mode(SearchMode m) const { auto p = *this; p.mode = m; return p; }
 };
 
+namespace detail {
+// The distinct values of y, ascending, and each value's place among them
+// (arrays.rs:223-231 unique; position map knn_classifier.rs:229-235).  Up to
+// kFewClasses values are kept sorted while y is read once (10,000 labels of
+// 10 classes: 0.03 ms; sorting a copy of y took 0.3).
+template <typename TY>
+void classes_of(const std::vector<TY>& y, std::vector<TY>& classes, std::vector<size_t>& yi) {
+  constexpr size_t kFewClasses = 64;
+  classes.clear();
+  bool few = true;
+  for (const TY& v : y) {
+    const auto at = std::lower_bound(classes.begin(), classes.end(), v);
+    if (at != classes.end() && *at == v) continue;
+    if (classes.size() == kFewClasses || !(v == v)) {
+      few = false;
+      break;
+    }
+    classes.insert(at, v);
+  }
+  if (!few) {
+    classes.assign(y.begin(), y.end());
+    std::sort(classes.begin(), classes.end());
+    classes.erase(std::unique(classes.begin(), classes.end()), classes.end());
+  }
+  yi.resize(y.size());
+  for (size_t i = 0; i < y.size(); ++i) {
+    auto at = std::lower_bound(classes.begin(), classes.end(), y[i]);
+    if (at == classes.end() || !(*at == y[i])) at = std::find(classes.begin(), classes.end(), y[i]);
+    yi[i] = static_cast<size_t>(at - classes.begin());
+  }
+}
+}  // namespace detail
+
+// A device search over the rows of x.
 template <typename T, typename D>
-std::vector<std::vector<T>> rows_of(const DenseMatrix<T>& x) {
+std::shared_ptr<LinearKNNSearch<T, D>> search_of(const DenseMatrix<T>& x, const D& distance) {
   const auto sh = x.shape();
-  std::vector<std::vector<T>> rows(sh.first);
-  for (size_t i = 0; i < sh.first; ++i) rows[i] = x.get_row(i);
-  return rows;
+  return std::make_shared<LinearKNNSearch<T, D>>(x.row_major(), sh.first, sh.second, distance);
 }
 
 // KNNClassifier (knn_classifier.rs:74-299)
@@ -518,14 +627,9 @@ class KNNClassifier {
                            const KNNClassifierParameters<TX, D>& parameters) {
     const size_t y_n = y.size();
     const size_t x_n = x.shape().first;
-    auto data = rows_of<TX, D>(x);
-    // arrays.rs:223-231 unique (sort + dedup); position map knn_classifier.rs:229-235
-    std::vector<TY> classes(y.begin(), y.end());
-    std::sort(classes.begin(), classes.end());
-    classes.erase(std::unique(classes.begin(), classes.end()), classes.end());
-    std::vector<size_t> yi(y_n);
-    for (size_t i = 0; i < y_n; ++i)
-      yi[i] = static_cast<size_t>(std::find(classes.begin(), classes.end(), y[i]) - classes.begin());
+    std::vector<TY> classes;
+    std::vector<size_t> yi;
+    detail::classes_of(y, classes, yi);
     if (x_n != y_n)
       throw Failed::fit("Size of x should equal size of y; |x|=[" + std::to_string(x_n) +
                         "], |y|=[" + std::to_string(y_n) + "]");
@@ -536,16 +640,21 @@ class KNNClassifier {
     m.k_ = parameters.k;
     m.weight_ = parameters.weight;
     m.mode_ = parameters.mode;
-    m.search_ = std::make_shared<LinearKNNSearch<TX, D>>(std::move(data), parameters.distance);
+    m.search_ = search_of(x, parameters.distance);
     return m;
   }
 
   // knn_classifier.rs:265-277, all rows in one device call
   std::vector<TY> predict(const DenseMatrix<TX>& x) const {
-    const auto rows = rows_of<TX, D>(x);
-    const auto found = search_->find_batch(rows, k_, mode_);
-    std::vector<TY> result(rows.size());
-    for (size_t i = 0; i < rows.size(); ++i) result[i] = classes_[predict_for_row(found[i])];
+    const auto sh = x.shape();
+    std::vector<TX> scratch;
+    const auto f = search_->find_packed(x.row_major_data(scratch), sh.first, sh.second, k_, mode_);
+    std::vector<TY> result(sh.first);
+    std::vector<double> d, c(classes_.size(), 0.0);
+    for (size_t i = 0; i < sh.first; ++i) {
+      d.assign(f.dist.begin() + i * k_, f.dist.begin() + i * k_ + f.count[i]);
+      result[i] = classes_[predict_for_row(f.idx.data() + i * k_, d, c)];
+    }
     return result;
   }
 
@@ -587,24 +696,23 @@ class KNNClassifier {
   }
 
  private:
-  // knn_classifier.rs:279-299
-  size_t predict_for_row(const std::vector<typename LinearKNNSearch<TX, D>::Neighbour>& sr) const {
-    std::vector<double> d(sr.size());
-    for (size_t i = 0; i < sr.size(); ++i) d[i] = std::get<1>(sr[i]);
+  // knn_classifier.rs:279-299; d: the neighbours' distances, c: zeros (and
+  // again on return)
+  size_t predict_for_row(const int64_t* idx, const std::vector<double>& d, std::vector<double>& c) const {
     const auto weights = calc_weights(weight_, d);
     double w_sum = 0.0;
     for (double w : weights) w_sum += w;
-    std::vector<double> c(classes_.size(), 0.0);
     double max_c = 0.0;
     size_t max_i = 0;
-    for (size_t i = 0; i < sr.size(); ++i) {
-      const size_t cls = y_[std::get<0>(sr[i])];
+    for (size_t i = 0; i < d.size(); ++i) {
+      const size_t cls = y_[static_cast<size_t>(idx[i])];
       c[cls] += weights[i] / w_sum;
       if (c[cls] > max_c) {
         max_c = c[cls];
         max_i = cls;
       }
     }
+    for (size_t i = 0; i < d.size(); ++i) c[y_[static_cast<size_t>(idx[i])]] = 0.0;
     return max_i;
   }
 
@@ -629,7 +737,6 @@ class KNNRegressor {
                           const KNNRegressorParameters<TX, D>& parameters) {
     const size_t y_n = y.size();
     const size_t x_n = x.shape().first;
-    auto data = rows_of<TX, D>(x);
     if (x_n != y_n)
       throw Failed::fit("Size of x should equal size of y; |x|=[" + std::to_string(x_n) +
                         "], |y|=[" + std::to_string(y_n) + "]");
@@ -639,25 +746,25 @@ class KNNRegressor {
     m.k_ = parameters.k;
     m.weight_ = parameters.weight;
     m.mode_ = parameters.mode;
-    m.search_ = std::make_shared<LinearKNNSearch<TX, D>>(std::move(data), parameters.distance);
+    m.search_ = search_of(x, parameters.distance);
     return m;
   }
 
   std::vector<TY> predict(const DenseMatrix<TX>& x) const {
-    const auto rows = rows_of<TX, D>(x);
-    const auto found = search_->find_batch(rows, k_, mode_);
-    std::vector<TY> result(rows.size());
-    for (size_t i = 0; i < rows.size(); ++i) {
+    const auto sh = x.shape();
+    std::vector<TX> scratch;
+    const auto f = search_->find_packed(x.row_major_data(scratch), sh.first, sh.second, k_, mode_);
+    std::vector<TY> result(sh.first);
+    std::vector<double> d;
+    for (size_t i = 0; i < sh.first; ++i) {
       // knn_regressor.rs:268-281
-      const auto& sr = found[i];
-      std::vector<double> d(sr.size());
-      for (size_t j = 0; j < sr.size(); ++j) d[j] = std::get<1>(sr[j]);
+      d.assign(f.dist.begin() + i * k_, f.dist.begin() + i * k_ + f.count[i]);
       const auto weights = calc_weights(weight_, d);
       double w_sum = 0.0;
       for (double w : weights) w_sum += w;
       TY acc = TY(0);
-      for (size_t j = 0; j < sr.size(); ++j)
-        acc += y_[std::get<0>(sr[j])] * static_cast<TY>(weights[j] / w_sum);
+      for (size_t j = 0; j < d.size(); ++j)
+        acc += y_[static_cast<size_t>(f.idx[i * k_ + j])] * static_cast<TY>(weights[j] / w_sum);
       result[i] = acc;
     }
     return result;
@@ -756,12 +863,13 @@ class KMeans {
   // initial centroids are their means in row order (kmeans.rs:275-292).
   static KMeans fit(const DenseMatrix<TX>& data, const KMeansParameters& parameters) {
     const auto sh = data.shape();
-    const auto rows = data.row_major();
+    std::vector<TX> scratch;
+    const TX* rows = data.row_major_data(scratch);
     if (parameters.k < 2) throw Failed::fit("invalid number of clusters: " + std::to_string(parameters.k));
     if (parameters.max_iter == 0)
       throw Failed::fit("invalid maximum number of iterations: " + std::to_string(parameters.max_iter));
     sc_index* ix = nullptr;
-    detail::check(sc_index_create(rows.data(), detail::dtype_of<TX>(), sh.first, sh.second, &ix));
+    detail::check(sc_index_create(rows, detail::dtype_of<TX>(), sh.first, sh.second, &ix));
     std::unique_ptr<sc_index, int (*)(sc_index*)> guard(ix, sc_index_destroy);
     std::vector<uint32_t> y(sh.first);
     detail::check(sc_kmeans_plus_plus(ix, parameters.k, parameters.seed.has_value() ? 1 : 0,
@@ -781,12 +889,13 @@ class KMeans {
   static KMeans fit_with_centroids(const DenseMatrix<TX>& data, const KMeansParameters& parameters,
                                    std::vector<double> centroids) {
     const auto sh = data.shape();
-    const auto rows = data.row_major();
+    std::vector<TX> scratch;
+    const TX* rows = data.row_major_data(scratch);
     if (parameters.k < 2) throw Failed::fit("invalid number of clusters: " + std::to_string(parameters.k));
     if (parameters.max_iter == 0)
       throw Failed::fit("invalid maximum number of iterations: " + std::to_string(parameters.max_iter));
     sc_index* ix = nullptr;
-    detail::check(sc_index_create(rows.data(), detail::dtype_of<TX>(), sh.first, sh.second, &ix));
+    detail::check(sc_index_create(rows, detail::dtype_of<TX>(), sh.first, sh.second, &ix));
     std::unique_ptr<sc_index, int (*)(sc_index*)> guard(ix, sc_index_destroy);
     return fit_from(ix, sh.second, parameters, std::move(centroids));
   }
@@ -794,9 +903,10 @@ class KMeans {
   // kmeans.rs:327-352
   std::vector<TY> predict(const DenseMatrix<TX>& x) const {
     const auto sh = x.shape();
-    const auto rows = x.row_major();
+    std::vector<TX> scratch;
+    const TX* rows = x.row_major_data(scratch);
     std::vector<uint32_t> lab(std::max<size_t>(sh.first, 1));
-    detail::check(sc_kmeans_predict(rows.data(), detail::dtype_of<TX>(), sh.first, sh.second,
+    detail::check(sc_kmeans_predict(rows, detail::dtype_of<TX>(), sh.first, sh.second,
                                     centroids_.data(), k_, lab.data()));
     std::vector<TY> out(sh.first);
     for (size_t i = 0; i < sh.first; ++i) out[i] = static_cast<TY>(lab[i]);
@@ -944,9 +1054,10 @@ class DBSCAN {
     const auto dm = parameters.distance.device_metric();
     if (!dm) throw Failed::because(FailedError::FindFailed, "metric has no device kernel");
     const auto sh = x.shape();
-    const auto rows = x.row_major();
+    std::vector<TX> scratch;
+    const TX* rows = x.row_major_data(scratch);
     sc_index* ix = nullptr;
-    detail::check(sc_index_create(rows.data(), detail::dtype_of<TX>(), sh.first, sh.second, &ix));
+    detail::check(sc_index_create(rows, detail::dtype_of<TX>(), sh.first, sh.second, &ix));
     DBSCAN m;
     m.index_.reset(ix, [](sc_index* p) { sc_index_destroy(p); });
     m.labels_.resize(std::max<size_t>(sh.first, 1));
@@ -964,10 +1075,11 @@ class DBSCAN {
   std::vector<TY> predict(const DenseMatrix<TX>& x) const {
     const auto sh = x.shape();
     if (sh.second != dim_) throw Panic("Input vector sizes are different.");
-    const auto rows = x.row_major();
+    std::vector<TX> scratch;
+    const TX* rows = x.row_major_data(scratch);
     std::vector<int32_t> out(std::max<size_t>(sh.first, 1));
     detail::check(sc_dbscan_predict(index_.get(), labels_.data(), num_classes_, eps_, metric_, p_,
-                                    rows.data(), sh.first, out.data()));
+                                    rows, sh.first, out.data()));
     std::vector<TY> y(sh.first);
     for (size_t i = 0; i < sh.first; ++i) y[i] = static_cast<TY>(out[i]);
     return y;

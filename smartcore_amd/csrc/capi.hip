@@ -114,7 +114,15 @@ struct Stager {
   void* buf[2] = {nullptr, nullptr};
   hipEvent_t ev[2] = {nullptr, nullptr};
   bool used[2] = {false, false};
+  uint64_t* counters = nullptr;  // pinned, for the counters of one search
   hipError_t init() {
+    if (!counters) {
+      hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&counters), 64, hipHostMallocDefault);
+      if (e != hipSuccess) {
+        counters = nullptr;
+        return e;
+      }
+    }
     for (int i = 0; i < 2; ++i) {
       if (!buf[i]) {
         hipError_t e = hipHostMalloc(&buf[i], kStageBytes, hipHostMallocDefault);
@@ -254,6 +262,64 @@ int download_staged(void* host, const void* dev, size_t bytes, hipStream_t strea
 }
 
 namespace {
+thread_local bool t_may_defer = false;  // the caller settles this search's counters
+thread_local bool t_deferred = false;
+}  // namespace
+
+bool defer_search_counters(const void* dev, hipStream_t stream) {
+  if (!t_may_defer || t_deferred) return false;
+  Stager& st = thread_stager();
+  if (st.init() != hipSuccess ||
+      hipMemcpyAsync(st.counters, dev, 2 * sizeof(uint64_t), hipMemcpyDeviceToHost, stream) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  t_deferred = true;
+  return true;
+}
+
+namespace {
+// Lets the searches of its lifetime leave their counters to be read after the
+// caller's own wait for the results.
+struct DeferCounters {
+  DeferCounters() {
+    t_may_defer = true;
+    t_deferred = false;
+  }
+  ~DeferCounters() { t_may_defer = t_deferred = false; }
+  // once the stream has been waited for
+  void settle() {
+    if (!t_deferred) return;
+    const uint64_t* h = thread_stager().counters;
+    last_stats().overflow_queries += static_cast<uint32_t>(h[0]);
+    last_stats().candidates += h[1];
+    t_deferred = false;
+  }
+};
+
+// A search's results, one after another on the device (idx, dist, count): one
+// copy and one wait when they fit a staging buffer.
+int download_results(int64_t* idx, double* dist, uint32_t* count, const char* dev, size_t qk, size_t q,
+                     hipStream_t stream) {
+  const size_t half = qk * sizeof(int64_t), total = 2 * half + q * sizeof(uint32_t);
+  if (total > kStageBytes) {
+    if (int rc = download_staged(idx, dev, half, stream)) return rc;
+    if (int rc = download_staged(dist, dev + half, half, stream)) return rc;
+    return download_staged(count, dev + 2 * half, q * sizeof(uint32_t), stream);
+  }
+  Stager& st = thread_stager();
+  SC_HIP(st.init());
+  SC_HIP(hipMemcpyAsync(st.buf[0], dev, total, hipMemcpyDeviceToHost, stream));
+  st.used[0] = true;
+  SC_HIP(hipEventRecord(st.ev[0], stream));
+  SC_HIP(hipEventSynchronize(st.ev[0]));
+  const char* h = static_cast<const char*>(st.buf[0]);
+  parallel_copy(idx, h, half);
+  parallel_copy(dist, h + half, half);
+  std::memcpy(count, h + 2 * half, q * sizeof(uint32_t));
+  return SC_OK;
+}
+
 // n rows of rb bytes to a stride of lb bytes, the padding zeroed (word
 // loops: rows here are a few dozen bytes, too short for memcpy calls)
 void copy_rows(char* __restrict__ dst, const char* __restrict__ src, size_t n, size_t rb, size_t lb) {
@@ -669,19 +735,18 @@ int sc_knn_search(const sc_index* index, const void* queries, size_t q, size_t k
   SC_HIP(hipSetDevice(index->device));
   hipStream_t s = stream_for(index);
   const size_t es = elem_size(index->dtype);
-  DevBuf dq, di, dd, dc;
+  const size_t qk = q * k;
+  DevBuf dq, out;
   SC_HIP(dq.alloc(q * index->ld * es, s));
-  SC_HIP(di.alloc(q * k * sizeof(int64_t), s));
-  SC_HIP(dd.alloc(q * k * sizeof(double), s));
-  SC_HIP(dc.alloc(q * sizeof(uint32_t), s));
+  SC_HIP(out.alloc(2 * qk * sizeof(int64_t) + q * sizeof(uint32_t), s));
   if (int rc = upload_padded(queries, index->dtype, q, index->d, index->ld, dq.p, s)) return rc;
-  if (int rc = search_device_impl(index, dq.p, q, k, metric, p, mode, di.as<int64_t>(),
-                                  dd.as<double>(), dc.as<uint32_t>(), s, true))
+  DeferCounters counters;
+  if (int rc = search_device_impl(index, dq.p, q, k, metric, p, mode, out.as<int64_t>(),
+                                  out.as<double>() + qk,
+                                  reinterpret_cast<uint32_t*>(out.as<double>() + 2 * qk), s, true))
     return rc;
-  if (int rc = download_staged(idx, di.p, q * k * sizeof(int64_t), s)) return rc;
-  if (int rc = download_staged(dist, dd.p, q * k * sizeof(double), s)) return rc;
-  if (int rc = download_staged(count, dc.p, q * sizeof(uint32_t), s)) return rc;
-  SC_HIP(hipStreamSynchronize(s));
+  if (int rc = download_results(idx, dist, count, out.as<char>(), qk, q, s)) return rc;
+  counters.settle();
   return SC_OK;
 }
 

@@ -189,6 +189,10 @@ int upload_staged(void* dev, const void* host, size_t bytes, hipStream_t stream)
 int upload_staged_rows(void* dev, const void* host, size_t n, size_t row_bytes, size_t ld_bytes,
                        hipStream_t stream);
 int download_staged(void* host, const void* dev, size_t bytes, hipStream_t stream);
+// A search's counters (listed queries, candidates: two u64 at dev): queues
+// their copy and returns true when the caller of the search adds them to
+// last_stats() after its own wait for the results; false: read them now.
+bool defer_search_counters(const void* dev, hipStream_t stream);
 // Several host row blocks, each widened to its own stride, placed back to
 // back on the device from `dev`: rows of consecutive blocks share staging
 // buffers, so many small blocks move as a few large copies.

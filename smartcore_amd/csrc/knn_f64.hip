@@ -366,7 +366,7 @@ int run_f64(const sc_index* index, const T* d_queries, int64_t q, int k, int64_t
     if (int rc = launch_serial_exact(index, qs, k, olist.as<uint32_t>(), list_n, d_idx + b0 * k,
                                      d_dist + b0 * k, d_count + b0, s))
       return rc;
-    if (stats) {
+    if (stats && !(qn == q && defer_search_counters(flags.p, s))) {
       uint64_t h[2] = {0, 0};
       SC_HIP(hipMemcpyAsync(h, flags.p, 16, hipMemcpyDeviceToHost, s));
       SC_HIP(hipStreamSynchronize(s));

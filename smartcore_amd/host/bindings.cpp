@@ -31,10 +31,12 @@ struct PyKNNParams {
   SearchMode mode = SearchMode::PlainFp64;
 };
 
+// A view of the array's rows: `a` outlives every use (the estimators copy
+// what they keep).
 template <typename T>
-DenseMatrix<T> to_matrix(py::array_t<T, py::array::c_style | py::array::forcecast> a) {
+DenseMatrix<T> to_matrix(const py::array_t<T, py::array::c_style | py::array::forcecast>& a) {
   if (a.ndim() != 2) throw Failed::input("x must be a 2-D array");
-  return DenseMatrix<T>::from_row_major(a.shape(0), a.shape(1), a.data());
+  return DenseMatrix<T>::view_row_major(a.shape(0), a.shape(1), a.data());
 }
 
 template <typename T, typename D>
@@ -111,7 +113,8 @@ class PyKNN {
 
   template <typename T>
   static V fit_t(py::array x, const std::vector<TY>& y, const PyKNNParams& p) {
-    auto mx = to_matrix<T>(py::array_t<T, py::array::c_style | py::array::forcecast>::ensure(x));
+    const auto a = py::array_t<T, py::array::c_style | py::array::forcecast>::ensure(x);
+    const auto mx = to_matrix<T>(a);
     switch (p.distance.metric) {
       case SC_EUCLIDIAN:
         return Est<T, TY, Euclidian<T>>::fit(mx, y, params_for<T>(p, Euclidian<T>{}));
@@ -184,7 +187,8 @@ class PyDBSCAN {
 
   template <typename T>
   static V fit_t(py::array x, const PyDBSCANParams& p) {
-    auto mx = to_matrix<T>(py::array_t<T, py::array::c_style | py::array::forcecast>::ensure(x));
+    const auto a = py::array_t<T, py::array::c_style | py::array::forcecast>::ensure(x);
+    const auto mx = to_matrix<T>(a);
     auto base = DBSCANParameters<T>{}.with_min_samples(p.min_samples).with_eps(p.eps)
                     .with_algorithm(p.algorithm);
     switch (p.distance.metric) {
