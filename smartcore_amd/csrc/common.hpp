@@ -247,6 +247,12 @@ int knn_exact_device(const sc_index* index, const void* d_queries, size_t q, siz
                      sc_metric metric, int p, int64_t* d_idx, double* d_dist, uint32_t* d_count,
                      hipStream_t stream, sc_stats* stats);
 
+// Few queries over few rows (knn_few.hip): whether a plain search goes there,
+// and the search.
+bool knn_few_applies(const sc_index* index, size_t q, size_t k, sc_metric metric);
+int knn_few_device(const sc_index* index, const void* d_queries, size_t q, size_t k, sc_metric metric,
+                   int64_t* d_idx, double* d_dist, uint32_t* d_count, hipStream_t s, sc_stats* stats);
+
 // The same for the Euclidian metric and k <= 64, on FP64 matrix instructions
 // (queries: at least one).
 int knn_f64_device(const sc_index* index, const void* d_queries, int64_t q, int k, int64_t* d_idx,

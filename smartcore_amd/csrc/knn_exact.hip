@@ -1,7 +1,8 @@
 // Exact brute-force kNN (LinearKNNSearch::find, linear_search.rs:52-84) for
 // the Manhattan and Minkowski metrics on f64 / f32 rows, and the sequential
 // kernel every form falls back to.  (Euclidian searches with k <= 64 run on
-// FP64 matrix instructions, knn_f64.hip: their sums have a dot-product form.)
+// FP64 matrix instructions, knn_f64.hip: their sums have a dot-product form;
+// few queries over few rows go to knn_few.hip.)
 //
 // Three kernels:
 //   scan    Tiled distance kernel.  A workgroup owns 32 queries x one
@@ -792,6 +793,8 @@ int knn_exact_device(const sc_index* index, const void* d_queries, size_t q, siz
                      sc_metric metric, int p, int64_t* d_idx, double* d_dist, uint32_t* d_count,
                      hipStream_t stream, sc_stats* stats) {
   if (q == 0) return SC_OK;
+  if (knn_few_applies(index, q, k, metric))
+    return knn_few_device(index, d_queries, q, k, metric, d_idx, d_dist, d_count, stream, stats);
   if (metric == SC_EUCLIDIAN && k <= KMAX_TILED)
     return knn_f64_device(index, d_queries, static_cast<int64_t>(q), static_cast<int>(k), d_idx,
                           d_dist, d_count, stream, stats);
