@@ -216,8 +216,9 @@ int sc_kmeans_batch_run(const sc_kmeans_problem* problems, size_t count, sc_dtyp
 /* KMeans::kmeans_plus_plus (kmeans.rs:354-413): initial labels (n) of the
  * index's rows for k clusters.  The random stream is rand 0.8.5's SmallRng
  * seeded by get_rng_impl (rand_custom.rs:8-33: has_seed ? seed : 0).  The
- * per-round distance updates run on the device in the rows' own type; the
- * sequential cost sum and cumulative scan run on the host in row order. */
+ * rounds run on the device, distances in the rows' own type; a round whose
+ * choice depends on the order in which the costs are added is repeated on the
+ * host in row order. */
 int sc_kmeans_plus_plus(const sc_index* index, size_t k, int has_seed, uint64_t seed,
                         uint32_t* labels);
 /* KMeans::predict (kmeans.rs:327-352): labels of n rows of x (host,
@@ -229,9 +230,9 @@ int sc_kmeans_predict(const void* x, sc_dtype dtype, size_t n, size_t d,
 /* DBSCAN::fit (dbscan.rs:274-354) over the index's rows with find_radius
  * (linear_search.rs:89-108) as its neighbourhood query: labels (n) get -1
  * for outliers and the cluster id otherwise, num_classes the number of
- * clusters.  The neighbourhoods of all rows are computed on the device in
- * one batched radius search; the expansion loop runs on the host in the
- * reference's order.  Errors: SC_FIT_FAILED "Invalid minPts"
+ * clusters.  Neighbourhoods, clusters and (Euclidian) their numbering are
+ * computed on the device; the labels are those of the reference's expansion
+ * loop.  Errors: SC_FIT_FAILED "Invalid minPts"
  * (min_samples < 1), "Invalid radius: " (eps <= 0). */
 int sc_dbscan_fit(const sc_index* index, double eps, size_t min_samples, sc_metric metric,
                   uint16_t p, int32_t* labels, size_t* num_classes);
@@ -295,8 +296,10 @@ int sc_last_stats(sc_stats* out);
  * HIP events on the stream it runs on.  sc_profile_enable(1) clears earlier
  * records.  sc_profile_read waits for the recorded events and returns the
  * summed duration and the launch count of one family: "knn_scan",
- * "knn_replay", "knn_serial", "knn_mixed_gemm", "knn_mixed_rescore",
- * "kmeans_assign", "kmeans_partial", "kmeans_reduce", "kmeans_mixed_assign". */
+ * "knn_replay", "knn_serial", "knn_scan_q16", "knn_mixed_prefix",
+ * "knn_mixed_gemm", "knn_mixed_rescore", "radius_sweep", "dbscan_group",
+ * "dbscan_pairs", "kmeans_assign", "kmeans_partial", "kmeans_reduce",
+ * "kmeans_mixed_assign", "kmeans_batch". */
 int sc_profile_enable(int on);
 int sc_profile_read(const char* kernel, double* total_ms, uint64_t* launches);
 
