@@ -740,11 +740,11 @@ __global__ __launch_bounds__(kSumThreads, DPL == 1 && !(PACK && sizeof(T) == 8) 
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
 #pragma unroll
-          for (int t = 0; t < kSumBatch<T>; ++t) {
-            // (+0.0 past the run's end, see sum_runs_packed)
-            acc[u][0] = acc[u][0] + static_cast<double>(t < nv[u] ? x[u][t][0] : T(0));
-            if (DPL > 1) acc[u][1] = acc[u][1] + static_cast<double>(t < nv[u] ? x[u][t][1] : T(0));
-          }
+          for (int t = 0; t < kSumBatch<T>; ++t)
+            if (t < nv[u]) {  // (the same in the whole wavefront: a scalar branch)
+              acc[u][0] = acc[u][0] + static_cast<double>(x[u][t][0]);
+              if (DPL > 1) acc[u][1] = acc[u][1] + static_cast<double>(x[u][t][1]);
+            }
           e[u] += nv[u];
         }
       }

@@ -115,7 +115,7 @@ __device__ __forceinline__ uint16_t bf16_rne(float f) {
 // kPrepLanes lanes (sub: this one), which read 16 bytes of it each in turn.
 // A thread per row asks for 64 lines per load and uses 4 bytes of each: the
 // preparation of 4,000,000 x 128 rows took 12.6 ms that way, 0.56 with
-// this (3 GB moved), and 8,192 queries 126 us, 15.
+// this (3 GB moved), and 65,536 queries 126 us, 15.
 // (The sums' order is free: what is made of them leaves 2^-40 for it.)
 constexpr int kPrepLanes = 8;
 constexpr int kPrepThreads = 256;
