@@ -172,6 +172,12 @@ constexpr uint32_t kUnresolved = 0xffffffffu;
 constexpr int64_t kListTotal = int64_t(1) << 26;
 constexpr int64_t kListMin = 256, kListMax = 65536;
 constexpr int64_t kSweepQueries = int64_t(1) << 19;  // per sweep
+// Fewer pairs take the two passes: a search so small waits for its launches,
+// and lists with many matches cost the sweep more of them (f32, us, two passes
+// and sweep: 212 queries x 14,151 x 21, 69 matches each: 150 and 161; 100 x
+// 10,000 x 48, 98 matches: 136 and 155, 11 matches: 114 and 98; 100 x 40,000 x
+// 16, 41 matches: 140 and 116; 600 x 10,000 x 16, 76 matches: 211 and 168).
+constexpr double kSweepMinPairs = 3.5e6;
 
 template <typename T>
 __global__ __launch_bounds__(kMT, 2) void radius_sweep_kernel(
@@ -521,7 +527,8 @@ int run_radius(const sc_index* ix, const T* dq, int64_t q, double p, double radi
   if (!std::isfinite(bound)) bound = INFINITY;
   // (a larger bound would admit sums that overflow in the rows' type)
   if constexpr (M == kEuclid) {
-    if (allow_cap && bound < sum_limit<T>()) {
+    if (allow_cap && bound < sum_limit<T>() &&
+        static_cast<double>(q) * static_cast<double>(n) > kSweepMinPairs) {
       if (q <= kSweepQueries) return run_radius_f64<T>(ix, dq, q, radius, bound, res, want_dist, s);
       res->q = static_cast<size_t>(q);
       res->offsets.assign(1, 0);
