@@ -286,17 +286,13 @@ int run_f64(const sc_index* index, const T* d_queries, int64_t q, int k, int64_t
   Lists<double> ls{};
   ls.nlevels = nlev;
   ls.pre_cap = pre_cap;
-  // the candidate store of a call is bounded by batches of queries (whole
-  // query tiles); a smaller batch has longer lists per query, so the size is
-  // found by halving
-  int64_t qb = q;
-  for (;;) {
-    plan(qb, ls.lv, ls.out);
-    const double bytes = static_cast<double>(qb) * (12.0 * ls.out.entries + 4.0 * ls.out.lists +
-                                                    4.0 * pre_cap + 8.0 * (cols + k + 1));
-    if (bytes <= 1.5 * 1024.0 * 1024.0 * 1024.0 || qb <= kMQ) break;
-    qb = std::max<int64_t>(kMQ, (qb / 2 + kMQ - 1) / kMQ * kMQ);
-  }
+  const Batches batches = plan_batches<double>(
+      q, plan,
+      [&](const ScanOut<double>& o) {
+        return 12.0 * o.entries + 4.0 * o.lists + 4.0 * pre_cap + 8.0 * (cols + k + 1);
+      },
+      ls.lv, ls.out);
+  const int64_t qb = batches.queries;
   DevBuf flags, olist, x2m, dense, pidx, pcnt, cidx, cu, ccnt, seed;
   SC_HIP(flags.alloc(64, s));  // [0] listed queries, [2..3] candidate total (u64)
   SC_HIP(olist.alloc(sizeof(uint32_t) * qb, s));
@@ -305,9 +301,9 @@ int run_f64(const sc_index* index, const T* d_queries, int64_t q, int k, int64_t
   SC_HIP(pidx.alloc(sizeof(uint32_t) * qb * pre_cap, s));
   SC_HIP(pcnt.alloc(sizeof(uint32_t) * qb, s));
   SC_HIP(seed.alloc(sizeof(double) * qb * k, s));
-  SC_HIP(cidx.alloc(sizeof(uint32_t) * qb * ls.out.entries, s));
-  SC_HIP(cu.alloc(sizeof(double) * qb * ls.out.entries, s));
-  SC_HIP(ccnt.alloc(sizeof(uint32_t) * qb * ls.out.lists, s));
+  SC_HIP(cidx.alloc(sizeof(uint32_t) * batches.entries, s));
+  SC_HIP(cu.alloc(sizeof(double) * batches.entries, s));
+  SC_HIP(ccnt.alloc(sizeof(uint32_t) * batches.lists, s));
   uint32_t* list_n = flags.as<uint32_t>();
   unsigned long long* total = reinterpret_cast<unsigned long long*>(flags.as<char>() + 8);
   hipLaunchKernelGGL(zero_words_kernel, dim3(1), dim3(64), 0, s, flags.as<uint32_t>(), int64_t{16});
@@ -315,13 +311,6 @@ int run_f64(const sc_index* index, const T* d_queries, int64_t q, int k, int64_t
     const int64_t qn = std::min(qb, q - b0);
     const T* qs = d_queries + b0 * ld;
     if (qn != qb) plan(qn, ls.lv, ls.out);
-    if (ls.out.entries > 0 && qn != qb && (ls.out.entries * qn > static_cast<int64_t>(cidx.cap / 4) ||
-                                           ls.out.lists * qn > static_cast<int64_t>(ccnt.cap / 4))) {
-      // a short last batch spreads over more pieces
-      SC_HIP(cidx.alloc(sizeof(uint32_t) * qn * ls.out.entries, s));
-      SC_HIP(cu.alloc(sizeof(double) * qn * ls.out.entries, s));
-      SC_HIP(ccnt.alloc(sizeof(uint32_t) * qn * ls.out.lists, s));
-    }
     ls.pre_idx = pidx.as<uint32_t>();
     ls.pre_count = pcnt.as<uint32_t>();
     ls.out.idx = cidx.as<uint32_t>();

@@ -630,14 +630,13 @@ int knn_l1q_device(const sc_index* index, const float* d_queries, int64_t q, int
   Lists<uint32_t> ls{};
   ls.nlevels = nlev;
   ls.pre_cap = pre_cap;
-  int64_t qb = q;
-  for (;;) {
-    plan(qb, ls.lv, ls.out);
-    const double bytes = static_cast<double>(qb) * (8.0 * ls.out.entries + 4.0 * ls.out.lists +
-                                                    4.0 * pre_cap + 4.0 * (cols + k + ldq));
-    if (bytes <= 1.5 * 1024.0 * 1024.0 * 1024.0 || qb <= 128) break;
-    qb = std::max<int64_t>(128, (qb / 2 + 127) / 128 * 128);
-  }
+  const Batches batches = plan_batches<uint32_t>(
+      q, plan,
+      [&](const ScanOut<uint32_t>& o) {
+        return 8.0 * o.entries + 4.0 * o.lists + 4.0 * pre_cap + 4.0 * (cols + k + ldq);
+      },
+      ls.lv, ls.out);
+  const int64_t qb = batches.queries;
   DevBuf flags, olist, qcodes, qerr, dense, pidx, pcnt, cidx, cu, ccnt, seed;
   SC_HIP(flags.alloc(64, s));  // [0] listed queries, [2..3] candidate total (u64)
   SC_HIP(olist.alloc(sizeof(uint32_t) * qb, s));
@@ -647,6 +646,9 @@ int knn_l1q_device(const sc_index* index, const float* d_queries, int64_t q, int
   SC_HIP(pidx.alloc(sizeof(uint32_t) * qb * pre_cap, s));
   SC_HIP(pcnt.alloc(sizeof(uint32_t) * qb, s));
   SC_HIP(seed.alloc(sizeof(uint32_t) * qb * k, s));
+  SC_HIP(cidx.alloc(sizeof(uint32_t) * batches.entries, s));
+  SC_HIP(cu.alloc(sizeof(uint32_t) * batches.entries, s));
+  SC_HIP(ccnt.alloc(sizeof(uint32_t) * batches.lists, s));
   uint32_t* list_n = flags.as<uint32_t>();
   unsigned long long* total = reinterpret_cast<unsigned long long*>(flags.as<char>() + 8);
   hipLaunchKernelGGL(zero_words_kernel, dim3(1), dim3(64), 0, s, flags.as<uint32_t>(), int64_t{16});
@@ -654,13 +656,6 @@ int knn_l1q_device(const sc_index* index, const float* d_queries, int64_t q, int
     const int64_t qn = std::min(qb, q - b0);
     const float* qs = d_queries + b0 * ld;
     if (qn != qb) plan(qn, ls.lv, ls.out);
-    // (a short last batch spreads over more pieces)
-    if (b0 == 0 || ls.out.entries * qn > static_cast<int64_t>(cidx.cap / 4) ||
-        ls.out.lists * qn > static_cast<int64_t>(ccnt.cap / 4)) {
-      SC_HIP(cidx.alloc(sizeof(uint32_t) * qn * ls.out.entries, s));
-      SC_HIP(cu.alloc(sizeof(uint32_t) * qn * ls.out.entries, s));
-      SC_HIP(ccnt.alloc(sizeof(uint32_t) * qn * ls.out.lists, s));
-    }
     ls.pre_idx = pidx.as<uint32_t>();
     ls.pre_count = pcnt.as<uint32_t>();
     ls.out.idx = cidx.as<uint32_t>();
