@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <cstdio>
 #include <memory>
@@ -225,6 +226,22 @@ class ProfScope {
   hipStream_t stream_;
   hipEvent_t start_ = nullptr;
 };
+
+// Blocks for `lanes` threads per row (or query).  A launch holds fewer than
+// 2^32 threads a dimension, which 2^28 rows of sixteen lanes pass, so the
+// kernels stride over the rows past the grid.
+constexpr int64_t kRowBlocks = int64_t(1) << 20;
+inline unsigned row_blocks(int64_t rows, int lanes, int block) {
+  const int64_t per = block / lanes;
+  return static_cast<unsigned>(std::min(kRowBlocks, (rows + per - 1) / per));
+}
+// The calling thread's row and the step to its next one.
+__device__ __forceinline__ int64_t lane_row(int lanes) {
+  return (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) / lanes;
+}
+__device__ __forceinline__ int64_t lane_row_step(int lanes) {
+  return static_cast<int64_t>(gridDim.x) * blockDim.x / lanes;
+}
 
 // Whether work on s is being recorded into a graph (or that cannot be told).
 bool stream_capturing(hipStream_t s);

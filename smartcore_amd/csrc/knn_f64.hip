@@ -82,15 +82,15 @@ template <typename T>
 __global__ void row_norms_kernel(const T* __restrict__ rows, int64_t n, int64_t npad, int ld,
                                  double shrink, double* __restrict__ y2m) {
   const int sub = threadIdx.x & 15;
-  const int64_t i = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) >> 4;
-  if (i >= npad) return;  // sixteen lanes together
-  double out = INFINITY;
-  if (i < n) {
-    bool finite;
-    const double s = row_norm(rows + i * ld, ld, sub, &finite);
-    if (finite) out = s < kNorm64Limit ? s * shrink : NAN;
+  for (int64_t i = lane_row(16); i < npad; i += lane_row_step(16)) {  // sixteen lanes together
+    double out = INFINITY;
+    if (i < n) {
+      bool finite;
+      const double s = row_norm(rows + i * ld, ld, sub, &finite);
+      if (finite) out = s < kNorm64Limit ? s * shrink : NAN;
+    }
+    if (sub == 0) y2m[i] = out;
   }
-  if (sub == 0) y2m[i] = out;
 }
 
 template <typename T>
@@ -98,14 +98,14 @@ __global__ void query_norms_kernel(const T* __restrict__ qs, int64_t q, int ld, 
                                    double* __restrict__ x2m, uint32_t* __restrict__ list,
                                    uint32_t* __restrict__ list_n) {
   const int sub = threadIdx.x & 15;
-  const int64_t i = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) >> 4;
-  if (i >= q) return;
-  bool finite;
-  const double s = row_norm(qs + i * ld, ld, sub, &finite);
-  if (sub != 0) return;
-  const bool in = finite && s < kNorm64Limit;
-  x2m[i] = in ? s * shrink : INFINITY;
-  if (finite && !in) list[atomicAdd(list_n, 1u)] = static_cast<uint32_t>(i);
+  for (int64_t i = lane_row(16); i < q; i += lane_row_step(16)) {
+    bool finite;
+    const double s = row_norm(qs + i * ld, ld, sub, &finite);
+    if (sub != 0) continue;
+    const bool in = finite && s < kNorm64Limit;
+    x2m[i] = in ? s * shrink : INFINITY;
+    if (finite && !in) list[atomicAdd(list_n, 1u)] = static_cast<uint32_t>(i);
+  }
 }
 
 // L of queries x the first `cols` rows (a multiple of kMR, rows past the
@@ -375,7 +375,7 @@ int ensure_norms64(sc_index* ix, DevBuf& local, const double** y2m, hipStream_t 
   const int ld = static_cast<int>(ix->ld);
   const double shrink = 1.0 - norm_gap(ld);
   auto launch = [&](double* out) -> int {
-    const dim3 grid(static_cast<unsigned>((npad * 16 + 255) / 256));
+    const dim3 grid(row_blocks(npad, 16, 256));
     if (ix->dtype == SC_F64)
       hipLaunchKernelGGL(row_norms_kernel<double>, grid, dim3(256), 0, s,
                          static_cast<const double*>(ix->rows), n, npad, ld, shrink, out);
@@ -416,7 +416,7 @@ int ensure_norms64(sc_index* ix, DevBuf& local, const double** y2m, hipStream_t 
 template <typename T>
 int query_norms64(const T* queries, int64_t q, int ld, double* x2m, uint32_t* list,
                   uint32_t* list_n, hipStream_t s) {
-  hipLaunchKernelGGL(query_norms_kernel<T>, dim3(static_cast<unsigned>((q * 16 + 255) / 256)), dim3(256),
+  hipLaunchKernelGGL(query_norms_kernel<T>, dim3(row_blocks(q, 16, 256)), dim3(256),
                      0, s, queries, q, ld, 1.0 - norm_gap(ld), x2m, list, list_n);
   SC_HIP(hipGetLastError());
   return SC_OK;

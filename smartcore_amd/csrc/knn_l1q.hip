@@ -154,17 +154,17 @@ __global__ void q16_rows_kernel(const float* __restrict__ rows, int64_t n, int64
                                 int ld, double lo, double h, uint32_t* __restrict__ codes,
                                 uint32_t* __restrict__ er) {
   const int sub = threadIdx.x & 7;
-  const int64_t i = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) >> 3;
-  if (i >= npad) return;
-  uint32_t e = 0u;
-  if (i < n) {
-    bool ok;
-    const double err = q16_vector(rows + i * ld, d, ld, lo, h, 1.0 / h, sub, codes + i * (ld / 2), &ok);
-    // err carries at most two roundings per term (the difference, the add):
-    // scale it up by more than that, then round up to an integer
-    e = static_cast<uint32_t>(ceil(err * (1.0 + (2.0 * d + 4.0) * 2.220446049250313e-16)));
+  for (int64_t i = lane_row(8); i < npad; i += lane_row_step(8)) {  // eight lanes together
+    uint32_t e = 0u;
+    if (i < n) {
+      bool ok;
+      const double err = q16_vector(rows + i * ld, d, ld, lo, h, 1.0 / h, sub, codes + i * (ld / 2), &ok);
+      // err carries at most two roundings per term (the difference, the add):
+      // scale it up by more than that, then round up to an integer
+      e = static_cast<uint32_t>(ceil(err * (1.0 + (2.0 * d + 4.0) * 2.220446049250313e-16)));
+    }
+    if (sub == 0) er[i] = e;
   }
-  if (sub == 0) er[i] = e;
 }
 
 // Queries: codes (clamped) and eq; a query with a value outside the domain
@@ -174,13 +174,13 @@ __global__ void q16_queries_kernel(const float* __restrict__ qs, int64_t q, int 
                                    double* __restrict__ eq, uint32_t* __restrict__ list,
                                    uint32_t* __restrict__ list_n) {
   const int sub = threadIdx.x & 7;
-  const int64_t i = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) >> 3;
-  if (i >= q) return;
-  bool ok;
-  const double err = q16_vector(qs + i * ld, d, ld, lo, h, 1.0 / h, sub, codes + i * (ld / 2), &ok);
-  if (sub != 0) return;
-  eq[i] = ok ? __ocml_mul_rtp_f64(err, 1.0 + (2.0 * d + 4.0) * 2.220446049250313e-16) : INFINITY;
-  if (!ok) list[atomicAdd(list_n, 1u)] = static_cast<uint32_t>(i);
+  for (int64_t i = lane_row(8); i < q; i += lane_row_step(8)) {
+    bool ok;
+    const double err = q16_vector(qs + i * ld, d, ld, lo, h, 1.0 / h, sub, codes + i * (ld / 2), &ok);
+    if (sub != 0) continue;
+    eq[i] = ok ? __ocml_mul_rtp_f64(err, 1.0 + (2.0 * d + 4.0) * 2.220446049250313e-16) : INFINITY;
+    if (!ok) list[atomicAdd(list_n, 1u)] = static_cast<uint32_t>(i);
+  }
 }
 
 
@@ -586,7 +586,7 @@ int ensure_q16(sc_index* ix, bool* coded, hipStream_t s) {
     (void)hipFree(codes);
     return hip_fail(hipErrorOutOfMemory, "hipMalloc(row code errors)");
   }
-  hipLaunchKernelGGL(q16_rows_kernel, dim3(static_cast<unsigned>((npad + 31) / 32)), dim3(256), 0, s,
+  hipLaunchKernelGGL(q16_rows_kernel, dim3(row_blocks(npad, 8, 256)), dim3(256), 0, s,
                      rows, n, npad, d, ld, lo, step, static_cast<uint32_t*>(codes), er);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) e = hipStreamSynchronize(s);
@@ -662,7 +662,7 @@ int knn_l1q_device(const sc_index* index, const float* d_queries, int64_t q, int
     ls.out.u = cu.as<uint32_t>();
     ls.out.count = ccnt.as<uint32_t>();
     hipLaunchKernelGGL(zero_words_kernel, dim3(1), dim3(64), 0, s, list_n, int64_t{1});
-    hipLaunchKernelGGL(q16_queries_kernel, dim3(static_cast<unsigned>((qn + 31) / 32)), dim3(256), 0, s,
+    hipLaunchKernelGGL(q16_queries_kernel, dim3(row_blocks(qn, 8, 256)), dim3(256), 0, s,
                        qs, qn, d, ld, index->q16_lo, index->q16_step, qcodes.as<uint32_t>(),
                        qerr.as<double>(), olist.as<uint32_t>(), list_n);
     SC_HIP(hipGetLastError());

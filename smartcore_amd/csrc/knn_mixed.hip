@@ -166,23 +166,23 @@ __global__ __launch_bounds__(kPrepThreads) void prep_rows_kernel(const float* __
                                  float* __restrict__ nyb, float* __restrict__ nry,
                                  float* __restrict__ nyh, uint32_t* __restrict__ bad) {
   const int sub = threadIdx.x % kPrepLanes;
-  const int64_t i = (static_cast<int64_t>(blockIdx.x) * kPrepThreads + threadIdx.x) / kPrepLanes;
-  if (i >= n) return;  // a row's lanes together
-  const RowSums t = prep_row<1>(rows + i * ld, out_b + i * ld, ld, sub);
-  if (sub != 0) return;
-  const double s = t.v2, sr = t.e2;
-  if (!t.finite || !(s < kNormLimit)) {
-    atomicOr(bad, 1u);
-    y2m[i] = INFINITY;
-    nyb[i] = 0.0f;
-    nry[i] = 0.0f;
-    nyh[i] = 0.0f;
-    return;
+  for (int64_t i = lane_row(kPrepLanes); i < n; i += lane_row_step(kPrepLanes)) {  // a row's lanes together
+    const RowSums t = prep_row<1>(rows + i * ld, out_b + i * ld, ld, sub);
+    if (sub != 0) continue;
+    const double s = t.v2, sr = t.e2;
+    if (!t.finite || !(s < kNormLimit)) {
+      atomicOr(bad, 1u);
+      y2m[i] = INFINITY;
+      nyb[i] = 0.0f;
+      nry[i] = 0.0f;
+      nyh[i] = 0.0f;
+      continue;
+    }
+    y2m[i] = __double2float_rd(s * (1.0 - kLoMargin));
+    nyb[i] = __double2float_ru(sqrt(s) * (1.0 + 9.094947017729282e-13));
+    nry[i] = __double2float_ru(sqrt(sr) * (1.0 + 9.094947017729282e-13));
+    nyh[i] = __double2float_ru((sqrt(s) + sqrt(sr)) * (1.0 + 9.094947017729282e-13));
   }
-  y2m[i] = __double2float_rd(s * (1.0 - kLoMargin));
-  nyb[i] = __double2float_ru(sqrt(s) * (1.0 + 9.094947017729282e-13));
-  nry[i] = __double2float_ru(sqrt(sr) * (1.0 + 9.094947017729282e-13));
-  nyh[i] = __double2float_ru((sqrt(s) + sqrt(sr)) * (1.0 + 9.094947017729282e-13));
 }
 
 // y2m of padding rows is +inf (their L is +inf), nyb, nry and nyh are 0.
@@ -207,26 +207,26 @@ __global__ __launch_bounds__(kPrepThreads) void prep_queries_kernel(const float*
                                     float* __restrict__ qa2, uint32_t* __restrict__ list,
                                     uint32_t* __restrict__ list_n) {
   const int sub = threadIdx.x % kPrepLanes;
-  const int64_t i = (static_cast<int64_t>(blockIdx.x) * kPrepThreads + threadIdx.x) / kPrepLanes;
-  if (i >= q) return;  // a row's lanes together
-  const RowSums t = prep_row<-2>(qs + i * ld, out_b + i * ld, ld, sub);
-  if (sub != 0) return;
-  const double s = t.v2, sr = t.e2, sh = t.h2;
-  if (!t.finite || !(s < kNormLimit)) {
-    // never a candidate in pass 1; the exact kernel takes it
-    x2m[i] = INFINITY;
-    cxb[i] = 0.0f;
-    qa1[i] = 0.0f;
-    qa2[i] = 0.0f;
-    const uint32_t slot = atomicAdd(list_n, 1u);
-    list[slot] = static_cast<uint32_t>(i);
-    return;
+  for (int64_t i = lane_row(kPrepLanes); i < q; i += lane_row_step(kPrepLanes)) {  // a row's lanes together
+    const RowSums t = prep_row<-2>(qs + i * ld, out_b + i * ld, ld, sub);
+    if (sub != 0) continue;
+    const double s = t.v2, sr = t.e2, sh = t.h2;
+    if (!t.finite || !(s < kNormLimit)) {
+      // never a candidate in pass 1; the exact kernel takes it
+      x2m[i] = INFINITY;
+      cxb[i] = 0.0f;
+      qa1[i] = 0.0f;
+      qa2[i] = 0.0f;
+      const uint32_t slot = atomicAdd(list_n, 1u);
+      list[slot] = static_cast<uint32_t>(i);
+      continue;
+    }
+    x2m[i] = __double2float_rd(s * (1.0 - kLoMargin));
+    cxb[i] = __double2float_ru(2.0 * kC1 * sqrt(s) * (1.0 + 9.5367431640625e-07));
+    qa1[i] = __double2float_ru(2.0 * sqrt(s) * (1.0 + 9.5367431640625e-07));
+    qa2[i] = __double2float_ru(2.0 * (sqrt(sr) + 128.0 * 2.384185791015625e-07 * sqrt(sh)) *
+                               (1.0 + 9.5367431640625e-07));
   }
-  x2m[i] = __double2float_rd(s * (1.0 - kLoMargin));
-  cxb[i] = __double2float_ru(2.0 * kC1 * sqrt(s) * (1.0 + 9.5367431640625e-07));
-  qa1[i] = __double2float_ru(2.0 * sqrt(s) * (1.0 + 9.5367431640625e-07));
-  qa2[i] = __double2float_ru(2.0 * (sqrt(sr) + 128.0 * 2.384185791015625e-07 * sqrt(sh)) *
-                             (1.0 + 9.5367431640625e-07));
 }
 
 __device__ __forceinline__ bf16x8 load_frag(const uint16_t* p) {
@@ -1130,7 +1130,7 @@ int ensure_bf16(sc_index* ix, hipStream_t s, bool* bad_out, int64_t* npad_out) {
                      0, s, terms, terms + npad, terms + 2 * npad, terms + 3 * npad, n, npad);
   if (n > 0)
     hipLaunchKernelGGL(prep_rows_kernel,
-                       dim3(static_cast<unsigned>((n * kPrepLanes + kPrepThreads - 1) / kPrepThreads)),
+                       dim3(row_blocks(n, kPrepLanes, kPrepThreads)),
                        dim3(kPrepThreads), 0, s, static_cast<const float*>(ix->rows), n, static_cast<int>(ix->ld),
                        static_cast<uint16_t*>(b), terms, terms + npad, terms + 2 * npad,
                        terms + 3 * npad, flag.as<uint32_t>());
@@ -1299,7 +1299,7 @@ int knn_mixed_device(const sc_index* cix, const void* d_queries, size_t q_, size
   const float* qf = static_cast<const float*>(d_queries);
 
   hipLaunchKernelGGL(prep_queries_kernel,
-                     dim3(static_cast<unsigned>((q * kPrepLanes + kPrepThreads - 1) / kPrepThreads)),
+                     dim3(row_blocks(q, kPrepLanes, kPrepThreads)),
                      dim3(kPrepThreads), 0, stream, qf, q, ld, qb.as<uint16_t>(), x2.as<float>(), cx.as<float>(),
                      cx.as<float>() + q, cx.as<float>() + 2 * q, lst.as<uint32_t>(), list_n);
   SC_HIP(hipGetLastError());
