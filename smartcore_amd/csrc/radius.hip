@@ -154,37 +154,66 @@ __global__ void gather_rows_kernel(const T* __restrict__ src, int ld,
 //            the radius go to a list per (query, piece) in row order.  The
 //            (query tile, row tile) pairs, query tiles outermost, are dealt
 //            to the workgroups in contiguous runs; a piece is the part of a
-//            run inside one query tile.
-//   resolve  one wavefront per query: the exact distance of every candidate,
-//            the matches moved to the front of the query's lists, and their
-//            count (kUnresolved when a list overflowed or the query's norm is
-//            out of the bound's range: those are searched by the count and
-//            fill passes).
+//            run inside one query tile.  A candidate whose upper bound is
+//            inside the radius too is a match; the others make their list
+//            unsure.
+//   resolve  a workgroup per query: the exact distances of the unsure lists'
+//            candidates, whose matches move to the front of the list, and the
+//            query's count (kUnresolved when a list overflowed or the query's
+//            norm is out of the bound's range).
 //   emit     the matches to their CSR place, with their distances.
+// Queries whose lists overflowed are swept once more into lists of the sizes
+// that the first sweep counted; norms out of range take the count and fill
+// passes.
 // One sweep takes the place of a count and a fill pass, and an MFMA per four
-// dimensions that of three vector instructions per dimension and pair.
-// 5,000 queries x 100,000 x 16 f32 rows, 40 matches each: 0.84 ms, 0.49 of it
-// kernels (2.6 and 2.34 before).
+// dimensions that of three vector instructions per dimension and pair.  With
+// many matches the sweep's time goes to appending them (5,000 queries x
+// 100,000 x 16 f32: 0.41 ms with 20 matches each, 1.01 with 1,417; the two
+// passes 2.7), so matches are neither counted nor summed twice: 0.12 ms for
+// 7.1 million of them, whole calls 581 and 2,387 us with 20 matches, 7,500 and
+// 9,700 with 1,417 (sweep and two passes).  Summing every candidate to count it, by
+// one wavefront per query, and sending queries past 65,536 entries to the two
+// passes made 10 queries x 1,000,000 x 8 f64 with 50,000 matches each 3,300 us;
+// they take 661 now and 683 with the two passes.
 constexpr uint32_t kUnresolved = 0xffffffffu;
-// Lists of a sweep: 256 MiB in all, but 256 to 65,536 entries per query (a
-// small query set sees many pieces, and clustered rows put a query's matches
-// into few of them).
+constexpr uint64_t kNoPlace = ~uint64_t(0);
+// Lists of a sweep: room for every pair, or 256 MiB in all (but 256 entries
+// per query).
 constexpr int64_t kListTotal = int64_t(1) << 26;
-constexpr int64_t kListMin = 256, kListMax = 65536;
+constexpr int64_t kListMin = 256;
 constexpr int64_t kSweepQueries = int64_t(1) << 19;  // per sweep
-// Fewer pairs take the two passes: a search so small waits for its launches,
-// and lists with many matches cost the sweep more of them (f32, us, two passes
-// and sweep: 212 queries x 14,151 x 21, 69 matches each: 150 and 161; 100 x
-// 10,000 x 48, 98 matches: 136 and 155, 11 matches: 114 and 98; 100 x 40,000 x
-// 16, 41 matches: 140 and 116; 600 x 10,000 x 16, 76 matches: 211 and 168).
+constexpr uint64_t kSecondMax = uint64_t(1) << 31;   // entries of a second sweep
+// Fewer pairs take the two passes, whose three launches fewer count there (us,
+// two passes and sweep): 1.0 M pairs, 1,000 queries x 1,000 x 8 f64, 29 matches
+// each: 120 and 131; 100 x 10,000 x 4 f64, 6 to 3,225 matches: 75 to 346 and 75
+// to 365; 2.0 M, 50 x 40,000 x 16 f32, 5 to 12,000: 89 to 381 and 79 to 397.  From
+// 3.0 M on the sweep is ahead at any number of matches: 212 x 14,151 x 21 f32, 5
+// to 3,999: 114 to 506 and 86 to 489; 1,000 x 3,000 x 32 f32, 5 to 886: 140 to 515 and
+// 110 to 504; 3 x 1,000,000 x 8 f64, 5 to 50,000: 202 to 363 and 131 to 329.
 constexpr double kSweepMinPairs = 3.5e6;
 
-template <typename T>
+// The candidate lists of a sweep: `lists` per query, each with room for cap
+// entries, or (second sweep) from where `starts` says, kNoPlace for the queries
+// that take no part.
+struct RadiusLists {
+  uint32_t* idx;
+  uint32_t* count;   // q x lists: candidates, after resolve matches
+  uint32_t* unsure;  // q x lists
+  const uint64_t* starts;
+  int lists;
+  int64_t cap;
+  __device__ __forceinline__ int64_t at(int64_t qi, int l) const {
+    return starts ? static_cast<int64_t>(starts[qi * lists + l]) : (qi * lists + l) * cap;
+  }
+  __device__ __forceinline__ bool takes(int64_t qi) const { return !starts || starts[qi * lists] != kNoPlace; }
+};
+
+// sure: sums up to it are inside the radius.
+template <typename T, bool SECOND>
 __global__ __launch_bounds__(kMT, 2) void radius_sweep_kernel(
     const T* __restrict__ rows, int64_t n, int ld, int d, const double* __restrict__ y2m,
     const T* __restrict__ queries, int64_t q, const double* __restrict__ x2m, Bound64 bd,
-    double bound, int64_t tiles, int64_t per, int lists, int64_t cap, uint32_t* __restrict__ idx,
-    uint32_t* __restrict__ count) {
+    double bound, double sure, int64_t tiles, int64_t per, RadiusLists out) {
   __shared__ MSmem sm;
   const MLane ml;
   const int64_t nqt = (q + kMQ - 1) / kMQ;
@@ -196,87 +225,122 @@ __global__ __launch_bounds__(kMT, 2) void radius_sweep_kernel(
     const int64_t te = min(tiles, tb + (end - pos));
     const int list = static_cast<int>(blockIdx.x - qt * tiles / per);
     const int64_t q0 = qt * kMQ;
-    double th[2];
-    uint32_t cnt[2] = {0u, 0u};  // the same in all four lanes of a column
+    pos += te - tb;
+    double th[2], x2[2];
+    int64_t at[2] = {0, 0};
+    uint32_t cnt[2] = {0u, 0u}, uns[2] = {0u, 0u};  // the same in all four lanes of a column
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int64_t qi = q0 + ml.query_of(j);
-      const double x2 = qi < q ? x2m[qi] : INFINITY;
-      th[j] = x2 < INFINITY ? acc_threshold(bd, bound, x2) : -INFINITY;
+      x2[j] = qi < q && (!SECOND || out.takes(qi)) ? x2m[qi] : INFINITY;
+      th[j] = x2[j] < INFINITY ? acc_threshold(bd, bound, x2[j]) : -INFINITY;
+      if (x2[j] < INFINITY) at[j] = out.at(qi, list);
     }
+    if (SECOND && !__syncthreads_or(x2[0] < INFINITY || x2[1] < INFINITY)) continue;
     mfma64_sweep<T, false>(sm, rows, n, ld, d, y2m, queries, q, q0, 0, tb, te,
                            [&](int64_t t, MAcc& acc, int par) {
-      tile_hits(ml, acc, th, sm.y2[par], [&](int, int j, int, int rl, bool hit, uint64_t m) {
+      tile_hits(ml, acc, th, sm.y2[par], [&](int i, int j, int v, int rl, bool hit, uint64_t m) {
         m &= ml.column();
         const uint32_t c = cnt[j] + __popcll(m & ml.below());
-        if (hit && static_cast<int64_t>(c) < cap)
-          idx[((q0 + ml.query_of(j)) * lists + list) * cap + c] = static_cast<uint32_t>(t * kMR + rl);
+        if (hit && (SECOND || static_cast<int64_t>(c) < out.cap))
+          out.idx[at[j] + c] = static_cast<uint32_t>(t * kMR + rl);
         cnt[j] += __popcll(m);
+        if (!SECOND) {
+          const double u = sum_upper(bd, acc[i][j][v] + x2[j], x2[j] + sm.y2[par][rl]);
+          uns[j] += __popcll(__ballot(hit && !(u <= sure)) & ml.column());
+        }
       });
     });
+    if (!SECOND) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int64_t qi = q0 + ml.query_of(j);
-      if (ml.lg == 0 && qi < q) count[qi * lists + list] = cnt[j];
+      for (int j = 0; j < 2; ++j) {
+        const int64_t qi = q0 + ml.query_of(j);
+        if (ml.lg == 0 && qi < q) {
+          out.count[qi * out.lists + list] = cnt[j];
+          out.unsure[qi * out.lists + list] = uns[j];
+        }
+      }
     }
-    pos += te - tb;
     __syncthreads();  // the sweep's LDS is staged anew
   }
 }
 
+// total: the candidates of a query whose lists overflowed, else 0.
+constexpr int kResolveThreads = 256;
 template <typename T>
-__global__ __launch_bounds__(64) void radius_resolve_kernel(
+__global__ __launch_bounds__(kResolveThreads) void radius_resolve_kernel(
     const T* __restrict__ rows, int ld, const T* __restrict__ queries, int64_t q, double radius,
-    int lists, int64_t cap, uint32_t* __restrict__ idx, const uint32_t* __restrict__ count,
-    uint32_t* __restrict__ matches) {
-  extern __shared__ __align__(16) uint32_t start[];  // lists + 1
-  const int lane = threadIdx.x;
+    RadiusLists ls, uint32_t* __restrict__ matches, uint32_t* __restrict__ total) {
+  __shared__ uint32_t s_sum[kResolveThreads / 64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
   const int64_t qi = blockIdx.x;
-  uint32_t acc = 0;
-  bool over = false;
-  for (int l0 = 0; l0 < lists; l0 += 64) {
-    const uint32_t c = l0 + lane < lists ? count[qi * lists + l0 + lane] : 0u;
-    over = over || static_cast<int64_t>(c) > cap;
-    uint32_t inc = c;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const uint32_t up = __shfl_up(inc, o);
-      if (lane >= o) inc += up;
-    }
-    if (l0 + lane < lists) start[l0 + lane] = acc + inc - c;
-    acc += __shfl(inc, 63);
-  }
-  if (lane == 0) start[lists] = acc;
-  if (__ballot(over) != 0) {
-    if (lane == 0) matches[qi] = kUnresolved;
+  uint32_t* count = ls.count + qi * ls.lists;
+  if (!ls.takes(qi)) {
+    if (threadIdx.x == 0) matches[qi] = kUnresolved;
     return;
   }
-  __syncthreads();
-  uint32_t* mine = idx + qi * lists * cap;
-  uint32_t found = 0;
-  for (uint32_t e0 = 0; e0 < acc; e0 += 64) {
-    const uint32_t e = e0 + lane;
-    bool match = false;
-    uint32_t row = 0;
-    if (e < acc) {
-      int lo = 0, hi = lists;  // the last list that starts at or below e
-      while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (start[mid] <= e)
-          lo = mid;
-        else
-          hi = mid;
-      }
-      row = mine[lo * cap + (e - start[lo])];
-      match = __builtin_sqrt(exact_sum<T, kEuclid>(queries + qi * ld, rows + static_cast<int64_t>(row) * ld, ld)) <= radius;
+  // the sum over the workgroup's threads, in thread 0
+  auto sum = [&](uint32_t v) {
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
+    if (lane == 0) s_sum[wave] = v;
+    __syncthreads();
+    if (threadIdx.x == 0)
+      for (int w = 1; w < waves; ++w) v += s_sum[w];
+    return v;
+  };
+  if (!ls.starts) {
+    uint32_t all = 0;
+    bool over = false;
+    for (int l = threadIdx.x; l < ls.lists; l += blockDim.x) {
+      const uint32_t c = count[l];
+      all += c;
+      over = over || static_cast<int64_t>(c) > ls.cap;
     }
-    // to the front: entry e lies at or past offset e, so no entry that is
-    // still to be read is overwritten
-    const uint64_t m = __ballot(match);
-    if (match) mine[found + __popcll(m & ((uint64_t(1) << lane) - 1))] = row;
-    found += static_cast<uint32_t>(__popcll(m));
+    if (__syncthreads_or(over)) {
+      // the counts stay those of the sweep: a second one goes by them
+      all = sum(all);
+      if (threadIdx.x == 0) {
+        matches[qi] = kUnresolved;
+        total[qi] = all;
+      }
+      return;
+    }
   }
-  if (lane == 0) matches[qi] = found;
+  uint32_t found = 0;
+  for (int l0 = 64 * wave; l0 < ls.lists; l0 += 64 * waves) {  // lane = list
+    const bool in = l0 + lane < ls.lists;
+    uint32_t c = in ? count[l0 + lane] : 0u;
+    uint64_t open = __ballot(in && ls.unsure[qi * ls.lists + l0 + lane] != 0u);
+    while (open) {  // the whole wavefront takes one list
+      const int src = __builtin_ctzll(open);
+      open &= open - 1;
+      const uint32_t m = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(c), src));
+      uint32_t* mine = ls.idx + ls.at(qi, l0 + src);
+      uint32_t kept = 0;
+      for (uint32_t e0 = 0; e0 < m; e0 += 64) {
+        bool match = false;
+        uint32_t row = 0;
+        if (e0 + lane < m) {
+          row = mine[e0 + lane];
+          match = __builtin_sqrt(exact_sum<T, kEuclid>(queries + qi * ld, rows + static_cast<int64_t>(row) * ld, ld)) <= radius;
+        }
+        // to the front: no entry that is still to be read is overwritten
+        const uint64_t b = __ballot(match);
+        if (match) mine[kept + __popcll(b & ((uint64_t(1) << lane) - 1))] = row;
+        kept += static_cast<uint32_t>(__popcll(b));
+      }
+      if (lane == src) {
+        c = kept;
+        count[l0 + lane] = kept;
+      }
+    }
+    found += c;
+  }
+  found = sum(found);
+  if (threadIdx.x != 0) return;
+  matches[qi] = found;
+  if (total) total[qi] = 0u;
 }
 
 __global__ void radius_mark_kernel(const uint32_t* __restrict__ list,
@@ -287,24 +351,78 @@ __global__ void radius_mark_kernel(const uint32_t* __restrict__ list,
     matches[list[i]] = kUnresolved;
 }
 
+// Where the lists of a second sweep start: base[qi] (kNoPlace: takes no part),
+// one list after another.  One wavefront per query.
+__global__ __launch_bounds__(64) void radius_starts_kernel(const uint64_t* __restrict__ base,
+                                                           const uint32_t* __restrict__ count, int lists,
+                                                           uint64_t* __restrict__ starts) {
+  const int lane = threadIdx.x;
+  const int64_t qi = blockIdx.x;
+  uint64_t at = base[qi];
+  for (int l0 = 0; l0 < lists; l0 += 64) {
+    const uint32_t c = l0 + lane < lists ? count[qi * lists + l0 + lane] : 0u;
+    uint32_t inc = c;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t up = __shfl_up(inc, o);
+      if (lane >= o) inc += up;
+    }
+    if (l0 + lane < lists) starts[qi * lists + l0 + lane] = at == kNoPlace ? kNoPlace : at + inc - c;
+    if (at != kNoPlace) at += __shfl(inc, 63);
+  }
+}
+
+// A wavefront takes a query's matches 64 at a time, every gridDim.y-th 64 of
+// them (few queries with many matches would leave the chip idle otherwise).
+// Its rows go through LDS by whole wavefronts (metric.hpp).
 template <typename T>
-__global__ __launch_bounds__(256) void radius_emit_kernel(
-    const T* __restrict__ rows, int ld, const T* __restrict__ queries, int64_t q, int64_t per_query,
-    const uint32_t* __restrict__ idx, const uint32_t* __restrict__ matches,
-    const uint64_t* __restrict__ offsets, int64_t* __restrict__ out_idx,
-    double* __restrict__ out_dist) {
-  const int lane = threadIdx.x & 63;
-  const int64_t qi = static_cast<int64_t>(blockIdx.x) * (blockDim.x / 64) + (threadIdx.x >> 6);
-  if (qi >= q) return;
+__global__ __launch_bounds__(64) void radius_emit_kernel(
+    const T* __restrict__ rows, int ld, const T* __restrict__ queries, RadiusLists ls,
+    const uint32_t* __restrict__ matches, const uint64_t* __restrict__ offsets,
+    int64_t* __restrict__ out_idx, double* __restrict__ out_dist, int staged) {
+  // the query row (staged), then the lists' starts (lists + 1)
+  extern __shared__ __align__(16) unsigned char emit_smem[];
+  __shared__ __align__(16) unsigned char tile[kSumTileBytes];
+  T* qrow = reinterpret_cast<T*>(emit_smem);
+  uint32_t* start = reinterpret_cast<uint32_t*>(qrow + (staged ? ld : 0));
+  const int lane = threadIdx.x;
+  const int64_t qi = blockIdx.x;
   const uint32_t c = matches[qi];
-  if (c == kUnresolved) return;
+  if (c == kUnresolved || 64u * blockIdx.y >= c) return;
+  if (staged)
+    for (int j = lane; j < ld; j += 64) qrow[j] = queries[qi * ld + j];
+  uint32_t acc = 0;
+  for (int l0 = 0; l0 < ls.lists; l0 += 64) {
+    const uint32_t v = l0 + lane < ls.lists ? ls.count[qi * ls.lists + l0 + lane] : 0u;
+    uint32_t inc = v;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t up = __shfl_up(inc, o);
+      if (lane >= o) inc += up;
+    }
+    if (l0 + lane < ls.lists) start[l0 + lane] = acc + inc - v;
+    acc += __shfl(inc, 63);
+  }
+  __syncthreads();
   const uint64_t o = offsets[qi];
-  for (uint32_t j = lane; j < c; j += 64) {
-    const uint32_t row = idx[qi * per_query + j];
-    out_idx[o + j] = row;
-    if (out_dist)
-      out_dist[o + j] =
-          __builtin_sqrt(exact_sum<T, kEuclid>(queries + qi * ld, rows + static_cast<int64_t>(row) * ld, ld));
+  for (uint64_t e0 = 64u * blockIdx.y; e0 < c; e0 += 64u * gridDim.y) {
+    const uint32_t e = static_cast<uint32_t>(min(e0 + lane, static_cast<uint64_t>(c) - 1));
+    int lo = 0, hi = ls.lists;  // the last list that starts at or below e
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (start[mid] <= e)
+        lo = mid;
+      else
+        hi = mid;
+    }
+    const uint32_t row = ls.idx[ls.at(qi, lo) + (e - start[lo])];
+    const bool mine = e0 + lane < c;
+    if (mine) out_idx[o + e] = row;
+    if (out_dist) {
+      const double sum = staged ? wave_exact_sums<T, kEuclid>(qrow, rows, row, ld, tile)
+                                : exact_sum<T, kEuclid>(queries + qi * ld, rows + static_cast<int64_t>(row) * ld, ld);
+      if (mine) out_dist[o + e] = __builtin_sqrt(sum);
+    }
   }
 }
 
@@ -344,6 +462,8 @@ int run_radius_f64(const sc_index* ix, const T* dq, int64_t q, double radius, do
   const int ld = static_cast<int>(ix->ld), d = static_cast<int>(ix->d);
   const T* rows = static_cast<const T*>(ix->rows);
   const Bound64 bd = bound64<T>(ld);
+  // sqrt(S) <= radius for every S up to this, whatever the roundings
+  const double sure = radius * radius * (1.0 - 1e-12);
   DevBuf local;
   const double* y2m = nullptr;
   if (int rc = ensure_norms64(const_cast<sc_index*>(ix), local, &y2m, s)) return rc;
@@ -352,32 +472,34 @@ int run_radius_f64(const sc_index* ix, const T* dq, int64_t q, double radius, do
   // two workgroups per CU fit; each takes the same number of tiles
   const int64_t per = std::max<int64_t>(1, (nqt * tiles + 511) / 512);
   const int lists = static_cast<int>(std::min<int64_t>((tiles + per - 1) / per + 1, tiles));
-  const int64_t entries = std::max(kListMin, std::min(kListMax, kListTotal / q));
+  const int64_t entries = std::max(kListMin, kListTotal / q);
   const int64_t cap = std::max<int64_t>(16, std::min<int64_t>(per * kMR, entries / lists));
-  DevBuf x2m, olist, flags, idx, cnt, mat;
+  const int64_t words = q * lists;
+  DevBuf x2m, olist, flags, idx, cnt, mat, tot;
   SC_HIP(x2m.alloc(sizeof(double) * q, s));
   SC_HIP(olist.alloc(sizeof(uint32_t) * q, s));
   SC_HIP(flags.alloc(16, s));
-  SC_HIP(idx.alloc(sizeof(uint32_t) * q * lists * cap, s));
-  SC_HIP(cnt.alloc(sizeof(uint32_t) * q * lists, s));
+  SC_HIP(idx.alloc(sizeof(uint32_t) * words * cap, s));
+  SC_HIP(cnt.alloc(sizeof(uint32_t) * 2 * words, s));  // count | unsure
   SC_HIP(mat.alloc(sizeof(uint32_t) * q, s));
-  const int64_t words = q * lists;
-  hipLaunchKernelGGL(radius_zero_kernel, dim3(static_cast<unsigned>(std::min<int64_t>(1024, (words + 255) / 256))),
-                     dim3(256), 0, s, cnt.as<uint32_t>(), words);
+  SC_HIP(tot.alloc(sizeof(uint32_t) * q, s));
+  const RadiusLists ls{idx.as<uint32_t>(), cnt.as<uint32_t>(), cnt.as<uint32_t>() + words, nullptr, lists, cap};
+  hipLaunchKernelGGL(radius_zero_kernel, dim3(static_cast<unsigned>(std::min<int64_t>(1024, (2 * words + 255) / 256))),
+                     dim3(256), 0, s, cnt.as<uint32_t>(), 2 * words);
   hipLaunchKernelGGL(radius_zero_kernel, dim3(1), dim3(64), 0, s, flags.as<uint32_t>(), int64_t{4});
   if (int rc = query_norms64<T>(dq, q, ld, x2m.as<double>(), olist.as<uint32_t>(),
                                 flags.as<uint32_t>(), s))
     return rc;
+  const dim3 groups(static_cast<unsigned>((nqt * tiles + per - 1) / per));
+  const dim3 resolve_threads(static_cast<unsigned>(std::min(kResolveThreads, (lists + 63) / 64 * 64)));
   {
     ProfScope ps("radius_sweep", s);
-    hipLaunchKernelGGL(radius_sweep_kernel<T>, dim3(static_cast<unsigned>((nqt * tiles + per - 1) / per)),
-                       dim3(kMT), 0, s, rows, n, ld, d, y2m, dq, q, x2m.as<double>(), bd, bound, tiles,
-                       per, lists, cap, idx.as<uint32_t>(), cnt.as<uint32_t>());
+    hipLaunchKernelGGL((radius_sweep_kernel<T, false>), groups, dim3(kMT), 0, s, rows, n, ld, d, y2m, dq, q,
+                       x2m.as<double>(), bd, bound, sure, tiles, per, ls);
     SC_HIP(hipGetLastError());
   }
-  hipLaunchKernelGGL(radius_resolve_kernel<T>, dim3(static_cast<unsigned>(q)), dim3(64),
-                     sizeof(uint32_t) * (lists + 1), s, rows, ld, dq, q, radius, lists, cap,
-                     idx.as<uint32_t>(), cnt.as<uint32_t>(), mat.as<uint32_t>());
+  hipLaunchKernelGGL(radius_resolve_kernel<T>, dim3(static_cast<unsigned>(q)), resolve_threads, 0, s, rows, ld,
+                     dq, q, radius, ls, mat.as<uint32_t>(), tot.as<uint32_t>());
   hipLaunchKernelGGL(radius_mark_kernel, dim3(4), dim3(256), 0, s, olist.as<uint32_t>(),
                      flags.as<uint32_t>(), mat.as<uint32_t>());
   SC_HIP(hipGetLastError());
@@ -386,12 +508,62 @@ int run_radius_f64(const sc_index* ix, const T* dq, int64_t q, double radius, do
   std::vector<int64_t> over;
   for (int64_t i = 0; i < q; ++i)
     if (hm[i] == kUnresolved) over.push_back(i);
+  // the second sweep's lists, and what is left to the two passes
+  DevBuf idx2, base2, start2, mat2;
+  RadiusLists ls2{};
+  std::vector<uint32_t> hm2;
+  if (!over.empty()) {
+    std::vector<uint32_t> ht(static_cast<size_t>(q));
+    if (int rc = download_staged(ht.data(), tot.p, sizeof(uint32_t) * ht.size(), s)) return rc;
+    std::vector<uint64_t> base(static_cast<size_t>(q), kNoPlace);
+    std::vector<int64_t> rest;
+    uint64_t at = 0;
+    for (const int64_t i : over) {
+      // (no candidates: a norm out of the bound's range)
+      if (ht[i] == 0 || at + ht[i] > kSecondMax) {
+        rest.push_back(i);
+        continue;
+      }
+      base[i] = at;
+      at += ht[i];
+    }
+    // (lists that do not fit the memory: the two passes)
+    if (at > 0 && idx2.alloc(sizeof(uint32_t) * at, s) == hipSuccess) {
+      SC_HIP(base2.alloc(sizeof(uint64_t) * q, s));
+      SC_HIP(start2.alloc(sizeof(uint64_t) * words, s));
+      SC_HIP(mat2.alloc(sizeof(uint32_t) * q, s));
+      if (int rc = upload_staged(base2.p, base.data(), sizeof(uint64_t) * q, s)) return rc;
+      ls2 = ls;
+      ls2.idx = idx2.as<uint32_t>();
+      ls2.starts = start2.as<uint64_t>();
+      hipLaunchKernelGGL(radius_starts_kernel, dim3(static_cast<unsigned>(q)), dim3(64), 0, s, base2.as<uint64_t>(),
+                         cnt.as<uint32_t>(), lists, start2.as<uint64_t>());
+      {
+        ProfScope ps("radius_sweep", s);
+        hipLaunchKernelGGL((radius_sweep_kernel<T, true>), groups, dim3(kMT), 0, s, rows, n, ld, d, y2m, dq, q,
+                           x2m.as<double>(), bd, bound, sure, tiles, per, ls2);
+      }
+      hipLaunchKernelGGL(radius_resolve_kernel<T>, dim3(static_cast<unsigned>(q)), resolve_threads, 0, s, rows,
+                         ld, dq, q, radius, ls2, mat2.as<uint32_t>(), static_cast<uint32_t*>(nullptr));
+      SC_HIP(hipGetLastError());
+      hm2.resize(static_cast<size_t>(q));
+      if (int rc = download_staged(hm2.data(), mat2.p, sizeof(uint32_t) * hm2.size(), s)) return rc;
+      for (const int64_t i : over)
+        if (base[i] != kNoPlace) hm[i] = hm2[i];
+      over.swap(rest);
+    } else if (at > 0) {
+      (void)hipGetLastError();
+    }
+  }
+  if (static_cast<int64_t>(over.size()) == q)
+    return run_radius<T, kEuclid>(ix, dq, q, 2.0, radius, res, want_dist, false, s);
   sc_radius_result sub;
   if (!over.empty())
     if (int rc = search_subset<T, kEuclid>(ix, dq, over, 2.0, radius, &sub, want_dist, s)) return rc;
   res->q = static_cast<size_t>(q);
   res->offsets.resize(static_cast<size_t>(q) + 1);
   uint64_t total = 0;
+  uint32_t most = 0;  // matches of a query that the lists hold
   size_t next = 0;
   for (int64_t i = 0; i < q; ++i) {
     res->offsets[i] = total;
@@ -400,6 +572,7 @@ int run_radius_f64(const sc_index* ix, const T* dq, int64_t q, double radius, do
       ++next;
     } else {
       total += hm[i];
+      most = std::max(most, hm[i]);
     }
   }
   res->offsets[q] = total;
@@ -411,10 +584,18 @@ int run_radius_f64(const sc_index* ix, const T* dq, int64_t q, double radius, do
   if (int rc = upload_staged(off.p, res->offsets.data(), sizeof(uint64_t) * (q + 1), s)) return rc;
   SC_HIP(oi.alloc(sizeof(int64_t) * total, s));
   if (want_dist) SC_HIP(od.alloc(sizeof(double) * total, s));
-  hipLaunchKernelGGL(radius_emit_kernel<T>, dim3(static_cast<unsigned>((q + 3) / 4)), dim3(256), 0, s,
-                     rows, ld, dq, q, static_cast<int64_t>(lists) * cap, idx.as<uint32_t>(),
-                     mat.as<uint32_t>(), off.as<uint64_t>(), oi.as<int64_t>(),
-                     want_dist ? od.as<double>() : nullptr);
+  // wavefronts for the whole chip, as far as there are matches for them
+  const unsigned split = static_cast<unsigned>(
+      std::max<int64_t>(1, std::min<int64_t>((int64_t{most} + 63) / 64, (16384 + q - 1) / q)));
+  const int staged = want_dist && sizeof(T) * ld <= 32768 ? 1 : 0;
+  auto emit = [&](const RadiusLists& l, const DevBuf& m) {
+    hipLaunchKernelGGL(radius_emit_kernel<T>, dim3(static_cast<unsigned>(q), split), dim3(64),
+                       (staged ? sizeof(T) * ld : 0) + sizeof(uint32_t) * (lists + 1), s, rows, ld, dq, l,
+                       m.as<uint32_t>(), off.as<uint64_t>(), oi.as<int64_t>(),
+                       want_dist ? od.as<double>() : nullptr, staged);
+  };
+  emit(ls, mat);
+  if (!hm2.empty()) emit(ls2, mat2);
   SC_HIP(hipGetLastError());
   if (int rc = download_staged(res->idx.data(), oi.p, sizeof(int64_t) * total, s)) return rc;
   if (want_dist)
