@@ -872,12 +872,21 @@ int kmeans_assign_launch(const sc_index* ix, const void* rows, int64_t n, const 
     SC_HIP(hipGetLastError());                                                                    \
     return SC_OK;                                                                                 \
   }
-  // One thread per row where it is the faster form: rows of up to 48 values
-  // (200,000 x 40, k = 32: 48 against 89 us), or 64 with few centroids for
-  // the tile's 64 (1,000,000 x 64, k = 64: 605 against 462 us; its cost goes
-  // with k, the tile's with ceil(k / 64)), and enough rows for the chip
-  // (20,000 x 6, k = 130: 35 against 26 us).
-  if (n >= 65536 || k <= 32) {
+  // One thread per row where it is the faster form.  A wavefront's chain over
+  // the centroids takes its time however few wavefronts there are (0.036 ld us
+  // per centroid up to about 200,000 rows), the tile's goes with the rows and
+  // with each started 64 centroids.  `each` is the number of centroids per
+  // started 64 at which the two take the same, fitted to 5,000 to 1,000,000 rows
+  // (f64, us, rows and tile: 5,000 x 16, k = 8: 9 and 10, k = 24: 17 and 10;
+  // 65,536 x 16, k = 24: 16 and 17, k = 64: 34 and 18, k = 1,000: 589 and 182;
+  // 100,000 x 48, k = 32: 49 and 54, k = 64: 112 and 55; 300,000 x 48, k = 48: 115
+  // and 125, k = 64: 165 and 127; 1,000,000 x 32, k = 64: 204 and 257).  Rows of
+  // 64 values: up to 32 centroids (1,000,000 x 64, k = 64: 605 and 462).
+  const int64_t ld = static_cast<int64_t>(ix->ld), filled = (int64_t{k} + 63) / 64;
+  int64_t each = (n + 25500) / 3900;
+  if (filled == 1) each = std::max(14 - ld / 8 + n / 6000, ld <= 32 ? (n - 6000) / 2500 : each);
+  if (n < 9000 * ld && !(filled == 1 && ld <= 32)) each = std::min<int64_t>(each, 48);
+  if (k <= filled * std::min<int64_t>(each, 64)) {
     SC_ASSIGN_ROWS(1) SC_ASSIGN_ROWS(2) SC_ASSIGN_ROWS(3)
     if (k <= 32) {
       SC_ASSIGN_ROWS(4)
