@@ -33,6 +33,7 @@
 
 #include <algorithm>
 #include <cfloat>
+#include <cmath>
 #include <string>
 #include <vector>
 
@@ -694,8 +695,8 @@ __global__ void kmeans_state_init_kernel(KmState* st) {
 // the row unless it ends within delta = 4 (n + 64) 2^-53 sum of the cutoff
 // on either side of that row (about one round in 10^4 at a million rows):
 // then, and when a sum is not finite, the round is left to the host, which
-// folds in row order.  The draws u do not depend on the data, so all rounds
-// are queued without a host round trip.  (100,000 x 16, k = 10: 0.25 ms, and
+// folds in row order.  The draws u do not depend on the data, so rounds are
+// queued one after another, with two host round trips in all.  (100,000 x 16, k = 10: 0.25 ms, and
 // 1,000,000 x 64, k = 64: 4.0; downloading and folding every round took 1.24
 // and 119.)
 constexpr int kPPRows = 1024;  // rows per partial sum
@@ -704,16 +705,17 @@ struct PPState {
   uint32_t round;  // the round the host has to decide, or 0
 };
 
+// chosen: the centre's row (negative: pick[label]).
 template <typename T>
 __global__ __launch_bounds__(kPPRows) void kmeanspp_round_kernel(
-    const T* __restrict__ rows, int64_t n, int ld, const int64_t* __restrict__ pick,
+    const T* __restrict__ rows, int64_t n, int ld, const int64_t* __restrict__ pick, int64_t chosen,
     double* __restrict__ dmin, uint32_t* __restrict__ y, uint32_t label, double* __restrict__ part,
     const PPState* __restrict__ st) {
   if (st->round) return;
   constexpr int PV = 16 / sizeof(T);
   typedef T Piece __attribute__((ext_vector_type(PV)));
   __shared__ double s_wave[kPPRows / 64];
-  const Piece* cen = reinterpret_cast<const Piece*>(rows + pick[label] * ld);
+  const Piece* cen = reinterpret_cast<const Piece*>(rows + (chosen >= 0 ? chosen : pick[label]) * ld);
   const int64_t i = static_cast<int64_t>(blockIdx.x) * kPPRows + threadIdx.x;
   double best = 0.0;
   if (i < n) {
@@ -1300,7 +1302,7 @@ int sc_kmeans_plus_plus(const sc_index* index, size_t k, int has_seed, uint64_t 
   // kmeans.rs:358-362: first centre is a uniformly drawn row; then one draw
   // per further centre
   std::vector<double> draws(k, 0.0);
-  const int64_t pick0 = static_cast<int64_t>(rng.gen_range(static_cast<uint64_t>(n)));
+  int64_t chosen = static_cast<int64_t>(rng.gen_range(static_cast<uint64_t>(n)));  // by the host
   for (size_t j = 1; j < k; ++j) draws[j] = rng.gen_f64();
   const int64_t nb = (n + kPPRows - 1) / kPPRows;
   DevBuf ddraw, dpick, dmin, dy, part, dst;
@@ -1313,44 +1315,66 @@ int sc_kmeans_plus_plus(const sc_index* index, size_t k, int has_seed, uint64_t 
   SC_HIP(hipMemsetAsync(dy.p, 0, sizeof(uint32_t) * n, s));
   SC_HIP(hipMemsetAsync(dst.p, 0, sizeof(PPState), s));
   if (int rc = upload_staged(ddraw.p, draws.data(), sizeof(double) * k, s)) return rc;
-  if (int rc = upload_staged(dpick.p, &pick0, sizeof(int64_t), s)) return rc;
-  auto round = [&](size_t label) -> int {
+  auto round = [&](size_t label, int64_t row) -> int {
+    ProfScope ps("kmeanspp_round", s);
     if (index->dtype == SC_F64)
       hipLaunchKernelGGL(kmeanspp_round_kernel<double>, dim3(static_cast<unsigned>(nb)), dim3(kPPRows), 0,
                          s, static_cast<const double*>(index->rows), n, static_cast<int>(index->ld),
-                         dpick.as<int64_t>(), dmin.as<double>(), dy.as<uint32_t>(),
+                         dpick.as<int64_t>(), row, dmin.as<double>(), dy.as<uint32_t>(),
                          static_cast<uint32_t>(label), part.as<double>(), dst.as<PPState>());
     else
       hipLaunchKernelGGL(kmeanspp_round_kernel<float>, dim3(static_cast<unsigned>(nb)), dim3(kPPRows), 0,
                          s, static_cast<const float*>(index->rows), n, static_cast<int>(index->ld),
-                         dpick.as<int64_t>(), dmin.as<double>(), dy.as<uint32_t>(),
+                         dpick.as<int64_t>(), row, dmin.as<double>(), dy.as<uint32_t>(),
                          static_cast<uint32_t>(label), part.as<double>(), dst.as<PPState>());
     SC_HIP(hipGetLastError());
     return SC_OK;
   };
-  // rounds first .. k: round j labels rows against centre j - 1 and picks
-  // centre j; the last only labels
-  for (size_t first = 1;;) {
-    for (size_t j = first; j <= k; ++j) {
-      if (int rc = round(j - 1)) return rc;
-      if (j < k) {
+  // round j labels rows against centre j - 1 and picks centre j; the last
+  // (round k) only labels.  Sixteen are queued at once, then all that are left;
+  // those after a round that the host has to decide are empty launches, so the
+  // next ones are queued one, two, four at a time, and one by one, with no pick
+  // on the device, while the costs' sum is not finite (two rows whose distance
+  // overflows or is NaN: k = 64 over 5,000 x 8 such rows took 17.6 ms with all
+  // rounds queued again each time, 2.0 now).
+  size_t run = 16;
+  bool host = false;
+  std::vector<double> hd;
+  for (size_t first = 1; first <= k;) {
+    const size_t last = first + std::min(run, k - first + 1) - 1;
+    for (size_t j = first; j <= last; ++j) {
+      if (int rc = round(j - 1, j == first ? chosen : -1)) return rc;
+      if (j < k && !host) {
         hipLaunchKernelGGL(kmeanspp_pick_kernel, dim3(1), dim3(kPPRows), 0, s, dmin.as<double>(), n,
                            part.as<double>(), nb, ddraw.as<double>(), static_cast<uint32_t>(j),
                            dpick.as<int64_t>(), dst.as<PPState>());
         SC_HIP(hipGetLastError());
       }
     }
-    PPState hs{};
-    SC_HIP(hipMemcpyAsync(&hs, dst.p, sizeof(hs), hipMemcpyDeviceToHost, s));
-    SC_HIP(hipStreamSynchronize(s));
-    if (hs.round == 0) break;
+    size_t at_round = first;
+    if (host) {
+      if (first == k) break;
+    } else {
+      PPState hs{};
+      SC_HIP(hipMemcpyAsync(&hs, dst.p, sizeof(hs), hipMemcpyDeviceToHost, s));
+      SC_HIP(hipStreamSynchronize(s));
+      if (hs.round == 0) {
+        run = first == 1 ? k : 2 * run;
+        chosen = -1;
+        first = last + 1;
+        continue;
+      }
+      at_round = hs.round;
+      SC_HIP(hipMemsetAsync(dst.p, 0, sizeof(PPState), s));
+    }
     // the host decides this centre as the reference does
-    std::vector<double> hd(static_cast<size_t>(n));
-    if (int rc = download_staged(hd.data(), dmin.p, sizeof(double) * n, s)) return rc;
+    hd.resize(static_cast<size_t>(n));
+    SC_HIP(hipMemcpyAsync(hd.data(), dmin.p, sizeof(double) * n, hipMemcpyDeviceToHost, s));
+    SC_HIP(hipStreamSynchronize(s));
     // kmeans.rs:381-394: sequential sum, cutoff, linear cumulative scan
     double sum = 0.0;
     for (int64_t i = 0; i < n; ++i) sum += hd[i];
-    const double cutoff = draws[hs.round] * sum;
+    const double cutoff = draws[at_round] * sum;
     double cost = 0.0;
     int64_t at = 0;
     while (at < n) {
@@ -1361,9 +1385,10 @@ int sc_kmeans_plus_plus(const sc_index* index, size_t k, int has_seed, uint64_t 
     // the reference would index past the end here (only reachable with a
     // NaN sum); stay on the last row instead
     if (at >= n) at = n - 1;
-    if (int rc = upload_staged(dpick.as<int64_t>() + hs.round, &at, sizeof(int64_t), s)) return rc;
-    SC_HIP(hipMemsetAsync(dst.p, 0, sizeof(PPState), s));
-    first = hs.round + 1;
+    chosen = at;
+    host = !std::isfinite(sum);
+    run = 1;
+    first = at_round + 1;
   }
   return download_staged(labels, dy.p, sizeof(uint32_t) * n, s);
 }
