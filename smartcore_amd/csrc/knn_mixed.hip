@@ -953,8 +953,7 @@ __global__ __launch_bounds__(kLevelThreads) void mixed_level_kernel(
   float kth = tid < 64 ? lane_value(b, k - 1) : 0.0f;
   const uint32_t total = start[nu];
   for (uint32_t e0 = 0; e0 < total;) {
-    // whole pairs while they fit (a longer one is left unmerged: its query
-    // goes to the serial kernel)
+    // whole pairs while they fit (a longer one is left to the replay)
     uint32_t m = min(total - e0, static_cast<uint32_t>(kLevelBatch));
     if (pairs && e0 + m < total) {
       const int u = unit_of(e0 + m);
@@ -1015,8 +1014,11 @@ __global__ __launch_bounds__(kLevelThreads) void mixed_level_kernel(
 // The replay, one wavefront per query (the heap lives across its lanes): the
 // candidates of all lists, in row order by now, 64 at a time across the
 // lists; the next 64 are requested before the current ones go through the
-// heap.  Queries whose lists overflowed, or a pair of whose lists could not
-// be merged, go to the serial exact kernel's list.
+// heap.  A pair of more than kLevelBatch entries still lies as its two halves:
+// the t-th of its rows is found by the halving of the split of t between them
+// (a dozen dependent reads per 64 entries, where the whole index would have to
+// be read again otherwise).  Queries whose lists overflowed go to the serial
+// exact kernel's list.
 __global__ __launch_bounds__(64 * kReplayWaves) void mixed_replay_kernel(
     int64_t q, int k, ListLayout lay, const uint32_t* __restrict__ cand_idx,
     const double* __restrict__ cand_S, const uint32_t* __restrict__ cand_count,
@@ -1032,17 +1034,17 @@ __global__ __launch_bounds__(64 * kReplayWaves) void mixed_replay_kernel(
   const int nl = lay.nlists();
   uint32_t* start = replay_smem + w * (nl + 1);
   const uint32_t* cc = cand_count + qi * nl;
-  bool over = false;
+  bool over = false, wide = false;
   uint32_t total = 0;
+  auto unmerged = [](uint32_t a, uint32_t b) {
+    return a != 0u && b != 0u && a + b > static_cast<uint32_t>(kLevelBatch);
+  };
   for (int l0 = 0; l0 < nl; l0 += 64) {
     const int l = l0 + lane;
     const uint32_t c = l < nl ? cc[l] : 0u;
     if (l < nl) {
       over = over || c > static_cast<uint32_t>(lay.cap(l));
-      if (l >= lay.nrun) {
-        const uint32_t o = cc[lay.nrun + ((l - lay.nrun) ^ 1)];
-        over = over || (c != 0u && o != 0u && c + o > static_cast<uint32_t>(kLevelBatch));
-      }
+      if (l >= lay.nrun) wide = wide || unmerged(c, cc[lay.nrun + ((l - lay.nrun) ^ 1)]);
     }
     uint32_t inc = c;
 #pragma unroll
@@ -1057,6 +1059,7 @@ __global__ __launch_bounds__(64 * kReplayWaves) void mixed_replay_kernel(
     if (lane == 0) list[atomicAdd(list_n, 1u)] = static_cast<uint32_t>(qi);
     return;
   }
+  const bool merge = __ballot(wide) != 0;
   if (lane == 0) start[nl] = total;
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -1073,7 +1076,27 @@ __global__ __launch_bounds__(64 * kReplayWaves) void mixed_replay_kernel(
       else
         hi = mid;
     }
-    const int64_t slot = qbase + lay.offset(lo) + (e - start[lo]);
+    int64_t slot = qbase + lay.offset(lo) + (e - start[lo]);
+    if (merge && lo >= lay.nrun) {
+      const int p = lay.nrun + ((lo - lay.nrun) & ~1);
+      const uint32_t na = start[p + 1] - start[p], nb = start[p + 2] - start[p + 1];
+      if (unmerged(na, nb)) {
+        const uint32_t* a = cand_idx + qbase + lay.offset(p);
+        const uint32_t* b = cand_idx + qbase + lay.offset(p + 1);
+        // i: how many of the first t rows are the first half's
+        const uint32_t t = e - start[p];
+        uint32_t i = t > nb ? t - nb : 0u, up = min(t, na);
+        while (i < up) {
+          const uint32_t mid = (i + up) >> 1;
+          if (a[mid] < b[t - 1 - mid])
+            i = mid + 1;
+          else
+            up = mid;
+        }
+        const bool first = i < na && (t - i >= nb || a[i] < b[t - i]);
+        slot = qbase + (first ? lay.offset(p) + i : lay.offset(p + 1) + (t - i));
+      }
+    }
     r = cand_idx[slot];
     v = cand_S[slot];
   };
