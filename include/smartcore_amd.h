@@ -116,7 +116,8 @@ int sc_knn_search(const sc_index* index, const void* queries, size_t q,
 /* Same with queries and outputs in HBM, ordered on `stream` (hipStream_t,
  * NULL = the default stream).  Returns after enqueueing unless an error
  * needs host work; the outputs are valid once the stream reaches the point
- * of the call. */
+ * of the call.  (The first SC_MIXED search of an index prepares its rows and
+ * waits for that.) */
 int sc_knn_search_device(const sc_index* index, const void* d_queries,
                          size_t q, size_t k, sc_metric metric, uint16_t p,
                          sc_mode mode, int64_t* d_idx, double* d_dist,

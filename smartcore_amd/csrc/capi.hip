@@ -718,6 +718,7 @@ int sc_index_destroy(sc_index* index) {
   if (index->rows_bf16) (void)hipFree(index->rows_bf16);
   if (index->norms2) (void)hipFree(index->norms2);
   if (index->norms64) (void)hipFree(index->norms64);
+  if (index->norms64_done) (void)hipEventDestroy(index->norms64_done);
   if (index->rows_q16) (void)hipFree(index->rows_q16);
   if (index->err_q16) (void)hipFree(index->err_q16);
   (void)hipSetDevice(cur);

@@ -118,8 +118,13 @@ struct sc_index {
   double q16_lo, q16_step;
   int q16_state;
   // Lazily built for the FP64 matrix form (guarded by mu): per row, padded to
-  // whole 128-row tiles, a lower bound of the squared norm.
+  // whole 128-row tiles, a lower bound of the squared norm.  norms64_done: the
+  // event after the kernel that writes them, on norms64_stream; norms64_ready:
+  // it has been seen.
   double* norms64;
+  hipEvent_t norms64_done;
+  hipStream_t norms64_stream;
+  bool norms64_ready;
   void* mu;         // std::mutex*
 };
 

@@ -385,12 +385,25 @@ int ensure_norms64(sc_index* ix, DevBuf& local, const double** y2m, hipStream_t 
     SC_HIP(hipGetLastError());
     return SC_OK;
   };
+  const bool capturing = stream_capturing(s);
   std::lock_guard<std::mutex> lk(*static_cast<std::mutex*>(ix->mu));
-  if (ix->norms64) {
+  if (ix->norms64 && !ix->norms64_ready) {
+    // (a query is not an operation of the stream: it is allowed beside a capture)
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool swapped = capturing && hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    if (!capturing || swapped) {
+      ix->norms64_ready = hipEventQuery(ix->norms64_done) == hipSuccess;
+      if (!ix->norms64_ready) (void)hipGetLastError();  // not ready is no error
+    }
+    if (swapped) (void)hipThreadExchangeStreamCaptureMode(&mode);
+  }
+  if (ix->norms64 && (ix->norms64_ready || (!capturing && s == ix->norms64_stream))) {
+    // (a new stream may have got the handle of the one that built them)
+    if (!ix->norms64_ready) SC_HIP(hipStreamWaitEvent(s, ix->norms64_done, 0));
     *y2m = ix->norms64;
     return SC_OK;
   }
-  if (stream_capturing(s)) {
+  if (ix->norms64 || capturing) {
     SC_HIP(local.alloc(sizeof(double) * npad, s));
     if (int rc = launch(local.as<double>())) return rc;
     *y2m = local.as<double>();
@@ -398,17 +411,21 @@ int ensure_norms64(sc_index* ix, DevBuf& local, const double** y2m, hipStream_t 
   }
   double* p = nullptr;
   SC_HIP(hipMalloc(reinterpret_cast<void**>(&p), sizeof(double) * npad));
-  int rc = launch(p);
-  if (rc == SC_OK) {
-    // calls on other streams may follow at once
-    const hipError_t e = hipStreamSynchronize(s);
-    if (e != hipSuccess) rc = hip_fail(e, "row norms");
+  hipEvent_t done = nullptr;
+  hipError_t e = hipEventCreateWithFlags(&done, hipEventDisableTiming);
+  int rc = e == hipSuccess ? launch(p) : hip_fail(e, "row norms");
+  if (rc == SC_OK && (e = hipEventRecord(done, s)) != hipSuccess) {
+    rc = hip_fail(e, "row norms");
+    (void)hipStreamSynchronize(s);  // p is freed below
   }
   if (rc != SC_OK) {
+    if (done) (void)hipEventDestroy(done);
     (void)hipFree(p);
     return rc;
   }
   ix->norms64 = p;
+  ix->norms64_done = done;
+  ix->norms64_stream = s;
   *y2m = p;
   return SC_OK;
 }

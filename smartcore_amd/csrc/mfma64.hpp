@@ -294,8 +294,11 @@ __device__ __forceinline__ void tile_hits(const MLane& ml, const MAcc& acc, cons
 }
 
 // y2m of every row of an index (kMR rows of padding past the last, +inf),
-// built once per index; on a capturing stream, where nothing may be kept or
-// waited for, into `local` for the call.
+// built once per index on the stream of the first call, which does not wait
+// for it.  Until it is complete, calls on other streams build their own into
+// `local` (waiting for it would put them behind all that the first stream has
+// queued), and so do those on a capturing stream, where nothing may be kept or
+// waited for.
 int ensure_norms64(sc_index* ix, DevBuf& local, const double** y2m, hipStream_t s);
 // The same for a call's queries (no padding).  Queries with a finite but too
 // large norm are appended to list (their x2m is +inf, like that of the
