@@ -756,10 +756,13 @@ int sc_dbscan_fit(const sc_index* index, double eps, size_t min_samples, sc_metr
     // the radius search's conservative bound on the sum
     const double bound = eps * eps * (1.0 + 1e-12) + 1e-300;
     // (false for NaN, and for radii that sums overflowing the rows' type pass)
-    if (index->dtype == SC_F64 ? bound < sum_limit<double>() : bound < sum_limit<float>())
-      return index->dtype == SC_F64
-                 ? fit_pairs<double>(index, eps, bound, min_samples, labels, num_classes, s)
-                 : fit_pairs<float>(index, eps, bound, min_samples, labels, num_classes, s);
+    if (index->dtype == SC_F64 ? bound < sum_limit<double>() : bound < sum_limit<float>()) {
+      const int rc = index->dtype == SC_F64
+                         ? fit_pairs<double>(index, eps, bound, min_samples, labels, num_classes, s)
+                         : fit_pairs<float>(index, eps, bound, min_samples, labels, num_classes, s);
+      if (rc != SC_ERR_OUT_OF_MEMORY) return rc;
+      clear_error();  // the neighbour lists may fit
+    }
   }
   sc_radius_result nb;
   // the expansion reads the neighbour rows only, not their distances

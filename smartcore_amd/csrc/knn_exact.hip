@@ -552,8 +552,9 @@ int run_tiled(const sc_index* index, const T* d_queries, int64_t q, int k, doubl
   return SC_OK;
 }
 
-// Euclidian searches come here with k > KMAX_TILED only (knn_f64.hip takes
-// the others), so their scan is not built.
+// Euclidian searches come here with k > KMAX_TILED (knn_f64.hip takes the
+// others), or when what that form keeps beside the rows does not fit the
+// memory, so their scan is not built.
 template <typename T, int M>
 int run_exact(const sc_index* index, const T* d_queries, int64_t q, int k, double p, int64_t* d_idx,
               double* d_dist, uint32_t* d_count, hipStream_t stream, sc_stats* stats) {
@@ -576,7 +577,7 @@ int run_exact(const sc_index* index, const T* d_queries, int64_t q, int k, doubl
         return rc;
     }
   }
-  if (k > KMAX_TILED) {
+  if (M == kEuclid || k > KMAX_TILED) {
     hipLaunchKernelGGL(iota_list_kernel, dim3(static_cast<unsigned>((q + 255) / 256)), dim3(256), 0,
                        stream, olist.as<uint32_t>(), overflow_n, q);
     SC_HIP(hipGetLastError());
@@ -795,9 +796,12 @@ int knn_exact_device(const sc_index* index, const void* d_queries, size_t q, siz
   if (q == 0) return SC_OK;
   if (knn_few_applies(index, q, k, metric))
     return knn_few_device(index, d_queries, q, k, metric, d_idx, d_dist, d_count, stream, stats);
-  if (metric == SC_EUCLIDIAN && k <= KMAX_TILED)
-    return knn_f64_device(index, d_queries, static_cast<int64_t>(q), static_cast<int>(k), d_idx,
-                          d_dist, d_count, stream, stats);
+  if (metric == SC_EUCLIDIAN && k <= KMAX_TILED) {
+    const int rc = knn_f64_device(index, d_queries, static_cast<int64_t>(q), static_cast<int>(k),
+                                  d_idx, d_dist, d_count, stream, stats);
+    if (rc != SC_ERR_OUT_OF_MEMORY) return rc;
+    clear_error();
+  }
   if (index->dtype == SC_F64)
     return dispatch_metric<double>(index, d_queries, q, k, metric, p, d_idx, d_dist, d_count,
                                    stream, stats);

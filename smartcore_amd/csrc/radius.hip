@@ -710,13 +710,18 @@ int run_radius(const sc_index* ix, const T* dq, int64_t q, double p, double radi
   if constexpr (M == kEuclid) {
     if (allow_cap && bound < sum_limit<T>() &&
         static_cast<double>(q) * static_cast<double>(n) > kSweepMinPairs) {
-      if (q <= kSweepQueries) return run_radius_f64<T>(ix, dq, q, radius, bound, res, want_dist, s);
+      if (q <= kSweepQueries) {
+        const int rc = run_radius_f64<T>(ix, dq, q, radius, bound, res, want_dist, s);
+        if (rc != SC_ERR_OUT_OF_MEMORY) return rc;
+        clear_error();  // the two passes keep nothing beside the rows
+        return run_radius<T, M>(ix, dq, q, p, radius, res, want_dist, false, s);
+      }
       res->q = static_cast<size_t>(q);
       res->offsets.assign(1, 0);
       for (int64_t b0 = 0; b0 < q; b0 += kSweepQueries) {
         sc_radius_result part;
-        if (int rc = run_radius_f64<T>(ix, dq + b0 * ld, std::min(kSweepQueries, q - b0), radius, bound,
-                                       &part, want_dist, s))
+        if (int rc = run_radius<T, M>(ix, dq + b0 * ld, std::min(kSweepQueries, q - b0), p, radius, &part,
+                                      want_dist, true, s))
           return rc;
         const uint64_t base = res->offsets.back();
         for (size_t i = 1; i < part.offsets.size(); ++i) res->offsets.push_back(base + part.offsets[i]);
