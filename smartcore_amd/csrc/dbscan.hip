@@ -37,36 +37,48 @@ using namespace sc;
 
 namespace {
 
-// The root of v's tree, halving the path on the way.  parent[x] <= x holds
-// for every value ever stored, so reads that are stale still point at an
-// ancestor, and the walk strictly decreases until it meets a root.
-__device__ uint32_t dbscan_rep(uint32_t* parent, uint32_t v) {
-  uint32_t cur = parent[v];
-  if (cur != v) {
-    uint32_t prev = v, next;
-    while (cur > (next = parent[cur])) {
-      parent[prev] = next;
-      prev = cur;
-      cur = next;
-    }
+// Union-find in one array, the larger of two trees' rows always under the
+// smaller, so that a tree's root is its smallest row.
+//
+// Every value ever stored in parent[x] is an ancestor of x and at most x.  A
+// read may be stale (another die's cache): it then gives an earlier, that is a
+// lower, ancestor, and what it takes for a root is set right by the swap, which
+// is not stale.  Pointing a row at its grandparent on the way (path splitting)
+// needs no swap: the row has a parent by then, and only roots are linked.
+__device__ uint32_t dbscan_rep(uint32_t* parent, uint32_t x) {
+  for (;;) {
+    const uint32_t up = parent[x];
+    if (up == x) return x;
+    const uint32_t above = parent[up];
+    if (above == up) return up;
+    parent[x] = above;
+    x = above;
   }
-  return cur;
 }
 
-// Joins the trees of u and v: the larger root is linked to the smaller by a
-// compare-and-swap; a failed swap returns a smaller value to continue from,
-// so the loop ends.
+// Joins the trees of u and v: Rem's algorithm (Dijkstra, 1976) without its
+// splicing.  Of the two rows, the one with the larger parent goes up; where it
+// has come to a root, that is linked under the other's parent by a
+// compare-and-swap.  The larger parent falls with every round, and the walk ends
+// where the two paths meet, which need not be at the root.
 __device__ void dbscan_link(uint32_t* parent, uint32_t u, uint32_t v) {
-  uint32_t ru = dbscan_rep(parent, u), rv = dbscan_rep(parent, v);
-  while (ru != rv) {
-    if (ru < rv) {
-      const uint32_t old = atomicCAS(&parent[rv], rv, ru);
-      if (old == rv) break;
-      rv = old;
+  uint32_t pu = parent[u], pv = parent[v];
+  while (pu != pv) {
+    if (pu < pv) {
+      const uint32_t x = u, px = pu;
+      u = v;
+      pu = pv;
+      v = x;
+      pv = px;
+    }
+    if (pu == u) {
+      pu = atomicCAS(&parent[u], u, pv);
+      if (pu == u) return;
     } else {
-      const uint32_t old = atomicCAS(&parent[ru], ru, rv);
-      if (old == ru) break;
-      ru = old;
+      const uint32_t above = parent[pu];
+      if (above != pu) parent[u] = above;
+      u = pu;
+      pu = above;
     }
   }
 }
