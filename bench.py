@@ -299,14 +299,19 @@ def bench_dbscan(args):
     lib.sc_profile_enable(0)
     kms, launches = profile_read(lib, "dbscan_pairs")
     k_s = kms / 1e3 / max(launches, 1)
+    # the row pairs that the sweep computed (the others lie in tiles further
+    # apart than eps), d multiplies and adds each
+    pairs = float(S.last_stats()["candidates"])
+    flops = 2.0 * d * pairs
     noise = int(np.sum(lab < 0))
     out = {"workload": f"DBSCAN eps={eps}, min_samples={min_samples}, Euclidian, {n:,}x{d} f64 "
                        "rows (10-class Gaussian mixture)",
            "value": float(n) * n / fit_s, "unit": "distance evaluations/s",
            "ms_per_fit": fit_s * 1e3, "clusters": int(nc), "noise_rows": noise, "dtype": "f64",
-           # how many pairs are computed depends on the data, so no rate is given
-           "roofline": {"bound": "fp64-mfma", "achieved": None, "peak": PEAK_FP64 / 1e12,
-                        "unit": "TFLOP/s", "frac": None, "traffic": None,
+           "pairs_computed": pairs,
+           "roofline": {"bound": "fp64-mfma", "achieved": flops / k_s / 1e12 if k_s > 0 else None,
+                        "peak": PEAK_FP64 / 1e12, "unit": "TFLOP/s",
+                        "frac": flops / k_s / PEAK_FP64 if k_s > 0 else None, "traffic": None,
                         "kernel": "dbscan_near_pairs_kernel (row pairs within the radius)",
                         "avg_ms": k_s * 1e3}}
     if not args.no_cpu:

@@ -69,10 +69,12 @@ typedef enum { SC_EUCLIDIAN = 0, SC_MANHATTAN = 1, SC_MINKOWSKI = 2 } sc_metric;
  * SC_PLAIN_FP64).  Minkowski has no SC_MIXED form. */
 typedef enum { SC_PLAIN_FP64 = 0, SC_MIXED = 1 } sc_mode;
 
-/* Per-call counters of the calling thread's last search (sc_last_stats). */
+/* Per-call counters of the calling thread's last search or DBSCAN fit
+ * (sc_last_stats). */
 typedef struct {
   uint64_t queries;            /* queries searched */
-  uint64_t candidates;         /* (index, distance) candidates replayed */
+  uint64_t candidates;         /* (index, distance) candidates replayed; Euclidian
+                                  DBSCAN fits: row pairs whose distance was computed */
   uint64_t overflow_queries;   /* queries recomputed by the sequential kernel */
   uint64_t shortlist_rescored; /* SC_MIXED: shortlist rows rescored in FP64 */
   uint64_t uncertified;        /* SC_MIXED: queries whose shortlist was not certified */

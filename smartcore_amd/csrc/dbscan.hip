@@ -380,7 +380,7 @@ __global__ __launch_bounds__(kMT, 2) void dbscan_pairs_kernel(
 // The tile pairs whose boxes are within the radius.  An item is a query tile
 // qt and a run of kRun tiles: the first threads test one tile's box each and
 // the ones that remain are swept as one list.  Items are taken from a counter
-// (the lists' lengths differ widely) until none is left.
+// (the lists' lengths differ widely) until none is left.  swept: tile pairs taken.
 constexpr int kRun = 128;
 static_assert(kRun == 2 * 64 && kRun <= kMT, "two wavefronts test a run");
 template <typename T>
@@ -388,7 +388,7 @@ __global__ __launch_bounds__(kMT, 2) void dbscan_near_pairs_kernel(
     const T* __restrict__ rows, int64_t nt, int ld, int d, const double* __restrict__ y2m,
     const double* __restrict__ box, Bound64 bd, double bound, double apart, int64_t items,
     uint2* __restrict__ pairs, unsigned long long cap, unsigned long long* __restrict__ cursor,
-    unsigned long long* __restrict__ next) {
+    unsigned long long* __restrict__ next, unsigned long long* __restrict__ swept) {
   __shared__ MSmem sm;
   __shared__ uint2 buf[kMT / 64][kPairBuf];
   __shared__ uint8_t list[kRun];
@@ -425,6 +425,7 @@ __global__ __launch_bounds__(kMT, 2) void dbscan_near_pairs_kernel(
     }
     __syncthreads();
     const uint32_t count = s_count[0] + s_count[1];
+    if (tid == 0 && count) atomicAdd(swept, static_cast<unsigned long long>(count));
     if ((near >> ml.lane) & 1)
       list[(ml.wave ? s_count[0] : 0u) + __popcll(near & ml.below())] = static_cast<uint8_t>(tid);
     __syncthreads();
@@ -669,7 +670,7 @@ int fit_pairs(const sc_index* index, double radius, double bound, size_t min_sam
   SC_HIP(cid.alloc(sizeof(uint32_t) * n, s));
   SC_HIP(lab.alloc(sizeof(uint32_t) * n, s));
   SC_HIP(starts.alloc(sizeof(uint32_t) * (nb + 1), s));
-  SC_HIP(cur.alloc(2 * sizeof(unsigned long long), s));  // pairs; items taken
+  SC_HIP(cur.alloc(3 * sizeof(unsigned long long), s));  // pairs; items taken; tile pairs swept
   const unsigned g = static_cast<unsigned>(std::min<int64_t>(4096, (n + 255) / 256));
   GroupedRows<T> gr;
   bool grouped = false;
@@ -689,7 +690,7 @@ int fit_pairs(const sc_index* index, double radius, double bound, size_t min_sam
     const uint32_t* place = grouped ? gr.place.template as<uint32_t>() : nullptr;
     uint2* pp = pairs.as<uint2>();
     unsigned long long* cp = cur.as<unsigned long long>();
-    SC_HIP(hipMemsetAsync(cp, 0, 2 * sizeof(unsigned long long), s));
+    SC_HIP(hipMemsetAsync(cp, 0, 3 * sizeof(unsigned long long), s));
     hipLaunchKernelGGL(dbscan_self_kernel, dim3(g), dim3(256), 0, s, y2m, n, deg.as<uint32_t>(),
                        par.as<uint32_t>());
     {
@@ -700,7 +701,7 @@ int fit_pairs(const sc_index* index, double radius, double bound, size_t min_sam
         const double apart = (bound * bd.up + bd.tiny) * (1.0 + 1e-12 + d * 4.5e-16);
         hipLaunchKernelGGL(dbscan_near_pairs_kernel<T>, dim3(512), dim3(kMT), 0, s, gr.rows.template as<T>(),
                            gr.nt, ld, d, gr.y2m.template as<double>(), gr.box.template as<double>(), bd,
-                           bound, apart, items, pp, cap, cp, cp + 1);
+                           bound, apart, items, pp, cap, cp, cp + 1, cp + 2);
       } else {
         hipLaunchKernelGGL(dbscan_pairs_kernel<T>, dim3(static_cast<unsigned>((total + per - 1) / per)),
                            dim3(kMT), 0, s, rows, n, ld, d, y2m, bd, bound, total, per, pp, cap, cp);
@@ -726,16 +727,18 @@ int fit_pairs(const sc_index* index, double radius, double bound, size_t min_sam
     hipLaunchKernelGGL(dbscan_labels_kernel, dim3(g), dim3(256), 0, s, n, root.as<uint32_t>(),
                        cid.as<uint32_t>(), lab.as<uint32_t>());
     SC_HIP(hipGetLastError());
-    unsigned long long found = 0;
+    unsigned long long done[3] = {0, 0, 0};
     uint32_t clusters = 0;
-    SC_HIP(hipMemcpyAsync(&found, cp, sizeof(found), hipMemcpyDeviceToHost, s));
+    SC_HIP(hipMemcpyAsync(done, cp, sizeof(done), hipMemcpyDeviceToHost, s));
     SC_HIP(hipMemcpyAsync(&clusters, starts.as<uint32_t>() + nb, sizeof(clusters), hipMemcpyDeviceToHost, s));
     SC_HIP(hipStreamSynchronize(s));
-    if (found > cap) {  // denser than the store: once more with room for all
-      cap = found;
+    if (done[0] > cap) {  // denser than the store: once more with room for all
+      cap = done[0];
       continue;
     }
     *num_classes = clusters;
+    last_stats().queries = static_cast<uint64_t>(n);
+    last_stats().candidates = (grouped ? done[2] : static_cast<uint64_t>(total)) * (kMQ * kMR);
     return download_staged(labels, lab.p, sizeof(uint32_t) * n, s);
   }
 }
@@ -756,6 +759,7 @@ int sc_dbscan_fit(const sc_index* index, double eps, size_t min_samples, sc_metr
   clear_error();
   if (!index || !labels || !num_classes) return fail(SC_PARAMETERS_ERROR, "null argument");
   *num_classes = 0;
+  last_stats() = sc_stats{};
   // dbscan.rs:278-284
   if (min_samples < 1) return fail(SC_FIT_FAILED, "Invalid minPts");
   if (eps <= 0.0) return fail(SC_FIT_FAILED, "Invalid radius: ");
