@@ -22,8 +22,9 @@
 //   scan     The rest in levels (knn_lists.hpp).  A workgroup sweeps 128-row
 //            tiles against 128 queries; a wavefront owns 32 queries against
 //            all 128 rows, each lane an 8 x 8 register tile, so that eight
-//            LDS words feed 64 v_sad_u16 and the kernel is bound by the
-//            vector unit (35 T lane instructions/s on this card), and a
+//            LDS words feed 64 v_sad_u16 (58 % of the 35 T lane
+//            instructions/s of this card at 96 dimensions: each dword's LDS
+//            reads are waited for before its sads, and the tile spills), and a
 //            query's hits are appended in row order without a barrier.  Up
 //            to 32 queries, the four wavefronts take four pieces of the rows
 //            against the same queries instead, and the rows' bytes bound it.
@@ -525,7 +526,11 @@ __global__ __launch_bounds__(kSadThreads, 3) void l1q_scan_kernel(
 // h (the smallest power of two with (max - min) / h <= 65534) is at most
 // 1/64 of the mean |v|, so the bound's band (about d h) stays a few percent
 // of a typical distance; otherwise, and for rows of more than 832 values, the
-// index keeps the f32 scan.
+// index keeps the f32 scan.  The width limit is that of an earlier scan, which
+// staged whole queries in LDS; a test holds that 900 values are declined.  This
+// kernel would take up to 16,384 and be the faster form (f32 scan and codes: 300
+// queries x 100,000 x 840: 28.9 and 1.2 ms; 1,000 x 20,000 x 4,096: 155 and 3.6; 50 x
+// 5,000 x 9,000: 3.6 and 3.1; 5 x 2,000 x 32,000: 9.9 and 10.4).
 constexpr int kQ16MaxLd = 832;
 
 }  // namespace
