@@ -155,7 +155,8 @@ __global__ __launch_bounds__(64 * kSelectWaves) void select_dense_kernel(
   const double* l = L + qi * cols;
   if (x2 < INFINITY) {
     double lv = l[lane], yv = y2m[lane];
-    for (int64_t c0 = 0; c0 < cols; c0 += 64) {
+    // (past cap, the query's list is lost; what was seen stays a bound)
+    for (int64_t c0 = 0; c0 < cols && cnt <= static_cast<uint32_t>(cap); c0 += 64) {
       const double cl = lv, cy = yv;
       if (c0 + 64 < cols) {  // the next chunk's loads run under this one's work
         lv = l[c0 + 64 + lane];
@@ -238,7 +239,16 @@ __global__ __launch_bounds__(kMT, 2) void scan_kernel(
           const int src = __builtin_ctzll(g);  // the column
           g &= g - 1;
           const uint32_t c = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(cnt[j]), src));
-          const uint32_t m = min(c, static_cast<uint32_t>(lv.cap));
+          if (c > static_cast<uint32_t>(lv.cap)) {
+            // its list is lost (the sequential kernel takes the query): no
+            // more rows for it
+            if (ml.lr == src) {
+              th[j] = -INFINITY;
+              mark[j] = c;
+            }
+            continue;
+          }
+          const uint32_t m = c;
           const double* u = out.u + slot_of(ml.wave * 32 + 16 * j + src, 0);
           // entries that other lanes of this wavefront stored
           __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");

@@ -380,7 +380,8 @@ __global__ __launch_bounds__(64 * kSelectWaves) void l1q_select_dense_kernel(
     int wv = w[lane];
     uint32_t ev = er[lane];
     int th = 0x7fffffff;
-    for (int64_t c0 = 0; c0 < cols; c0 += 64) {
+    // (past cap, the query's list is lost; what was seen stays a bound)
+    for (int64_t c0 = 0; c0 < cols && cnt <= static_cast<uint32_t>(cap); c0 += 64) {
       const int cw = wv;
       const uint32_t ce = ev;
       if (c0 + 64 < cols) {  // the next chunk's loads run under this one's work
@@ -501,6 +502,15 @@ __global__ __launch_bounds__(kSadThreads, 3) void l1q_scan_kernel(
       for (int ql = 0; ql < 32; ++ql) {
         const uint32_t c = s_cnt[sl.wave][ql];
         if (c - s_mark[sl.wave][ql] < grow) continue;  // the same in all lanes
+        if (c > static_cast<uint32_t>(lv.cap)) {
+          // its list is lost (the sequential kernel takes the query): no more
+          // rows for it
+          if (sl.lane == 0) {
+            s_th[sl.wave][ql] = -0x7fffffff - 1;
+            s_mark[sl.wave][ql] = c;
+          }
+          continue;
+        }
         KSmallest<uint32_t> ks;
         ks.clear();
         ks.take(out.u + slot_of(ql, 0), min(c, static_cast<uint32_t>(lv.cap)), sl.lane, k);
