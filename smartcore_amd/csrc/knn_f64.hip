@@ -356,10 +356,8 @@ int run_f64(const sc_index* index, const T* d_queries, int64_t q, int k, int64_t
     }
     {
       ProfScope ps("knn_replay", s);
-      hipLaunchKernelGGL((finish_kernel<T, kEuclid, double>), dim3(static_cast<unsigned>(qn)), dim3(kFinishThreads),
-                         finish_lds<T>(ld, ls.out.lists), s, rows, ld, qs, qn, k, ls,
-                         d_idx + b0 * k, d_dist + b0 * k, d_count + b0, olist.as<uint32_t>(), list_n,
-                         stats ? total : nullptr);
+      launch_finish<T, kEuclid>(rows, ld, qs, qn, k, ls, d_idx + b0 * k, d_dist + b0 * k, d_count + b0,
+                                olist.as<uint32_t>(), list_n, stats ? total : nullptr, s);
       SC_HIP(hipGetLastError());
     }
     if (int rc = launch_serial_exact(index, qs, k, olist.as<uint32_t>(), list_n, d_idx + b0 * k,

@@ -715,10 +715,8 @@ int knn_l1q_device(const sc_index* index, const float* d_queries, int64_t q, int
     }
     {
       ProfScope ps("knn_mixed_rescore", s);
-      hipLaunchKernelGGL((finish_kernel<float, kManhattan, uint32_t>), dim3(static_cast<unsigned>(qn)),
-                         dim3(kFinishThreads), finish_lds<float>(ld, ls.out.lists), s, rows, ld, qs, qn,
-                         k, ls, d_idx + b0 * k, d_dist + b0 * k, d_count + b0, olist.as<uint32_t>(),
-                         list_n, stats ? total : nullptr);
+      launch_finish<float, kManhattan>(rows, ld, qs, qn, k, ls, d_idx + b0 * k, d_dist + b0 * k,
+                                       d_count + b0, olist.as<uint32_t>(), list_n, stats ? total : nullptr, s);
       SC_HIP(hipGetLastError());
     }
     if (int rc = launch_serial_manhattan_f32(index, qs, k, olist.as<uint32_t>(), list_n, d_idx + b0 * k,

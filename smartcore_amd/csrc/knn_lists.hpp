@@ -23,8 +23,14 @@ namespace {
 
 constexpr int64_t kDenseRows = 1024;
 constexpr int kListTile = 128;       // rows per tile of every scan
+// The finish's threads per query: with a workgroup of 128 for each query, the
+// 256 CUs are busy from 512 queries on; fewer get more threads each.
 constexpr int kFinishThreads = 128;
-constexpr int kFinishBatch = 512;    // candidates rescored and replayed at a time
+constexpr int kFinishWide = 512;
+constexpr int64_t kFinishWideQueries = 512;
+constexpr size_t kFinishWideLds = 8192;  // beside 52 KB of tiles and batch
+// candidates rescored and replayed at a time
+constexpr int finish_batch(int threads) { return threads == kFinishWide ? 1024 : 512; }
 constexpr int kSelectWaves = 4;
 constexpr int kMaxLevels = 8;
 
@@ -147,33 +153,34 @@ inline size_t finish_lds(int ld, int64_t lists) {
 
 // S of every candidate and the heap replay (see the file comment).  The
 // candidates are numbered across the lists by a prefix sum of the counts and
-// taken kFinishBatch at a time: all threads compute their S, then the first
+// taken a batch at a time: all threads compute their S, then the first
 // wavefront replays the batch from LDS, 64 entries at a time.
-template <typename T, int M, typename V>
-__global__ __launch_bounds__(kFinishThreads) void finish_kernel(
+template <typename T, int M, typename V, int THREADS>
+__global__ __launch_bounds__(THREADS) void finish_kernel(
     const T* __restrict__ rows, int ld, const T* __restrict__ queries, int64_t q, int k, Lists<V> ls,
     int64_t* __restrict__ out_idx, double* __restrict__ out_dist, uint32_t* __restrict__ out_count,
     uint32_t* __restrict__ list, uint32_t* __restrict__ list_n,
     unsigned long long* __restrict__ total_cand) {
+  constexpr int kBatch = finish_batch(THREADS);
   // the query row (unless it is too wide), then the lists' starts (nl + 1)
   extern __shared__ __align__(16) unsigned char finish_smem[];
   const bool staged = finish_staged<T>(ld);
   T* qrow = reinterpret_cast<T*>(finish_smem);
   uint32_t* start = reinterpret_cast<uint32_t*>(qrow + (staged ? ld : 0));
-  __shared__ double s_S[kFinishBatch];
-  __shared__ uint32_t s_row[kFinishBatch];
-  __shared__ __align__(16) unsigned char tiles[kFinishThreads / 64][kSumTileBytes];
+  __shared__ double s_S[kBatch];
+  __shared__ uint32_t s_row[kBatch];
+  __shared__ __align__(16) unsigned char tiles[THREADS / 64][kSumTileBytes];
   __shared__ uint32_t s_over;
   const int64_t qi = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63;
   const int nl = 1 + static_cast<int>(ls.out.lists);
   if (tid == 0) s_over = 0u;
   if (staged)
-    for (int j = tid; j < ld; j += kFinishThreads) qrow[j] = queries[qi * ld + j];
+    for (int j = tid; j < ld; j += THREADS) qrow[j] = queries[qi * ld + j];
   __syncthreads();
   // exclusive prefix sum of the counts: each thread takes a run of lists
-  __shared__ uint32_t s_wave[kFinishThreads / 64];
-  const int run = (nl + kFinishThreads - 1) / kFinishThreads;
+  __shared__ uint32_t s_wave[THREADS / 64];
+  const int run = (nl + THREADS - 1) / THREADS;
   const int l0 = min(tid * run, nl), l1 = min(l0 + run, nl);
   uint32_t sum = 0;
   bool over = false;
@@ -208,7 +215,7 @@ __global__ __launch_bounds__(kFinishThreads) void finish_kernel(
     start[l] = at;
     at += c;
   }
-  if (tid == kFinishThreads - 1) start[nl] = at;
+  if (tid == THREADS - 1) start[nl] = at;
   if (tid == 0 && s_over) {
     list[atomicAdd(list_n, 1u)] = static_cast<uint32_t>(qi);
     out_count[qi] = 0u;
@@ -218,9 +225,9 @@ __global__ __launch_bounds__(kFinishThreads) void finish_kernel(
   const uint32_t total = start[nl];
   double hd = INFINITY, top = INFINITY;
   uint32_t hi = 0xffffffffu;
-  for (uint32_t e0 = 0; e0 < total; e0 += kFinishBatch) {
-    const uint32_t m = min(total - e0, static_cast<uint32_t>(kFinishBatch));
-    for (uint32_t b0 = tid & ~63u; b0 < m; b0 += kFinishThreads) {  // a wavefront's 64
+  for (uint32_t e0 = 0; e0 < total; e0 += kBatch) {
+    const uint32_t m = min(total - e0, static_cast<uint32_t>(kBatch));
+    for (uint32_t b0 = tid & ~63u; b0 < m; b0 += THREADS) {  // a wavefront's 64
       const uint32_t e = min(b0 + lane, m - 1);
       // the list of candidate e0 + e: the last whose start is at or below it
       int lo = 0, hi_l = nl;
@@ -272,6 +279,24 @@ __global__ __launch_bounds__(kFinishThreads) void finish_kernel(
     if (total_cand && lane == 0) atomicAdd(total_cand, static_cast<unsigned long long>(total));
     lane_heap_store(hd, hi, lane, k, out_idx + qi * k, out_dist + qi * k, out_count + qi);
   }
+}
+
+// 20 queries over 600,000 x 32 f32 rows sorted by class, whose first rows tell
+// little of the others (tens of thousands of candidates each), Manhattan:
+// 2.8 ms with 128 threads per query, 1.1 with 512; one query with the usual few
+// hundred: 45 and 37 us.
+template <typename T, int M, typename V>
+void launch_finish(const T* rows, int ld, const T* queries, int64_t q, int k, const Lists<V>& ls,
+                   int64_t* out_idx, double* out_dist, uint32_t* out_count, uint32_t* list,
+                   uint32_t* list_n, unsigned long long* total_cand, hipStream_t s) {
+  const size_t lds = finish_lds<T>(ld, ls.out.lists);
+  const dim3 grid(static_cast<unsigned>(q));
+  if (q <= kFinishWideQueries && lds <= kFinishWideLds)
+    hipLaunchKernelGGL((finish_kernel<T, M, V, kFinishWide>), grid, dim3(kFinishWide), lds, s, rows, ld,
+                       queries, q, k, ls, out_idx, out_dist, out_count, list, list_n, total_cand);
+  else
+    hipLaunchKernelGGL((finish_kernel<T, M, V, kFinishThreads>), grid, dim3(kFinishThreads), lds, s, rows, ld,
+                       queries, q, k, ls, out_idx, out_dist, out_count, list, list_n, total_cand);
 }
 
 // The rows at which the levels begin and end: the dense prefix of `cols`
