@@ -502,20 +502,14 @@ __global__ __launch_bounds__(kSadThreads, 3) void l1q_scan_kernel(
       for (int ql = 0; ql < 32; ++ql) {
         const uint32_t c = s_cnt[sl.wave][ql];
         if (c - s_mark[sl.wave][ql] < grow) continue;  // the same in all lanes
-        if (c > static_cast<uint32_t>(lv.cap)) {
-          // its list is lost (the sequential kernel takes the query): no more
-          // rows for it
-          if (sl.lane == 0) {
-            s_th[sl.wave][ql] = -0x7fffffff - 1;
-            s_mark[sl.wave][ql] = c;
-          }
-          continue;
-        }
         KSmallest<uint32_t> ks;
         ks.clear();
         ks.take(out.u + slot_of(ql, 0), min(c, static_cast<uint32_t>(lv.cap)), sl.lane, k);
         if (sl.lane == 0) {
-          const int th = q16_threshold(ks.kth, eqv[q0 + ql], rho);
+          // past cap its list is lost (the sequential kernel takes the query):
+          // no more rows for it
+          const int th = c > static_cast<uint32_t>(lv.cap) ? -0x7fffffff - 1
+                                                           : q16_threshold(ks.kth, eqv[q0 + ql], rho);
           if (th < s_th[sl.wave][ql]) s_th[sl.wave][ql] = th;
           s_mark[sl.wave][ql] = c;
         }
