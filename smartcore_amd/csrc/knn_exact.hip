@@ -390,34 +390,54 @@ __global__ __launch_bounds__(64 * kReplayWaves) void knn_replay_kernel(
 }
 
 // One workgroup per listed query; persistent over the list so the grid can
-// be launched before the list length is known.  Each wavefront takes 64 rows at
-// a time (through LDS, metric.hpp) and leaves their distances in one of two
-// buffers; the first wavefront replays the rows below the root in row order
-// while the others are at the next rows; the root that they test against is two
-// chunks old, and older means higher.  LANES: the heap lies across the first
-// wavefront's lanes (k <= 64), else in the outputs.  2,000 queries over 100,000 x 8 f32
-// equal rows: 6.8 ms with a thread per row reading value by value and two
-// barriers per 256 rows, 1.4 ms here; 3 queries that enter each of 300,000 x 32 f64
-// rows: 151 and 36 ms, 0.12 us per entry: the heap's serial chain.
-constexpr int kSerialThreads = 512;
+// be launched before the list length is known.  Each thread takes a row of 256
+// and leaves its distance in one of two buffers; the first wavefront replays
+// the rows below the root in row order while the others are at the next rows;
+// the root that they test against is two chunks old, and older means higher.
+// LANES: the heap lies across the first wavefront's lanes (k <= 64), else in
+// the outputs.
+//
+// Hardly any search lists a query, so what matters first is that an empty
+// launch starts beside another stream's scan: a mixed scan of 96 dimensions
+// leaves 64 VGPRs per SIMD lane.  With rows staged through LDS tiles by 512
+// threads (106 VGPRs, 49 KB), or by 256 (80, 25 KB), requests of the serving
+// loop waited here for up to 0.6 ms.  So the query row comes through the scalar
+// cache and a row 64 bytes at a time.  2,000 queries over 100,000 x 8 f32 equal rows: 6.8 ms with
+// value by value reads and two barriers per 256 rows, 1.5 here, 1.4 with the
+// tiles of 512; 3 queries that enter each of 300,000 x 32 f64 rows: 151, 36 and
+// 36 ms (0.12 us per entry, the heap's serial chain); 200 queries over 300,000 x 32 f64
+// equal rows, the whole call: 8.1, 4.0 and 2.6 ms (64 rows' lines per load).
+constexpr int kSerialThreads = 256;
 constexpr int kSerialWaves = kSerialThreads / 64;
-template <typename T>
-__host__ __device__ inline bool serial_staged(int ld) {
-  return ld * sizeof(T) <= 32768;
+// exact_sum with the values of 64 bytes in flight and x the same in all lanes
+template <typename T, int M>
+__device__ __forceinline__ double serial_sum(const T* __restrict__ x, const T* __restrict__ y, int ld, double p) {
+  constexpr int PV = 16 / sizeof(T);
+  typedef T Piece __attribute__((ext_vector_type(PV)));
+  double s = 0.0;
+#pragma unroll 1
+  for (int j = 0; j < ld; j += 4 * PV) {
+    Piece v[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) v[c] = *reinterpret_cast<const Piece*>(y + j + c * PV);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+#pragma unroll
+      for (int w = 0; w < PV; ++w) s = s + Term<T, M>::f(x[j + c * PV + w], v[c][w], p);
+      __builtin_amdgcn_sched_barrier(0);  // (terms formed ahead of the fold would hold 32 VGPRs)
+    }
+  }
+  return s;
 }
 template <typename T, int M, bool LANES>
 __global__ __launch_bounds__(kSerialThreads) void knn_serial_kernel(
     const T* __restrict__ refs, int64_t n, int ld, const T* __restrict__ queries, int k, double p,
     const uint32_t* __restrict__ list, const uint32_t* __restrict__ list_n, int64_t* __restrict__ out_idx,
     double* __restrict__ out_dist, uint32_t* __restrict__ out_count) {
-  extern __shared__ __align__(16) unsigned char serial_smem[];  // the query row, unless it is too wide
-  __shared__ __align__(16) unsigned char tiles[kSerialWaves][kSumTileBytes];
   __shared__ double s_d[2][kSerialThreads];
   __shared__ uint64_t s_mask[2][kSerialWaves];
   // the root after chunk c, read by all at chunk c + 2
   __shared__ double s_root[2];
-  T* qrow = reinterpret_cast<T*>(serial_smem);
-  const bool staged = serial_staged<T>(ld);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const uint32_t total = *list_n;
   for (uint32_t li = blockIdx.x; li < total; li += gridDim.x) {
@@ -427,8 +447,6 @@ __global__ __launch_bounds__(kSerialThreads) void knn_serial_kernel(
     double lane_d = INFINITY, top = INFINITY;
     asm volatile("" : "+v"(lane_d), "+v"(top));  // (a uniform 64-bit literal would lose its upper half)
     uint32_t lane_i = 0xffffffffu;
-    if (staged)
-      for (int j = tid; j < ld; j += kSerialThreads) qrow[j] = queries[qi * ld + j];
     if (!LANES)
       for (int j = tid; j < k; j += kSerialThreads) {
         hd[j] = INFINITY;
@@ -439,10 +457,7 @@ __global__ __launch_bounds__(kSerialThreads) void knn_serial_kernel(
     int buf = 0;
     for (int64_t c0 = 0; c0 < n; c0 += kSerialThreads, buf ^= 1) {
       const int64_t r = c0 + tid;
-      const uint32_t row = static_cast<uint32_t>(min(r, n - 1));
-      const double s = staged ? wave_exact_sums<T, M>(qrow, refs, row, ld, tiles[wave], p)
-                              : exact_sum<T, M>(queries + qi * ld, refs + static_cast<int64_t>(row) * ld, ld, p);
-      const double d = finalize<M>(s, p);
+      const double d = finalize<M>(serial_sum<T, M>(queries + qi * ld, refs + min(r, n - 1) * ld, ld, p), p);
       s_d[buf][tid] = d;
       const uint64_t below = __ballot(r < n && d < s_root[buf]);
       if (lane == 0) s_mask[buf][wave] = below;
@@ -503,22 +518,13 @@ int launch_serial(const sc_index* index, const T* d_queries, int k, double p, co
                   hipStream_t stream) {
   ProfScope ps("knn_serial", stream);
   const int ld = static_cast<int>(index->ld);
-  const size_t lds = serial_staged<T>(ld) ? sizeof(T) * ld : 0;
   const T* rows = static_cast<const T*>(index->rows);
   const int64_t n = static_cast<int64_t>(index->n);
-  static const bool attr = [] {  // static and dynamic LDS together pass 64 KB
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&knn_serial_kernel<T, M, true>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, 32768);
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&knn_serial_kernel<T, M, false>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, 32768);
-    return true;
-  }();
-  (void)attr;
   if (k <= KMAX_TILED)
-    hipLaunchKernelGGL((knn_serial_kernel<T, M, true>), dim3(groups), dim3(kSerialThreads), lds, stream, rows, n,
+    hipLaunchKernelGGL((knn_serial_kernel<T, M, true>), dim3(groups), dim3(kSerialThreads), 0, stream, rows, n,
                        ld, d_queries, k, p, list, list_n, d_idx, d_dist, d_count);
   else
-    hipLaunchKernelGGL((knn_serial_kernel<T, M, false>), dim3(groups), dim3(kSerialThreads), lds, stream, rows, n,
+    hipLaunchKernelGGL((knn_serial_kernel<T, M, false>), dim3(groups), dim3(kSerialThreads), 0, stream, rows, n,
                        ld, d_queries, k, p, list, list_n, d_idx, d_dist, d_count);
   SC_HIP(hipGetLastError());
   return SC_OK;

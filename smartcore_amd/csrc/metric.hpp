@@ -58,12 +58,11 @@ struct Term<float, kMinkowski> {
   }
 };
 
-// The reference's sum of one (query, row) pair: terms in dimension order,
+// The reference's sum of one (query, row) pair (p-free metrics): terms in dimension order,
 // 16 values of both requested before they are folded (rows are padded to
-// multiples of 16 values).  p: Minkowski's order.
+// multiples of 16 values).
 template <typename T, int M>
-__device__ __forceinline__ double exact_sum(const T* __restrict__ x, const T* __restrict__ y, int ld,
-                                            double p = 0.0) {
+__device__ __forceinline__ double exact_sum(const T* __restrict__ x, const T* __restrict__ y, int ld) {
   constexpr int PV = 16 / sizeof(T);
   typedef T Piece __attribute__((ext_vector_type(PV)));
   const Piece* xp = reinterpret_cast<const Piece*>(x);
@@ -79,7 +78,7 @@ __device__ __forceinline__ double exact_sum(const T* __restrict__ x, const T* __
 #pragma unroll
     for (int c = 0; c < 16 / PV; ++c)
 #pragma unroll
-      for (int w = 0; w < PV; ++w) s = s + Term<T, M>::f(xv[c][w], yv[c][w], p);
+      for (int w = 0; w < PV; ++w) s = s + Term<T, M>::f(xv[c][w], yv[c][w], 0.0);
   }
   return s;
 }
@@ -94,8 +93,7 @@ constexpr int kSumTileStride = 64 + 16;  // bytes of a row's 64 in the tile
 constexpr int kSumTileBytes = 64 * kSumTileStride;
 template <typename T, int M>
 __device__ __forceinline__ double wave_exact_sums(const T* x, const T* __restrict__ rows,
-                                                  uint32_t row, int ld, unsigned char* tile,
-                                                  double order = 0.0) {
+                                                  uint32_t row, int ld, unsigned char* tile) {
   constexpr int PV = 16 / sizeof(T);
   constexpr int CW = 64 / sizeof(T);  // values of a chunk (ld is a multiple)
   typedef T Piece __attribute__((ext_vector_type(PV)));
@@ -125,7 +123,7 @@ __device__ __forceinline__ double wave_exact_sums(const T* x, const T* __restric
 #pragma unroll
     for (int p = 0; p < 4; ++p)
 #pragma unroll
-      for (int w = 0; w < PV; ++w) s = s + Term<T, M>::f(x[c0 + p * PV + w], y[p][w], order);
+      for (int w = 0; w < PV; ++w) s = s + Term<T, M>::f(x[c0 + p * PV + w], y[p][w], 0.0);
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
   }

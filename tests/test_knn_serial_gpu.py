@@ -1,4 +1,4 @@
-"""The sequential kernel that overflowing queries and k > 64 go to, at the edges of its chunks (512
+"""The sequential kernel that overflowing queries and k > 64 go to, at the edges of its chunks (256
 rows), wavefronts and row widths, against the oracle: rows that each enter the heap, equal rows,
 non-finite values; indices in heap order and distance bits."""
 import numpy as np
@@ -29,7 +29,7 @@ def check(x, y, k, metric, om, mode=S.SC_PLAIN_FP64):
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 @pytest.mark.parametrize("metric,om", METRICS)
-@pytest.mark.parametrize("n,d,k", [(65, 1, 65), (511, 3, 100), (512, 16, 512), (513, 17, 66), (1_025, 40, 200),
+@pytest.mark.parametrize("n,d,k", [(65, 1, 65), (255, 5, 70), (257, 2, 90), (511, 3, 100), (512, 16, 512), (513, 17, 66), (1_025, 40, 200),
                                    (1_600, 33, 70), (700, 4_100, 90), (700, 8_200, 90)])
 def test_large_k(n, d, k, metric, om, dtype):
     rng = np.random.default_rng(n + d)
