@@ -138,11 +138,10 @@ __global__ void dbscan_root_kernel(int64_t n, const uint8_t* __restrict__ core, 
 // radius (in the bound's terms, so no pair that the reference would count)
 // is skipped.  Any order gives the same pairs, and so the same labels.  The
 // grouping costs about 128 distances per row.  200,000 x 8 rows in ten
-// clusters with 55 neighbours each: 12.7 ms without groups, 3.4 with them and
-// the two-step join (the sweep 10.9 and 2.3); 91 when the neighbour lists went
-// to the host.  Fewer rows are swept whole in the time the grouping takes
-// (32,768 rows of that kind: 0.46 ms with groups and 0.49 without; 16,384:
-// 0.41 and 0.25).
+// clusters with 55 neighbours each: 11.2 ms without groups, 3.2 with them (the
+// sweep 2.35); 91 when the neighbour lists went to the host.  Fewer rows are
+// swept whole in the time the grouping takes (32,768 rows of that kind: 0.44
+// ms with groups and 0.47 without; 16,384: 0.42 and 0.24).
 constexpr int64_t kGroupMinRows = 32768;
 constexpr int kMaxPivots = 128;
 constexpr int kPivotDims = 64;  // values of a row that the grouping looks at, at most
@@ -482,10 +481,10 @@ __global__ void dbscan_self_kernel(const double* __restrict__ y2m, int64_t n,
 }
 
 // Joins the core ends of every step-th pair.  Joining all pairs at once
-// spends its time on long walks and failed swaps at a few roots (2.0 ms for
-// 5.5 million pairs); a sixteenth of the pairs already joins nearly all of a
+// spends its time on walks and failed swaps at a few roots (0.45 ms for 5.5
+// million pairs); a sixteenth of the pairs already joins nearly all of a
 // cluster, and once every row points at its root the other pairs mostly find
-// their ends joined with two loads (0.6 in all).
+// their ends joined with two loads (0.22 in all).
 constexpr int kJoinSample = 16;
 __global__ __launch_bounds__(256) void dbscan_join_kernel(const uint2* __restrict__ pairs,
                                                           unsigned long long cap,

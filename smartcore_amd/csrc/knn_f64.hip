@@ -30,10 +30,11 @@
 // 1e-13 of the norms for f64 rows and 2e-7 of the distance for f32 rows, so
 // hardly a row is tested in vain.
 //
-// Bound by the FP64 matrix rate (72 TFLOP/s in a large matrix product on
-// this card): 4,096 queries x 200,000 x 64 f64 rows take 2.49 ms (12.8 ms
-// with a tile of vector subtract, multiply, add), 3,001 x 750,000 x 100 f32
-// 8.2 ms (42.0), 56 TFLOP/s.  The prefix is 1,024 rows because its selection
+// The scan uses 64 % of the FP64 matrix rate (72 TFLOP/s in a large matrix
+// product on this card) at 64 dimensions and 76 % at 100; mfma64.hpp has what
+// bounds it.  4,096 queries x 200,000 x 64 f64 rows take 2.42 ms (12.8 ms with
+// a tile of vector subtract, multiply, add), 3,001 x 750,000 x 100 f32 8.1 ms
+// (42.0), 55 TFLOP/s.  The prefix is 1,024 rows because its selection
 // is a walk per query; two levels then leave about 250 candidates per query
 // at k = 10, and one more level would cost two launches to save 100.
 #include <hip/hip_runtime.h>

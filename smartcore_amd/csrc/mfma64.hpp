@@ -8,9 +8,12 @@
 // without a barrier (a 2 x 2 arrangement of 64 x 64 needs 8 reads, but two
 // barriers per tile to order a query's rows across two wavefronts: 4,096
 // queries x 200,000 x 64 took 2.91 ms with it and 2.56 ms without, 5,000 x
-// 100,000 x 16 within a radius 0.91 and 0.84).  The kernel is bound by the matrix pipe (64 cycles per
-// MFMA and SIMD): the vector form needs three FP64 instructions per element
-// (subtract, multiply, add) where the MFMA needs one fused multiply-add.
+// 100,000 x 16 within a radius 0.91 and 0.84).  What it needs most is the
+// matrix pipe (64 cycles per MFMA and SIMD): the vector form needs three FP64
+// instructions per element (subtract, multiply, add) where the MFMA needs one
+// fused multiply-add.  It reaches 64 % of a large matrix product's rate at 64
+// dimensions and 76 % at 100: a barrier per 16 dimensions, and at a tile's end
+// 64 FP64 compares per lane beside an idle matrix pipe, whatever the rows' length.
 // Dimension chunks of 16 go through two LDS buffers: chunk c + 1 is stored
 // and chunk c + 2 requested while chunk c's MFMAs run, with one barrier per
 // chunk; the chunk stream runs on across tiles, so a tile's first chunk is
