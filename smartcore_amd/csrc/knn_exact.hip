@@ -22,7 +22,7 @@
 //           enter the heap are no-ops there too, so the heap array (order
 //           included) is the reference's.
 //   serial  For queries whose candidate list overflowed its capacity (or k
-//           above the tiled limit): one workgroup per query computes 512
+//           above the tiled limit): one workgroup per query computes 256
 //           distances at a time and its first wavefront replays the heap over
 //           those that beat the current root.  Exact for any input.
 #include <hip/hip_runtime.h>
